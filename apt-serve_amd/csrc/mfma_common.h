@@ -52,6 +52,8 @@ __device__ __forceinline__ uint16_t f32_to_bf16_bits(float x) {
 
 // Hand-placed wait points: a __syncthreads() would add fences that wait for every outstanding DMA load.
 #define APS_WAIT_VM(n) asm volatile("s_waitcnt vmcnt(" #n ")" ::: "memory")
+template <int N>
+__device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
 #define APS_WAIT_LGKM0() asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory")
 #define APS_BARRIER() asm volatile("s_barrier" ::: "memory")
 

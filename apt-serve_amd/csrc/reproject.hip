@@ -15,8 +15,9 @@
 // limit, and 16x16x32 (32 multiply-adds per accumulator element and instruction)
 // needs less energy per flop than 32x32x16 (16): alone, with operands in
 // registers, they sustain 1.8 against 1.4-1.6 PFLOP/s (aps_mfma_probe).
-// The K loop moves BK = 64 at a time through a two-stage LDS ring (2 x (32 + 32)
-// KiB of the 160 KiB per CU; 144 KiB with the epilogue images): tile t+1 is
+// The K loop moves BK = 64 at a time through an LDS ring of two stages (2 x (32 + 32)
+// KiB of the 160 KiB per CU; three and four stages for the smaller tiles of 128 and
+// 64 rows; 144 KiB with the epilogue images): tile t+1 is
 // copied global -> LDS by buffer_load ... lds (no VGPR round trip) while the
 // matrix cores consume tile t.
 //
@@ -39,6 +40,8 @@
 //
 // Workgroups are renumbered so that the 32 workgroups an XCD runs together
 // form an 8 x 4 block of tiles and share their A and W panels in that XCD's L2.
+#include <algorithm>
+
 #include "aps_common.h"
 #include "mfma_common.h"
 #include "row_stream_core.h"
@@ -51,7 +54,6 @@ constexpr int kThreads = 512;
 constexpr int kWaves = kThreads / 64;
 constexpr int WN = 64;                            // columns of a wavefront tile
 constexpr int kWTileBytes = BN * BK * 2;          // 32 KiB
-constexpr int kStages = 2;
 constexpr int kEpiPitch = WN * 2 + 16;            // bytes per row of a wave's epilogue image
 // The tile has 2 x 4 wavefronts of (32*MI rows) x 64 columns: 64*MI rows in all.  MI = 4 is the tile for large
 // M; with 49..128 rows it would spend most of its matrix-core time on rows that do not exist (and that time,
@@ -61,6 +63,10 @@ struct TileShape {
   static constexpr int kWm = 32 * MI, kBm = 2 * kWm;
   static constexpr int kATileBytes = kBm * BK * 2;
   static constexpr int kStageBytes = kATileBytes + kWTileBytes;
+  // As many stages as the LDS of a CU holds: with two, a tile's loads have one k-tile's time to arrive, and the 64-
+  // and 128-row tiles, whose k-tiles are short, waited for them (512 x 5120 on 15360 weight rows: 84 us with three
+  // stages of the 128-row tile, 111 with two of the 192-row one).
+  static constexpr int kStages = MI <= 2 ? 5 - MI : 2;
   static constexpr int kEpiWaveBytes = kWm * kEpiPitch;
   static constexpr int kLdsBytes =
       kWaves * kEpiWaveBytes > kStages * kStageBytes ? kWaves * kEpiWaveBytes : kStages * kStageBytes;
@@ -156,7 +162,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     const GemmArgs g) {
   using T = TileShape<MI>;
   constexpr int WM = T::kWm, TBM = T::kBm, kStageBytes = T::kStageBytes, kTileBytes = T::kATileBytes;
-  constexpr int kEpiWaveBytes = T::kEpiWaveBytes;
+  constexpr int kEpiWaveBytes = T::kEpiWaveBytes, S = T::kStages;
+  constexpr int kLoads = MI + 4;   // DMA loads of a wavefront per k-tile
   extern __shared__ __attribute__((aligned(1024))) char lds[];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -222,11 +229,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
   }
 
-  const int kt_base_ = tail_part >= 0 ? tail_part * g.tail_kt : (g.partial ? (int)blockIdx.y * g.kt_per_split : 0);
-  auto issue_loads = [&](int kt) {
-    char* sa = lds + (kt & 1) * kStageBytes;
+  const int kt_base = tail_part >= 0 ? tail_part * g.tail_kt : (g.partial ? (int)blockIdx.y * g.kt_per_split : 0);
+  const int nk_total = (int)(g.k / BK);
+  const int nk = tail_part >= 0 ? min(g.tail_kt, nk_total - kt_base)
+                                : (g.partial ? min(g.kt_per_split, nk_total - kt_base) : nk_total);
+  auto issue_loads = [&](int kt, int stage) {
+    char* sa = lds + stage * kStageBytes;
     char* sw = sa + kTileBytes;
-    const uint32_t koff = (uint32_t)(kt_base_ + kt) * (BK * 2);
+    const uint32_t koff = (uint32_t)(kt_base + kt) * (BK * 2);
 #pragma unroll
     for (int j = 0; j < MI; ++j) {
       const int i = wave * MI + j;  // 8-row group of the A tile handled by this wave-wide load (8*MI groups)
@@ -264,8 +274,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 #pragma unroll
       for (int e = 0; e < 4; ++e) acc[i][j][e] = 0.f;
 
-  auto read_frags = [&](int kt, int ks, u32x4(&af)[RT], u32x4(&wf)[4]) {
-    const char* sa = lds + (kt & 1) * kStageBytes;
+  auto read_frags = [&](int stage, int ks, u32x4(&af)[RT], u32x4(&wf)[4]) {
+    const char* sa = lds + stage * kStageBytes;
     const char* sw = sa + kTileBytes;
 #pragma unroll
     for (int i = 0; i < 4; ++i) wf[i] = *(const u32x4*)(sw + w_row_off + i * (16 * BK * 2) + chunk_off[ks]);
@@ -290,37 +300,40 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
   };
 
-  const int nk_total = (int)(g.k / BK);
-  const int kt_base = kt_base_;
-  const int nk = tail_part >= 0 ? min(g.tail_kt, nk_total - kt_base)
-                                : (g.partial ? min(g.kt_per_split, nk_total - kt_base) : nk_total);
   u32x4 a0[RT], w0[4], a1[RT], w1[4];
-  issue_loads(0);
-  if (nk > 1) {
-    issue_loads(1);
-    // tile 0 has landed, tile 1 (4 + MI loads per wavefront) may still be in flight
-    if constexpr (MI == 4) APS_WAIT_VM(8); else if constexpr (MI == 3) APS_WAIT_VM(7);
-    else if constexpr (MI == 2) APS_WAIT_VM(6); else APS_WAIT_VM(5);
-  } else {
-    APS_WAIT_VM(0);
-  }
+  // the first S tiles; tile 0 has landed when those issued after it are all that is in flight
+  const int ahead = min(nk, S) - 1;
+  issue_loads(0, 0);
+  if (ahead > 0) issue_loads(1, 1);
+  if (S > 2 && ahead > 1) issue_loads(2, 2);
+  if (S > 3 && ahead > 2) issue_loads(3, 3);
+  auto wait_tiles = [&](int tiles) {   // until at most `tiles` tiles are in flight
+    if (S > 3 && tiles >= 3) wait_vm<3 * kLoads>();
+    else if (S > 2 && tiles == 2) wait_vm<2 * kLoads>();
+    else if (tiles == 1) wait_vm<kLoads>();
+    else wait_vm<0>();
+  };
+  wait_tiles(ahead);
   APS_BARRIER();
   read_frags(0, 0, a0, w0);
-  int kt = 0;
-  for (; kt + 2 < nk; ++kt) {  // steady state: a tile kt+2 exists, the body has no branches
-    read_frags(kt, 1, a1, w1); mfma_step(a0, w0); interleave();
-    APS_WAIT_LGKM0();  // every fragment of tile kt is in registers: its stage is free
-    APS_WAIT_VM(0);    // tile kt+1 has landed (this wave's part; the barrier covers the others)
+  int kt = 0, stage = 0;
+  auto next = [&](int st) { return st + 1 == S ? 0 : st + 1; };
+  for (; kt + S < nk; ++kt) {  // steady state: a tile kt+S exists, the body has no branches
+    read_frags(stage, 1, a1, w1); mfma_step(a0, w0); interleave();
+    APS_WAIT_LGKM0();             // every fragment of tile kt is in registers: its stage is free
+    wait_vm<(S - 2) * kLoads>();  // tile kt+1 has landed (this wave's part; the barrier covers the others)
     APS_BARRIER();
-    issue_loads(kt + 2);
-    read_frags(kt + 1, 0, a0, w0); mfma_step(a1, w1); interleave();
+    issue_loads(kt + S, stage);
+    stage = next(stage);
+    read_frags(stage, 0, a0, w0); mfma_step(a1, w1); interleave();
   }
-  for (; kt < nk; ++kt) {  // last two tiles: nothing left to issue
-    read_frags(kt, 1, a1, w1); mfma_step(a0, w0); interleave();
+  for (; kt < nk; ++kt) {  // last S tiles: nothing left to issue
+    read_frags(stage, 1, a1, w1); mfma_step(a0, w0); interleave();
     APS_WAIT_LGKM0();
-    APS_WAIT_VM(0);
+    wait_tiles(max(nk - kt - 2, 0));
     APS_BARRIER();
-    if (kt + 1 < nk) read_frags(kt + 1, 0, a0, w0);
+    stage = next(stage);
+    if (kt + 1 < nk) read_frags(stage, 0, a0, w0);
     mfma_step(a1, w1);
   }
 
@@ -1085,45 +1098,56 @@ using namespace aps;
 
 extern "C" {
 
-// Tile rows / 64 for m rows beyond the row-streaming kernels' range.  Up to 128 rows: the smallest tile that
-// covers m.  Beyond: 192 or 256 rows, whichever needs less time by the count "rounds of workgroups over the
-// CUs x rows per tile" (a tie goes to the 256-row tile, which is the one tuned for large products).  Measured
-// on the 13B layer shapes this rule picks the faster of the two at every m from 160 to 4096; the 192-row tile
-// wins most of that range because its rounds are shorter and rows past m cost it less matrix-core time.
-static int tile_mi(int64_t m, int64_t n) {
-  if (m <= 64) return 1;
-  if (m <= 128) return 2;
-  auto cost = [&](int mi) {
-    const int64_t tiles = ((m + 64 * mi - 1) / (64 * mi)) * (n / BN);
-    return ((tiles + kNumCus - 1) / kNumCus) * mi;
-  };
-  return cost(3) < cost(4) ? 3 : 4;
+// Tile rows / 64 and K split of a product beyond the row-streaming kernels' range: the pair with the least time by
+// this account (us), fitted to the 13B layer shapes at 20 row counts from 49 to 16384:
+//   rounds of workgroups over the CUs x (k-tiles of a workgroup x time of a k-tile + 5), and for a split 6 (the second
+//   launch and its workspace) + the fp32 parts written and read once at 4.2 TB/s.
+// A k-tile takes 0.85 / 1.0 / 1.3 / 1.5 us with 64 / 128 / 192 / 256 tile rows: 256 rows are the cheapest per row, the
+// 128-row tile, whose 48 KiB stages fit the LDS three times, beats 192 rows wherever it does not need another round
+// (361 x 5120 on 20480 weight rows: 84 us; 192 rows 118, 256 rows 110).  More than 8 parts were slower than 8 at every
+// size (5120 x 5120, 64 rows: 22 us with 8, 27 with 12).
+struct TilePlan { int mi, splits; };
+static TailPlan tail_of(int mi, int64_t m, int64_t n, int64_t nk) {
+  return mi == 4 ? plan_tail(((m + BM - 1) / BM) * (n / BN), nk) : TailPlan{0, 1, 0, 0};
+}
+static TilePlan tile_plan(int64_t m, int64_t n, int64_t k, bool may_split) {
+  static constexpr double kTileUs[4] = {0.85, 1.0, 1.3, 1.5};
+  const int64_t nk = k / BK;
+  TilePlan best{4, 1};
+  double least = 1e300;
+  for (int mi = 4; mi >= 1; --mi) {
+    const int64_t bm = 64 * mi, tiles = ((m + bm - 1) / bm) * (n / BN);
+    const int max_splits = may_split ? (int)std::max<int64_t>(1, std::min<int64_t>(8, kNumCus / tiles)) : 1;
+    for (int s = 1; s <= max_splits; ++s) {
+      if (s > 1 && nk / s < 4) break;
+      const int64_t full = tiles * s / kNumCus, rest = tiles * s % kNumCus;
+      double rounds = (double)full;
+      if (rest) {
+        const int ways = may_split && s == 1 ? tail_of(mi, m, n, nk).ways : 1;
+        rounds += ways > 1 ? 1.0 / ways + 0.1 : 1.0;
+      }
+      double us = rounds * ((double)((nk + s - 1) / s) * kTileUs[mi - 1] + 5.0);
+      if (s > 1) us += 6.0 + (double)s * m * n * 8 / 4.2e6;
+      if (us < least) { least = us; best = {mi, s}; }
+    }
+  }
+  return best;
 }
 
 int aps_linear_nt_splits(int64_t m, int64_t n, int64_t k) {
-  // Few tiles (a decode step's handful of tokens) cannot pull the weights at HBM speed with one workgroup
-  // per tile: split K until about two waves of workgroups exist, keeping at least 4 k-tiles per split.
+  // Few tiles cannot pull the weights at HBM speed with one workgroup per tile: K is split until most CUs have one.
   if (m <= 0 || n <= 0 || k <= 0 || n % BN != 0 || k % BK != 0) return 1;
   if (m <= kRsMaxRows) return 1;  // streamed in one launch
   if (APS_KSPLIT && ksplit_covers(m, n, k)) return 1;   // K split inside the workgroups
   if (m <= kWsMaxRows) return weight_stream_plan(m, n, k).parts;
-  const int64_t bm = 64 * tile_mi(m, n);
-  const int64_t tiles = ((m + bm - 1) / bm) * (n / BN);
-  const int64_t nk = k / BK;
-  // as many splits as still give one workgroup per CU (a second, partly filled round costs more than it gains),
-  // at least 4 k-tiles each
-  int64_t s = kNumCus / tiles;
-  if (s > 32) s = 32;
-  while (s > 1 && nk / s < 4) --s;
-  return (int)(s < 1 ? 1 : s);
+  return tile_plan(m, n, k, true).splits;
 }
 
 // Tail plan of a product, or none: only full-size tiles without a uniform K split are cut.
 static TailPlan tail_plan_of(int64_t m, int64_t n, int64_t k) {
-  if (m <= kWsMaxRows || n <= 0 || k <= 0 || n % BN != 0 || k % BK != 0 || tile_mi(m, n) != 4 ||
-      aps_linear_nt_splits(m, n, k) > 1)
-    return TailPlan{0, 1, 0, 0};
-  return plan_tail(((m + BM - 1) / BM) * (n / BN), k / BK);
+  if (m <= kWsMaxRows || n <= 0 || k <= 0 || n % BN != 0 || k % BK != 0) return TailPlan{0, 1, 0, 0};
+  const TilePlan tp = tile_plan(m, n, k, true);
+  return tp.splits > 1 ? TailPlan{0, 1, 0, 0} : tail_of(tp.mi, m, n, k / BK);
 }
 
 int64_t aps_linear_nt_workspace_bytes(int64_t m, int64_t n, int64_t k) {
@@ -1158,7 +1182,9 @@ static int launch_gemm(const void* x, const void* weight, const void* bias, cons
   g.a = (const char*)x; g.w = (const char*)weight; g.bias = bias;
   g.lda_b = x_stride * 2; g.ldw_b = w_stride * 2;
   g.m = m; g.n = n; g.k = k;
-  const int mi = tile_mi(m, n);
+  const bool may_split = workspace && !(gs && m <= kWsMaxRows);  // (the split plan of few rows belongs to the streams)
+  const TilePlan plan = tile_plan(m, n, k, may_split);
+  const int mi = plan.mi;
   g.tiles_m = (int)((m + 64 * mi - 1) / (64 * mi)); g.tiles_n = (int)(n / BN);
   g.out = om;
   hipStream_t s = (hipStream_t)stream;
@@ -1213,8 +1239,8 @@ static int launch_gemm(const void* x, const void* weight, const void* bias, cons
   if (total >= ((int64_t)1 << 30)) return APS_ERR_UNSUPPORTED;
   const int64_t per_xcd = (total + kNumXcd - 1) / kNumXcd;
   int splits = 1;
-  if (workspace && !(gs && m <= kWsMaxRows)) {   // (the split plan of few rows belongs to the streaming kernels)
-    splits = aps_linear_nt_splits(m, n, k);
+  if (may_split) {
+    splits = plan.splits;
     if (splits > 1 && (workspace_bytes < (int64_t)splits * m * n * 4 || (addr(workspace) & 15))) return APS_ERR_WORKSPACE;
   }
   const int64_t nk_all = k / BK;

@@ -43,6 +43,20 @@ def test_linear_nt_small(dev, M, N, K, dtype):
     check(out2, OR._linear_fp32(x, w, None), dtype)
 
 
+@pytest.mark.parametrize("nk", [1, 2, 3, 4, 5, 9])
+@pytest.mark.parametrize("M", [64, 200, 380, 500])       # 64-, 128-, 192- and 256-row tiles at this N
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_linear_nt_ring_of_k_tiles(dev, M, nk, dtype):
+    """The LDS ring of every tile size (four, three, two stages) around its fill and drain: fewer k-tiles than
+    stages, as many, one more, and several rounds, on enough tiles that the plan neither splits K nor changes size."""
+    N, K = 25600, 64 * nk
+    assert ops._lib.load().aps_linear_nt_splits(M, N, K) == 1
+    x = randn((M, K), M, dtype)
+    w = (randn((N, K), nk) * 0.05).to(dtype)
+    b = (randn((N,), 3) * 0.2).to(dtype)
+    check(ops.linear_nt(x.to(dev), w.to(dev), b.to(dev)), OR._linear_fp32(x, w, b), dtype)
+
+
 @pytest.mark.parametrize("M", [3, 8, 16, 17, 32, 33, 48])
 @pytest.mark.parametrize("N,K", [(256, 64), (512, 1600), (1024, 2048), (2560, 5120), (16896, 1024), (20992, 512)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
