@@ -859,7 +859,12 @@ int launch_weight_stream(const GemmArgs& g, int parts, int64_t k_per_part, hipSt
 // this is for few rows and one-digit thousands of K.  A wavefront requests its share of the image copies, then
 // everything it streams (2 P loads of 1 KiB), waits for the copies alone, and multiplies as the rows arrive.
 constexpr int kKsMaxRows = 8;
-constexpr int ksplit_lds_bytes(int m, int pairs) { return m * pairs * 512 * 2 + kScWaves * kKsMaxRows * 16 * 4; }
+// The partial products (4 KiB) overlay the image: 8 rows of 5120 are then exactly half the LDS of a CU and two
+// workgroups share it.  Behind the image they left room for one: 8 x 5120 on 20480 weight rows 44.7 -> 35.5 us, on
+// 15360 35.5 -> 28.2, on 5120 19.7 -> 14.8.
+constexpr int ksplit_lds_bytes(int m, int pairs) {
+  return std::max(m * pairs * 512 * 2, kScWaves * kKsMaxRows * 16 * 4);
+}
 #ifndef APS_KSPLIT
 #define APS_KSPLIT 1
 #endif
@@ -943,7 +948,8 @@ __global__ __launch_bounds__(kScThreads) void weight_ksplit_kernel(const GemmArg
     acc = mfma16<BF16>(af, bf, acc);
   }
   // lane (g4, c) holds image rows 4 g4 + i (rows 8..15 do not exist) x weight row n0 + c
-  float* red = (float*)(lds + m * kRowBytes);
+  float* red = (float*)lds;
+  __syncthreads();   // the image is dead: the partial products take its place
   if (g4 < 2) {
 #pragma unroll
     for (int i = 0; i < 4; ++i) red[(wave * kKsMaxRows + 4 * g4 + i) * 16 + c] = acc[i];
