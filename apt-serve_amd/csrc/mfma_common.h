@@ -43,11 +43,18 @@ __device__ __forceinline__ uint16_t f32_to_f16_bits_rounded(float x) {
   asm volatile("" : "+v"(x));
   return __builtin_bit_cast(uint16_t, (_Float16)x);
 }
-__device__ __forceinline__ uint16_t f32_to_bf16_bits(float x) {
-  uint32_t u = __float_as_uint(x);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
+// Rounded to nearest even by the conversion instruction of gfx950 (v_cvt_pk_bf16_f32; a NaN stays a quiet NaN).  The
+// same in integer arithmetic, with a test for NaN, was 32 branches per tile of the prompt attention.
+__device__ __forceinline__ uint16_t f32_to_bf16_bits(float x) { return __builtin_bit_cast(uint16_t, (__bf16)x); }
+// Two values in one register, low half first: one conversion instruction for the pair in bf16.
+typedef float float2v __attribute__((ext_vector_type(2)));
+typedef _Float16 half2p __attribute__((ext_vector_type(2)));
+typedef __bf16 bf16x2p __attribute__((ext_vector_type(2)));
+template <bool BF16>
+__device__ __forceinline__ uint32_t pack2(float a, float b) {
+  const float2v v = {a, b};
+  if constexpr (BF16) return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2p));
+  else return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, half2p));
 }
 
 // Hand-placed wait points: a __syncthreads() would add fences that wait for every outstanding DMA load.

@@ -103,10 +103,7 @@ __device__ __forceinline__ uint16_t f32_to_q(float x) {
     asm volatile("" : "+v"(x));
     return __builtin_bit_cast(uint16_t, (_Float16)x);
   } else {  // bf16, round to nearest even
-    uint32_t u = __float_as_uint(x);
-    if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x40);
-    u += 0x7fffu + ((u >> 16) & 1u);
-    return (uint16_t)(u >> 16);
+    return __builtin_bit_cast(uint16_t, (__bf16)x);
   }
 }
 

@@ -19,16 +19,14 @@
 // the paged K/V cache through the sequence's block table; query i of a sequence with qlen new tokens and klen
 // tokens in all attends to keys 0 .. i + (klen - qlen).  Everything after the address of a key row is shared.
 #include "aps_common.h"
+#include "mfma_common.h"
 
 #include <math.h>
 
+#include <algorithm>
+
 namespace aps {
 namespace {
-
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float float16v __attribute__((ext_vector_type(16)));
-typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
 constexpr int BQ = 128;   // queries per workgroup
 constexpr int BKV = 64;   // keys per iteration
@@ -46,39 +44,19 @@ struct PrefillArgs {
   const int32_t* cu_seqlens_k; const int32_t* block_tables;
   int64_t table_stride, table_width, block_stride_b, num_blocks;
   int block_size;
+  int groups_shift;   // kPaged16: block_size = 16 << groups_shift
 };
 
-template <bool BF16>
-__device__ __forceinline__ float16v mfma32(const u32x4& a, const u32x4& b, const float16v& c) {
-  if constexpr (BF16)
-    return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0,
-                                                   0, 0);
-  else
-    return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(half8, a), __builtin_bit_cast(half8, b), c, 0, 0,
-                                                  0);
-}
+// Where the keys come from: packed rows; blocks of 16, 32, 64, ... tokens, so that 16 consecutive keys from a multiple
+// of 16 on lie together in one block; the same key by key, for row pitches past 32 MiB and blocks of any other size.
+enum KeySource { kPacked, kPaged16, kPackedAny, kPagedAny };
 
-template <bool BF16>
-__device__ __forceinline__ uint32_t pack2(float a, float b) {
-  if constexpr (BF16) {
-    auto cv = [](float x) -> uint32_t {
-      uint32_t u = __float_as_uint(x);
-      if ((u & 0x7fffffffu) > 0x7f800000u) return (u >> 16) | 0x40;
-      u += 0x7fffu + ((u >> 16) & 1u);
-      return u >> 16;
-    };
-    return cv(a) | (cv(b) << 16);
-  } else {
-    return (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)a) |
-           ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)b) << 16);
-  }
-}
-
-template <bool BF16, int D, bool PAGED>
+template <bool BF16, int D, int SRC>
 // Two wavefronts per SIMD: the kernel needs ~244 registers, and left to itself the compiler splits them into
 // 244 + 64 accumulation registers, which leaves room for one.
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_attention_kernel(
     const PrefillArgs a) {
+  constexpr bool PAGED = SRC == kPaged16 || SRC == kPagedAny;
   constexpr int KS = D / 16;          // k-steps of the score product
   constexpr int DT = D / 32;          // 32-row tiles of O^T
   constexpr int KROW = D * 2;         // bytes per key row in LDS
@@ -134,37 +112,93 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   // each: 16 lanes read 256 contiguous bytes of a key row), transposes the 8x8 block in registers with v_perm and
   // stores 8 rows d of 16 bytes (8 keys).  The pieces of the next tile are loaded into registers before the
   // current tile is multiplied and written to LDS after it.
+  //
+  // The addresses of a tile cost as much as its softmax when every key's offset is multiplied out by every lane (48
+  // quarter-rate multiplications, 130 with the divisions of a block table), so a lane keeps its offset inside a tile
+  // and the tile's (packed) or 16-key group's (kPaged16) start is scalar work: 4 x 2048 tokens of 40 x 128 f16
+  // 274 -> 251 us; six chunked prompts of 2048 new and 4200 cached tokens in bf16 (with the conversions to bf16 by
+  // instruction instead of integer arithmetic) 187 -> 107 us.
   constexpr int PER_K = BKV * KCH / kThreads;
   const bool v_thread = tid < 8 * KCH;           // whole wavefronts
   const int vo = tid / KCH, vch = tid % KCH;
+  const int v_row = (vo & 1) * 4;                // first key of the octet inside its group of 16; the others:
+  auto v_step = [](int j) { return (j & 3) + (j >> 2) * 8; };   // (see the file comment)
   const char* k_base = a.k + (PAGED ? 0 : (int64_t)s0 * a.k_stride_b) + (int64_t)head * D * 2;
-  const char* v_base = a.v + (PAGED ? 0 : (int64_t)s0 * a.v_stride_b) + (int64_t)head * D * 2 + vch * 16;
-  // byte offset of key gk of the sequence from k_base / v_base (`stride_b`: the operand's token row stride)
-  auto key_off = [&](int gk, int64_t stride_b) -> int64_t {
-    if constexpr (PAGED) {
-      const int bi = gk / a.block_size;
-      int64_t blk = a.block_tables[(int64_t)seq * a.table_stride + bi];
-      blk = blk < 0 ? 0 : (blk >= a.num_blocks ? a.num_blocks - 1 : blk);  // a bad table: wrong numbers, no fault
-      return blk * a.block_stride_b + (int64_t)(gk - bi * a.block_size) * stride_b;
-    } else {
-      return (int64_t)gk * stride_b;
-    }
+  const char* v_base = a.v + (PAGED ? 0 : (int64_t)s0 * a.v_stride_b) + (int64_t)head * D * 2;
+  const int32_t* table = PAGED ? a.block_tables + (int64_t)seq * a.table_stride : nullptr;
+  auto block_start = [&](int blk) -> int64_t {   // a bad table: wrong numbers, no fault
+    const int64_t b = blk < 0 ? 0 : (blk >= a.num_blocks ? a.num_blocks - 1 : (int64_t)blk);
+    return b * a.block_stride_b;
   };
+  // kPackedAny, kPagedAny: byte offset of key gk of the sequence from k_base / v_base
+  auto key_off = [&](int gk, int64_t stride_b) -> int64_t {
+    if constexpr (!PAGED) return (int64_t)gk * stride_b;
+    const int bi = gk / a.block_size;
+    return block_start(table[bi]) + (int64_t)(gk - bi * a.block_size) * stride_b;
+  };
+  // kPaged16: lane l holds the block of the tile's group l % 4 (groups past the sequence: its last one)
+  const int last_group = (len - 1) >> 4;
+  auto load_blocks = [&](int kv0) { return table[min((kv0 >> 4) + (lane & 3), last_group) >> a.groups_shift]; };
+  int blocks = SRC == kPaged16 ? load_blocks(0) : 0;   // of the next tile to be fetched
   u32x4 kreg[PER_K], vreg[8];
+  const uint32_t k_lane = (uint32_t)((SRC == kPacked ? tid / KCH : (tid / KCH) & 15) * (uint32_t)a.k_stride_b +
+                                     (tid % KCH) * 16);
+  const uint32_t v_lane = (uint32_t)(((SRC == kPacked ? (vo >> 1) * 16 : 0) + v_row) * (uint32_t)a.v_stride_b + vch * 16);
   auto fetch_tile = [&](int kv0) {
+    if constexpr (SRC == kPacked) {   // rows past the sequence read as zeros; the mask removes their scores
+      const int64_t left = len - kv0 - 1;
+      const __amdgpu_buffer_rsrc_t rk = make_rsrc(k_base + kv0 * a.k_stride_b, left * a.k_stride_b + D * 2);
+      const __amdgpu_buffer_rsrc_t rv = make_rsrc(v_base + kv0 * a.v_stride_b, left * a.v_stride_b + D * 2);
 #pragma unroll
-    for (int j = 0; j < PER_K; ++j) {
-      const int c = tid + j * kThreads;
-      const int key = c / KCH, ch = c % KCH;
-      const int gk = min(kv0 + key, len - 1);
-      kreg[j] = *(const u32x4*)(k_base + key_off(gk, a.k_stride_b) + ch * 16);
-    }
-    if (v_thread) {
+      for (int j = 0; j < PER_K; ++j)
+        kreg[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                rk, k_lane + j * (kThreads / KCH) * (uint32_t)a.k_stride_b, 0, 0));
+      if (v_thread) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {  // stored position 8*vo + j holds this key (see the file comment)
-        const int key = (vo >> 1) * 16 + (vo & 1) * 4 + (j & 3) + (j >> 2) * 8;
-        const int gk = min(kv0 + key, len - 1);
-        vreg[j] = *(const u32x4*)(v_base + key_off(gk, a.v_stride_b));
+        for (int j = 0; j < 8; ++j)
+          vreg[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                  rv, v_lane + v_step(j) * (uint32_t)a.v_stride_b, 0, 0));
+      }
+    } else if constexpr (SRC == kPaged16) {
+      auto group_start = [&](int g) {   // of group g of the tile (wave-uniform), from k_base / v_base
+        const int in_block = min((kv0 >> 4) + g, last_group) & ((1 << a.groups_shift) - 1);
+        return block_start(__builtin_amdgcn_readlane(blocks, g)) + (int64_t)(in_block * 16) * a.k_stride_b;
+      };
+      const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+#pragma unroll
+      for (int j = 0; j < PER_K; ++j) {   // keys past the sequence lie in its last block: finite or not, they are masked
+        const int g = KCH == 16 ? j : (wave_u >> 1) + 2 * j;
+        const __amdgpu_buffer_rsrc_t rk = make_rsrc(k_base + group_start(g), 15 * a.k_stride_b + D * 2);
+        kreg[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, k_lane, 0, 0));
+      }
+      if (v_thread) {
+        int64_t start;
+        if constexpr (KCH == 16) {
+          const int64_t lo = group_start(2 * wave_u), hi = group_start(2 * wave_u + 1);
+          start = half ? hi : lo;
+        } else {
+          const int64_t g0 = group_start(0), g1 = group_start(1), g2 = group_start(2), g3 = group_start(3);
+          start = (lane & 16) ? (half ? g3 : g1) : (half ? g2 : g0);
+        }
+        // rows past the sequence would be multiplied by zero probabilities, but may hold anything: its last row instead
+        const int lim = min(15, len - 1 - 16 * min((kv0 >> 4) + (vo >> 1), last_group));
+        const char* vp = v_base + start + vch * 16;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          vreg[j] = *(const u32x4*)(vp + __umul24(min(v_row + v_step(j), lim), (uint32_t)a.v_stride_b));
+      }
+      blocks = load_blocks(kv0 + BKV);
+    } else {
+#pragma unroll
+      for (int j = 0; j < PER_K; ++j) {
+        const int c = tid + j * kThreads;
+        kreg[j] = *(const u32x4*)(k_base + key_off(min(kv0 + c / KCH, len - 1), a.k_stride_b) + (c % KCH) * 16);
+      }
+      if (v_thread) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          vreg[j] = *(const u32x4*)(v_base + key_off(min(kv0 + (vo >> 1) * 16 + v_row + v_step(j), len - 1), a.v_stride_b) +
+                                    vch * 16);
       }
     }
   };
@@ -231,7 +265,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     for (int t = 0; t < 2; ++t)
 #pragma unroll
       for (int e = 0; e < 16; ++e) mx = fmaxf(mx, st[t][e]);
-    mx = fmaxf(mx, __shfl_xor(mx, 32));
+    {   // the other 32 keys of this query: one exchange between the halves of the wavefront, no LDS
+      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
+      mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
+    }
     const float m_use = (mx == -INFINITY) ? 0.f : mx;
     const float neg_m = -m_use * a.scale_log2;
     float psum = 0.f;
@@ -243,7 +280,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         st[t][e] = p;
         psum += p;
       }
-    psum += __shfl_xor(psum, 32);
     // the running maximum rarely moves after the first tiles: rescale O only when some query of the wavefront
     // needs it (a wave-uniform branch)
     const bool moved = mx != m_run;
@@ -275,6 +311,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   }
 
   // ---- normalise and store: lane owns query my_q, rows d = 32 t + 8 (e/4) + 4 half + e%4
+  l_run += __shfl_xor(l_run, 32);   // each half-wave has summed its own keys
   if (!q_live) return;
   const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
   char* op = a.out + (int64_t)(s0 + my_q) * a.out_stride_b + (int64_t)head * D * 2;
@@ -302,16 +339,24 @@ int launch_prefill(PrefillArgs& a, bool paged, int64_t num_seqs, int64_t max_seq
   if (q_tiles > 65535 || num_seqs > 65535 || num_heads > 65535) return APS_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)num_heads, (unsigned)num_seqs, (unsigned)q_tiles);
   hipStream_t s = (hipStream_t)stream;
+  // 64 rows within 32-bit offsets; 16 << shift tokens a block and a row pitch that a 24-bit product takes
+  int src = paged ? kPagedAny : kPackedAny;
+  if (!paged && std::max(a.k_stride_b, a.v_stride_b) < (1 << 25)) src = kPacked;
+  if (paged && a.block_size >= 16 && (a.block_size & (a.block_size - 1)) == 0 && a.v_stride_b < (1 << 24)) {
+    src = kPaged16;
+    a.groups_shift = __builtin_ctz((unsigned)a.block_size) - 4;
+  }
 #define APS_LAUNCH_PF(B, D_, P) APS_LAUNCH((prefill_attention_kernel<B, D_, P>), grid, dim3(kThreads), 0, s, a)
 #define APS_LAUNCH_PF_D(B, P)                                        \
   do {                                                               \
     if (head_size == 64) APS_LAUNCH_PF(B, 64, P); else APS_LAUNCH_PF(B, 128, P); \
   } while (0)
-  if (paged) {
-    if (dtype == APS_F16) APS_LAUNCH_PF_D(false, true); else APS_LAUNCH_PF_D(true, true);
-  } else {
-    if (dtype == APS_F16) APS_LAUNCH_PF_D(false, false); else APS_LAUNCH_PF_D(true, false);
-  }
+#define APS_LAUNCH_PF_S(P) do { if (dtype == APS_F16) APS_LAUNCH_PF_D(false, P); else APS_LAUNCH_PF_D(true, P); } while (0)
+  if (src == kPacked) APS_LAUNCH_PF_S(kPacked);
+  else if (src == kPaged16) APS_LAUNCH_PF_S(kPaged16);
+  else if (src == kPackedAny) APS_LAUNCH_PF_S(kPackedAny);
+  else APS_LAUNCH_PF_S(kPagedAny);
+#undef APS_LAUNCH_PF_S
 #undef APS_LAUNCH_PF_D
 #undef APS_LAUNCH_PF
   return launch_status();

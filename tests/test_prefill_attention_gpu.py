@@ -76,10 +76,13 @@ def test_argument_validation(dev):
 
 # ------------------------------------------------------------------ prefix branch (keys from the paged cache)
 
-def run_prefix(dev, klens, qlens, H, D, dtype=torch.float16, seed=0, BS=16):
+def run_prefix(dev, klens, qlens, H, D, dtype=torch.float16, seed=0, BS=16, poison=False):
     from test_oracle_attention import build_paged
     B = len(klens)
     kc, vc, bt, _, _ = build_paged(B, H, D, BS, klens, seed, dtype=dtype)
+    for b, n in enumerate(klens if poison else []):     # what a block holds past its sequence must not matter
+        kc[bt[b, (n - 1) // BS].long(), (n - 1) % BS + 1:] = float("nan")
+        vc[bt[b, (n - 1) // BS].long(), (n - 1) % BS + 1:] = float("nan")
     q = randn((sum(qlens), H, D), seed + 5, dtype)
     cu_q = torch.tensor([0] + list(np.cumsum(qlens)), dtype=torch.int32)
     cu_k = torch.tensor([0] + list(np.cumsum(klens)), dtype=torch.int32)
@@ -101,6 +104,39 @@ def test_prefix_attention_over_the_paged_cache(dev, H, D, dtype):
     klens = [37, 16, 300, 129, 64, 700, 1]
     qlens = [5, 16, 130, 1, 64, 257, 1]
     run_prefix(dev, klens, qlens, H, D, dtype)
+
+
+@pytest.mark.parametrize("BS", [16, 32, 64, 128, 24, 48])   # powers of two from 16 on: addressing by groups of 16 keys
+@pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (128, torch.float16)])
+def test_prefix_attention_block_sizes_and_block_remainders(dev, BS, D, dtype):
+    """Last blocks filled by 1 .. all tokens, NaN behind them, last key groups of a tile wholly past the sequence."""
+    klens = [1, 15, 16, 17, 48, 63, 64, 65, 113, 129, 200]
+    qlens = [1, 15, 3, 17, 40, 63, 1, 65, 100, 129, 131]
+    run_prefix(dev, klens, qlens, 2, D, dtype, seed=7, BS=BS, poison=True)
+
+
+def test_packed_rows_past_the_sequence_and_wide_row_pitch(dev):
+    """Keys of the next sequence (NaN here) take no part, whatever the remainder of the last key tile; and K/V rows
+    32 MiB apart, which are addressed key by key, give what close ones do."""
+    H, D = 2, 64
+    for n in (1, 17, 63, 64, 65, 130):
+        q, k, v = (randn((n + 70, H, D), 3 + i) for i in range(3))
+        k[n:], v[n:] = float("nan"), float("nan")
+        cu = torch.tensor([0, n, n + 70], dtype=torch.int32, device=dev)
+        alone = ops.flash_attn_varlen_func(q[:n].to(dev), k[:n].to(dev), v[:n].to(dev), cu_seqlens_q=cu[:2],
+                                           max_seqlen_q=n, softmax_scale=0.125)
+        both = ops.flash_attn_varlen_func(q.to(dev), k.to(dev), v.to(dev), cu_seqlens_q=cu, max_seqlen_q=max(n, 70),
+                                          softmax_scale=0.125)
+        assert torch.equal(both[:n], alone) and torch.isfinite(alone).all()
+    n = 70
+    q, k, v = (randn((n, H, D), 13 + i).to(dev) for i in range(3))
+    cu = torch.tensor([0, n], dtype=torch.int32, device=dev)
+    wide = torch.empty(n << 24, dtype=torch.float16, device=dev)
+    kw = wide.as_strided((n, H, D), (1 << 24, D, 1)).copy_(k)
+    vw = wide.as_strided((n, H, D), (1 << 24, D, 1), 4096).copy_(v)
+    a, b = (ops.flash_attn_varlen_func(q, x, y, cu_seqlens_q=cu, max_seqlen_q=n, softmax_scale=0.125)
+            for x, y in ((k, v), (kw, vw)))
+    assert torch.equal(a, b)
 
 
 def test_prefix_attention_block_size_32_and_argument_errors(dev):
