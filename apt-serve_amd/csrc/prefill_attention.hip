@@ -3,16 +3,18 @@
 // One 256-thread workgroup owns 128 consecutive queries of one (sequence, head); each of its four
 // wavefronts owns 32 of them.  Keys/values are consumed 64 at a time through LDS.
 //
-// The score tile is computed transposed, S^T = K Q^T, with v_mfma_f32_32x32x16: in the result layout
-// a lane owns ONE query (column lane%32) and 16 of the 32 keys of a tile, so the running max / sum of
-// the online softmax are per-lane scalars plus one exchange with lane^32.  The same registers, rounded
-// to the operand dtype, are directly the B operand (k = keys) of O^T = V^T P^T, provided V^T is laid
-// out in LDS in the key order the result layout produces:
-//     position (key/16)*16 + ((key%8)/4)*8 + (key%16/8)*4 + key%4   holds   key.
-// V is transposed on its way into LDS: a thread loads an 8x8 block (the 8 keys of one 16-byte run of stored
-// positions, 8 consecutive d), transposes it in registers and stores 8 rows of V^T; K is staged row-major
-// with its 16-byte chunks XOR-swizzled by key%16 so the fragment reads do not collide in the 64 banks.
-// The next tile's pieces travel global -> registers while the current tile is multiplied.
+// The score tile is computed transposed, S^T = K Q^T, with v_mfma_f32_16x16x32: in the result layout
+// a lane owns ONE query (column lane%16) of each of its wavefront's two query tiles and 4 of the 16 keys of
+// every key tile, so the running max / sum of the online softmax are per-lane scalars plus two exchanges
+// between the 16-lane rows.  The same registers, rounded to the operand dtype, are directly the B operand
+// (k = keys) of O^T = V^T P^T, provided V^T comes in the key order the result layout produces: the lane
+// of quad g takes keys 4g .. 4g+3 of two neighbouring key tiles.
+// K and V tiles are copied global -> LDS (buffer_load ... lds) one tile ahead into a ring of two stages, row-major
+// with their 16- and 32-byte pieces XOR-swizzled on the source side; V^T fragments are read with ds_read_b64_tr_b16,
+// which hands the 16 lanes of a row a 4-key x 16-d block transposed.  No tile passes through registers, and one
+// barrier a tile is enough.
+// (The part lowers its clock under real operands, and 16x16x32 costs less energy per flop than 32x32x16:
+// 4 x 2048 tokens of 40 x 128 f16 251 -> 243 us, and 243 -> 221 with the copies in place of staging registers.)
 //
 // PAGED variant (a prompt step that continues a cached prefix: chunked prompts, prefix caching): the queries are
 // the step's new tokens, the keys and values the whole sequence so far — prefix and new tokens alike — read from
@@ -47,6 +49,24 @@ struct PrefillArgs {
   int groups_shift;   // kPaged16: block_size = 16 << groups_shift
 };
 
+// Two stages of a K and a V tile
+template <int D>
+constexpr int prefill_lds_bytes() { return 2 * 2 * BKV * D * 2; }
+
+// One 1 KiB copy global -> LDS: lane l's 16 bytes at offset voff + soff of the buffer land at lds + 16 l.  From assembly:
+// the compiler, seeing a copy into LDS, waits for every load in flight before the next LDS read of any stage.
+__device__ __forceinline__ void copy_to_lds(uint32_t lds, const u32x4& rsrc, uint32_t voff, uint32_t soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
+               : "memory");
+}
+__device__ __forceinline__ u32x4 raw_rsrc(const char* p, int64_t bytes) {   // make_rsrc for the assembly
+  const uint64_t a = (uint64_t)p;
+  const uint32_t n = bytes <= 0 ? 0u : (bytes > 0xffffffffll ? 0xffffffffu : (uint32_t)bytes);
+  return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)),
+               (uint32_t)__builtin_amdgcn_readfirstlane((int)n), 0x00020000u};
+}
+
 // Where the keys come from: packed rows; blocks of 16, 32, 64, ... tokens, so that 16 consecutive keys from a multiple
 // of 16 on lie together in one block; the same key by key, for row pitches past 32 MiB and blocks of any other size.
 enum KeySource { kPacked, kPaged16, kPackedAny, kPagedAny };
@@ -57,20 +77,18 @@ template <bool BF16, int D, int SRC>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_attention_kernel(
     const PrefillArgs a) {
   constexpr bool PAGED = SRC == kPaged16 || SRC == kPagedAny;
-  constexpr int KS = D / 16;          // k-steps of the score product
-  constexpr int DT = D / 32;          // 32-row tiles of O^T
+  constexpr int KS = D / 32;          // k-steps of the score product
+  constexpr int KT = BKV / 16;        // key tiles of a score tile
+  constexpr int DT = D / 16;          // 16-row tiles of O^T
   constexpr int KROW = D * 2;         // bytes per key row in LDS
   constexpr int KCH = KROW / 16;      // 16-byte chunks per key row
-  // V^T in LDS: row d = 64 keys in stored order (8 chunks of 8 keys, 16 bytes each); chunk o of row d sits at
-  // slot o ^ ((d/8 ^ d/2) % 8), and rows 64.. start 128 bytes (32 banks) later.  With that both the fragment
-  // reads (16 lanes = 16 consecutive d, one chunk) and the transposed stores (16 lanes = rows 8 apart, one
-  // chunk) touch 16 different 16-byte bank groups.
-  constexpr int VROW = BKV * 2;
-  __shared__ __attribute__((aligned(16))) char k_lds[BKV * KROW];
-  __shared__ __attribute__((aligned(16))) char vt_lds[D * VROW + 128];
-  auto vt_addr = [&](int d, int chunk) {
-    return vt_lds + d * VROW + ((d >> 6) << 7) + ((chunk ^ (((d >> 3) ^ (d >> 1)) & 7)) << 4);
-  };
+  constexpr int kTile = BKV * KROW, kStage = 2 * kTile;
+  extern __shared__ __attribute__((aligned(1024))) char lds[];
+  // K in LDS: 16-byte chunk c of key row r sits at slot c ^ k_swz(r), so that 16 consecutive rows read at one chunk (a
+  // fragment) meet 16 different bank groups.  V: chunk c at slot c ^ v_swz(r), which moves 32-byte pieces: a transposing
+  // read takes 32 bytes of each of 8 consecutive rows per pass, from 8 different bank groups.
+  auto k_swz = [](int key) { return KCH == 16 ? key & 15 : (key >> 1) & 7; };
+  auto v_swz = [](int key) { return KCH == 16 ? (key & 7) << 1 : ((key >> 1) & 3) << 1; };
 
   // Grid (head, sequence, query tile), the last query tiles first: under the causal mask a workgroup's work grows
   // with its tile's position, and workgroups start in grid order, so the long ones go first and the short ones
@@ -87,45 +105,42 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   const int off = len - qlen;        // query i sees keys 0 .. i + off
   const int q0 = (int)(gridDim.z - 1 - blockIdx.z) * BQ;
   if (q0 >= qlen) return;
-  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-  const int qcol = lane & 31, half = lane >> 5;
-  const int my_q = q0 + wave * 32 + qcol;      // query index inside the sequence's new tokens (may be >= qlen)
-  const bool q_live = my_q < qlen;
-
-  // Q^T fragments: B operand, lane = (query, 8 consecutive d of each 16-wide k-step)
-  u32x4 qf[KS];
-  {
-    const char* qp = a.q + (int64_t)(s0 + (q_live ? my_q : qlen - 1)) * a.q_stride_b + (int64_t)head * D * 2;
+  const int tid = threadIdx.x & (kThreads - 1), wave = tid >> 6, lane = tid & 63;
+  const int qcol = lane & 15, quad = lane >> 4;
+  int my_q[2];                                 // query index inside the sequence's new tokens (may be >= qlen)
 #pragma unroll
-    for (int s = 0; s < KS; ++s) qf[s] = *(const u32x4*)(qp + (16 * s + 8 * half) * 2);
+  for (int u = 0; u < 2; ++u) my_q[u] = q0 + wave * 32 + 16 * u + qcol;
+
+  // Q^T fragments: B operand, lane = (query, 8 consecutive d of each 32-wide k-step)
+  u32x4 qf[2][KS];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    const char* qp = a.q + (int64_t)(s0 + min(my_q[u], qlen - 1)) * a.q_stride_b + (int64_t)head * D * 2;
+#pragma unroll
+    for (int s = 0; s < KS; ++s) qf[u][s] = *(const u32x4*)(qp + (32 * s + 8 * quad) * 2);
   }
 
-  float16v o[DT];
+  float4v o[2][DT];
 #pragma unroll
-  for (int t = 0; t < DT; ++t)
+  for (int u = 0; u < 2; ++u)
 #pragma unroll
-    for (int e = 0; e < 16; ++e) o[t][e] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;
+    for (int t = 0; t < DT; ++t) o[u][t] = float4v{0.f, 0.f, 0.f, 0.f};
+  float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
 
-  // Staging.  K: thread tid moves the 16-byte pieces tid + 256*j of the tile (row-major, swizzled).  V: thread
-  // (octet o, d-chunk ch), o = tid / KCH < 8, loads the 8 keys whose stored positions are 8o .. 8o+7 (16 bytes = 8 d
-  // each: 16 lanes read 256 contiguous bytes of a key row), transposes the 8x8 block in registers with v_perm and
-  // stores 8 rows d of 16 bytes (8 keys).  The pieces of the next tile are loaded into registers before the
-  // current tile is multiplied and written to LDS after it.
-  //
-  // The addresses of a tile cost as much as its softmax when every key's offset is multiplied out by every lane (48
-  // quarter-rate multiplications, 130 with the divisions of a block table), so a lane keeps its offset inside a tile
-  // and the tile's (packed) or 16-key group's (kPaged16) start is scalar work: 4 x 2048 tokens of 40 x 128 f16
-  // 274 -> 251 us; six chunked prompts of 2048 new and 4200 cached tokens in bf16 (with the conversions to bf16 by
-  // instruction instead of integer arithmetic) 187 -> 107 us.
-  constexpr int PER_K = BKV * KCH / kThreads;
-  const bool v_thread = tid < 8 * KCH;           // whole wavefronts
-  const int vo = tid / KCH, vch = tid % KCH;
-  const int v_row = (vo & 1) * 4;                // first key of the octet inside its group of 16; the others:
-  auto v_step = [](int j) { return (j & 3) + (j >> 2) * 8; };   // (see the file comment)
+  // Copies.  A wave-wide copy moves RPC = 64 / KCH key rows; wavefront w makes copies w, w + 4, ... of K's and of V's, so
+  // that a lane always moves the same row of a group of 16 keys (and has one swizzle), and the group is wave-uniform.
+  // A lane keeps its offset inside a tile; the tile's (kPacked) or the group's (kPaged16) start is scalar work.  (Every
+  // lane multiplying out 64-bit offsets of twelve rows a tile, 130 quarter-rate multiplications with the divisions of a
+  // block table, cost as much as the softmax.)
+  constexpr int RPC = 64 / KCH, PER = BKV / RPC / 4;   // key rows of a copy; copies per wavefront and operand
+  const int wave_u = __builtin_amdgcn_readfirstlane(wave);
+  const int key0 = RPC * wave + lane / KCH;            // this lane's key in its wavefront's first copy; + 4 RPC each
+  const int slot = lane % KCH;
   const char* k_base = a.k + (PAGED ? 0 : (int64_t)s0 * a.k_stride_b) + (int64_t)head * D * 2;
   const char* v_base = a.v + (PAGED ? 0 : (int64_t)s0 * a.v_stride_b) + (int64_t)head * D * 2;
-  const int32_t* table = PAGED ? a.block_tables + (int64_t)seq * a.table_stride : nullptr;
+  // (constant address space: scalar loads, which do not share a counter with the copies)
+  const auto table = (const __attribute__((address_space(4))) int32_t*)(PAGED ? a.block_tables + (int64_t)seq * a.table_stride
+                                                                              : a.cu_seqlens);
   auto block_start = [&](int blk) -> int64_t {   // a bad table: wrong numbers, no fault
     const int64_t b = blk < 0 ? 0 : (blk >= a.num_blocks ? a.num_blocks - 1 : (int64_t)blk);
     return b * a.block_stride_b;
@@ -134,197 +149,195 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   auto key_off = [&](int gk, int64_t stride_b) -> int64_t {
     if constexpr (!PAGED) return (int64_t)gk * stride_b;
     const int bi = gk / a.block_size;
-    return block_start(table[bi]) + (int64_t)(gk - bi * a.block_size) * stride_b;
+    return block_start(a.block_tables[(int64_t)seq * a.table_stride + bi]) + (int64_t)(gk - bi * a.block_size) * stride_b;
   };
-  // kPaged16: lane l holds the block of the tile's group l % 4 (groups past the sequence: its last one)
+  // kPaged16: the blocks of the wavefront's groups of the next tile to be copied (past the sequence: its last group)
   const int last_group = (len - 1) >> 4;
-  auto load_blocks = [&](int kv0) { return table[min((kv0 >> 4) + (lane & 3), last_group) >> a.groups_shift]; };
-  int blocks = SRC == kPaged16 ? load_blocks(0) : 0;   // of the next tile to be fetched
-  u32x4 kreg[PER_K], vreg[8];
-  const uint32_t k_lane = (uint32_t)((SRC == kPacked ? tid / KCH : (tid / KCH) & 15) * (uint32_t)a.k_stride_b +
-                                     (tid % KCH) * 16);
-  const uint32_t v_lane = (uint32_t)(((SRC == kPacked ? (vo >> 1) * 16 : 0) + v_row) * (uint32_t)a.v_stride_b + vch * 16);
-  auto fetch_tile = [&](int kv0) {
+  auto group_of = [&](int kv0, int j) { return min((kv0 >> 4) + (KCH == 16 ? j : (wave_u >> 1) + 2 * j), last_group); };
+  int blocks[PER];
+  auto load_blocks = [&](int kv0) {
+    if constexpr (SRC == kPaged16) {
+#pragma unroll
+      for (int j = 0; j < PER; ++j) blocks[j] = table[group_of(kv0, j) >> a.groups_shift];
+    }
+  };
+  const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
+  const int row_in = SRC == kPaged16 ? key0 & 15 : key0;
+  const uint32_t k_lane = (uint32_t)row_in * (uint32_t)a.k_stride_b + (slot ^ k_swz(key0)) * 16;
+  const uint32_t v_lane = (uint32_t)row_in * (uint32_t)a.v_stride_b + (slot ^ v_swz(key0)) * 16;
+  auto copy_tile = [&](int kv0, int stage) {
+    const uint32_t dst = lds_base + stage * kStage + wave_u * 1024;   // copy i of an operand: bytes [1024 i, 1024 i + 1024)
     if constexpr (SRC == kPacked) {   // rows past the sequence read as zeros; the mask removes their scores
       const int64_t left = len - kv0 - 1;
-      const __amdgpu_buffer_rsrc_t rk = make_rsrc(k_base + kv0 * a.k_stride_b, left * a.k_stride_b + D * 2);
-      const __amdgpu_buffer_rsrc_t rv = make_rsrc(v_base + kv0 * a.v_stride_b, left * a.v_stride_b + D * 2);
+      const u32x4 rk = raw_rsrc(k_base + kv0 * a.k_stride_b, left * a.k_stride_b + D * 2);
+      const u32x4 rv = raw_rsrc(v_base + kv0 * a.v_stride_b, left * a.v_stride_b + D * 2);
 #pragma unroll
-      for (int j = 0; j < PER_K; ++j)
-        kreg[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                rk, k_lane + j * (kThreads / KCH) * (uint32_t)a.k_stride_b, 0, 0));
-      if (v_thread) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          vreg[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                  rv, v_lane + v_step(j) * (uint32_t)a.v_stride_b, 0, 0));
+      for (int j = 0; j < PER; ++j) {
+        copy_to_lds(dst + j * 4096, rk, k_lane, j * 4 * RPC * (uint32_t)a.k_stride_b);
+        copy_to_lds(dst + kTile + j * 4096, rv, v_lane, j * 4 * RPC * (uint32_t)a.v_stride_b);
       }
     } else if constexpr (SRC == kPaged16) {
-      auto group_start = [&](int g) {   // of group g of the tile (wave-uniform), from k_base / v_base
-        const int in_block = min((kv0 >> 4) + g, last_group) & ((1 << a.groups_shift) - 1);
-        return block_start(__builtin_amdgcn_readlane(blocks, g)) + (int64_t)(in_block * 16) * a.k_stride_b;
-      };
-      const int wave_u = __builtin_amdgcn_readfirstlane(wave);
 #pragma unroll
-      for (int j = 0; j < PER_K; ++j) {   // keys past the sequence lie in its last block: finite or not, they are masked
-        const int g = KCH == 16 ? j : (wave_u >> 1) + 2 * j;
-        const __amdgpu_buffer_rsrc_t rk = make_rsrc(k_base + group_start(g), 15 * a.k_stride_b + D * 2);
-        kreg[j] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rk, k_lane, 0, 0));
+      for (int j = 0; j < PER; ++j) {
+        const int g = group_of(kv0, j);
+        const int64_t start =
+            block_start(blocks[j]) + (int64_t)((g & ((1 << a.groups_shift) - 1)) * 16) * a.k_stride_b;
+        // what a block holds past its sequence may be anything, and a zero probability does not cancel a NaN: the buffer
+        // ends with the sequence's last row and the others read as zeros
+        const int64_t bytes = min(15, len - 1 - 16 * g) * a.k_stride_b + D * 2;
+        copy_to_lds(dst + j * 4096, raw_rsrc(k_base + start, bytes), k_lane, 0);
+        copy_to_lds(dst + kTile + j * 4096, raw_rsrc(v_base + start, bytes), v_lane, 0);
       }
-      if (v_thread) {
-        int64_t start;
-        if constexpr (KCH == 16) {
-          const int64_t lo = group_start(2 * wave_u), hi = group_start(2 * wave_u + 1);
-          start = half ? hi : lo;
-        } else {
-          const int64_t g0 = group_start(0), g1 = group_start(1), g2 = group_start(2), g3 = group_start(3);
-          start = (lane & 16) ? (half ? g3 : g1) : (half ? g2 : g0);
-        }
-        // rows past the sequence would be multiplied by zero probabilities, but may hold anything: its last row instead
-        const int lim = min(15, len - 1 - 16 * min((kv0 >> 4) + (vo >> 1), last_group));
-        const char* vp = v_base + start + vch * 16;
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          vreg[j] = *(const u32x4*)(vp + __umul24(min(v_row + v_step(j), lim), (uint32_t)a.v_stride_b));
-      }
-      blocks = load_blocks(kv0 + BKV);
+      load_blocks(kv0 + BKV);
     } else {
 #pragma unroll
-      for (int j = 0; j < PER_K; ++j) {
-        const int c = tid + j * kThreads;
-        kreg[j] = *(const u32x4*)(k_base + key_off(min(kv0 + c / KCH, len - 1), a.k_stride_b) + (c % KCH) * 16);
-      }
-      if (v_thread) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j)
-          vreg[j] = *(const u32x4*)(v_base + key_off(min(kv0 + (vo >> 1) * 16 + v_row + v_step(j), len - 1), a.v_stride_b) +
-                                    vch * 16);
+      for (int j = 0; j < PER; ++j) {
+        const int gk = min(kv0 + key0 + j * 4 * RPC, len - 1);
+        char* const l = lds + stage * kStage + (wave_u + 4 * j) * 1024;
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) void*)(k_base + key_off(gk, a.k_stride_b) + (slot ^ k_swz(key0)) * 16),
+            (__attribute__((address_space(3))) void*)l, 16, 0, 0);
+        __builtin_amdgcn_global_load_lds(
+            (const __attribute__((address_space(1))) void*)(v_base + key_off(gk, a.v_stride_b) + (slot ^ v_swz(key0)) * 16),
+            (__attribute__((address_space(3))) void*)(l + kTile), 16, 0, 0);
       }
     }
   };
-  auto store_tile = [&]() {
-#pragma unroll
-    for (int j = 0; j < PER_K; ++j) {
-      const int c = tid + j * kThreads;
-      const int key = c / KCH, ch = c % KCH;
-      *(u32x4*)(k_lds + key * KROW + ((ch ^ (key & (KCH - 1) & 15)) * 16)) = kreg[j];
-    }
-    if (v_thread) {
-#pragma unroll
-      for (int dd = 0; dd < 8; ++dd) {  // row d = 8*vch + dd: dword p = (key position 2p, 2p+1)
-        const uint32_t sel = (dd & 1) ? 0x07060302u : 0x05040100u;
-        u32x4 col;
-#pragma unroll
-        for (int p4 = 0; p4 < 4; ++p4)
-          col[p4] = __builtin_amdgcn_perm(vreg[2 * p4 + 1][dd >> 1], vreg[2 * p4][dd >> 1], sel);
-        *(u32x4*)vt_addr(vch * 8 + dd, vo) = col;
-      }
-    }
+  // V^T fragment (16 d of tile t, keys of this lane's quad in key tile kt): the lane gives the address of its share of the
+  // 4 x 16 block, key i / 4 and d 4 (i % 4) for i = lane % 16, and receives d = i of the four keys
+  const int v_key = 4 * quad + (qcol >> 2);
+  const uint32_t v_frag = (uint32_t)(kTile + v_key * KROW + (qcol & 1) * 8);
+  const int v_piece = (qcol & 3) >> 1;
+  auto read_v = [&](int stage, int kt, int t) -> uint2 {
+    typedef short short4v __attribute__((ext_vector_type(4)));
+    const uint32_t at = v_frag + stage * kStage + kt * 16 * KROW + (((2 * t + v_piece) ^ v_swz(v_key)) << 4);
+    return __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16(
+                                         (__attribute__((address_space(3))) short4v*)(lds + at)));
   };
 
   const int kv_end = min(len, q0 + BQ + off);  // causal: keys beyond the tile's last query are never needed
   const int wave_q0 = q0 + wave * 32 + off;    // last key the first query of this wavefront sees
-  fetch_tile(0);
-  for (int kv0 = 0; kv0 < kv_end; kv0 += BKV) {
-    __syncthreads();  // previous tile fully consumed
-    store_tile();
-    __syncthreads();
-    if (kv0 + BKV < kv_end) fetch_tile(kv0 + BKV);  // in flight while this tile is multiplied
-    if (kv0 > wave_q0 + 31) continue;               // every key of the tile lies after this wavefront's queries
+  load_blocks(0);
+#pragma unroll
+  for (int u = 0; u < 2; ++u)   // the queries have arrived before the first copy is counted
+#pragma unroll
+    for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[u][s]));
+  copy_tile(0, 0);
+  for (int kv0 = 0, stage = 0; kv0 < kv_end; kv0 += BKV, stage ^= 1) {
+    APS_WAIT_LGKM0();  // no fragment read of the previous tile is under way,
+    APS_WAIT_VM(0);    // and this wavefront's copies of this tile have landed: past the barrier everyone's
+    APS_BARRIER();
+    if (kv0 + BKV < kv_end) copy_tile(kv0 + BKV, stage ^ 1);  // in flight while this tile is multiplied
+    if (kv0 > wave_q0 + 31) continue;                         // every key of the tile lies after this wavefront's queries
+    const char* const k_lds = lds + stage * kStage;
 
-    // ---- S^T = K Q^T for the two 32-key tiles
-    float16v st[2];
+    // ---- S^T = K Q^T: a K fragment serves both query tiles
+    float4v st[2][KT];
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int e = 0; e < 16; ++e) st[t][e] = 0.f;
-      const int key = t * 32 + qcol;  // A operand row of this lane
+      for (int t = 0; t < KT; ++t) st[u][t] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int s = 0; s < KS; ++s) {
-        const int ch = 2 * s + half;
-        const u32x4 kf = *(const u32x4*)(k_lds + key * KROW + ((ch ^ (key & (KCH - 1) & 15)) * 16));
-        st[t] = mfma32<BF16>(kf, qf[s], st[t]);
+    for (int s = 0; s < KS; ++s)
+#pragma unroll
+      for (int t = 0; t < KT; ++t) {
+        const int key = t * 16 + qcol, ch = 4 * s + quad;  // A operand row of this lane
+        const u32x4 kf = *(const u32x4*)(k_lds + key * KROW + ((ch ^ k_swz(key)) * 16));
+#pragma unroll
+        for (int u = 0; u < 2; ++u) st[u][t] = mfma16<BF16>(kf, qf[u][s], st[u][t]);
       }
-    }
-    // ---- online softmax for this lane's query (its 32 keys here, the other 32 in lane^32)
+    // ---- online softmax for this lane's two queries (16 keys of each here, the others in lanes 16, 32, 48 apart)
     // Only a tile that reaches past the wavefront's first query or past the sequence needs the mask.
     // The maximum is taken on the raw scores (the scale is positive) and the scale goes into the exponent's
     // fused multiply-add: max, fma, exp2 and add per score, nothing else.
     const bool masked = kv0 + BKV - 1 > wave_q0 || kv0 + BKV > len;
-    float mx = m_run;   // raw-score domain
     if (masked) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t)
+      for (int u = 0; u < 2; ++u) {
+        const int last = min(my_q[u] + off, len - 1) - kv0 - 4 * quad;   // the last key of this lane's that is seen
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-          const int key = kv0 + t * 32 + 8 * (e >> 2) + 4 * half + (e & 3);
-          if (!(key <= my_q + off && key < len)) st[t][e] = -INFINITY;
-        }
-    }
+        for (int t = 0; t < KT; ++t)
 #pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) mx = fmaxf(mx, st[t][e]);
-    {   // the other 32 keys of this query: one exchange between the halves of the wavefront, no LDS
-      const auto sw = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx), __float_as_uint(mx), false, false);
-      mx = fmaxf(__uint_as_float(sw[0]), __uint_as_float(sw[1]));
-    }
-    const float m_use = (mx == -INFINITY) ? 0.f : mx;
-    const float neg_m = -m_use * a.scale_log2;
-    float psum = 0.f;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int e = 0; e < 16; ++e) {
-        const float p = __builtin_amdgcn_exp2f(fmaf(st[t][e], a.scale_log2, neg_m));
-        st[t][e] = p;
-        psum += p;
+          for (int e = 0; e < 4; ++e)
+            if (16 * t + e > last) st[u][t][e] = -INFINITY;
       }
+    }
+    float mx[2], m_use[2], neg_m[2];
+    bool moved = false;
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      mx[u] = m_run[u];   // raw-score domain
+#pragma unroll
+      for (int t = 0; t < KT; ++t)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) mx[u] = fmaxf(mx[u], st[u][t][e]);
+      // the other keys of this query: exchanges between the 16-lane rows of the wavefront, no LDS
+      const auto s16 = __builtin_amdgcn_permlane16_swap(__float_as_uint(mx[u]), __float_as_uint(mx[u]), false, false);
+      mx[u] = fmaxf(__uint_as_float(s16[0]), __uint_as_float(s16[1]));
+      const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(mx[u]), __float_as_uint(mx[u]), false, false);
+      mx[u] = fmaxf(__uint_as_float(s32[0]), __uint_as_float(s32[1]));
+      m_use[u] = (mx[u] == -INFINITY) ? 0.f : mx[u];
+      neg_m[u] = -m_use[u] * a.scale_log2;
+      moved |= mx[u] != m_run[u];
+    }
     // the running maximum rarely moves after the first tiles: rescale O only when some query of the wavefront
     // needs it (a wave-uniform branch)
-    const bool moved = mx != m_run;
     if (__builtin_amdgcn_ballot_w64(moved) != 0) {
-      const float alpha = __builtin_amdgcn_exp2f((m_run - m_use) * a.scale_log2);
-      l_run *= alpha;
 #pragma unroll
-      for (int t = 0; t < DT; ++t)
+      for (int u = 0; u < 2; ++u) {
+        const float alpha = __builtin_amdgcn_exp2f((m_run[u] - m_use[u]) * a.scale_log2);
+        l_run[u] *= alpha;
 #pragma unroll
-        for (int e = 0; e < 16; ++e) o[t][e] *= alpha;
+        for (int t = 0; t < DT; ++t) o[u][t] *= alpha;
+        m_run[u] = mx[u];
+      }
     }
-    l_run += psum;
-    m_run = mx;
-    // ---- O^T += V^T P^T : four k-steps of 16 keys; P^T fragment = 8 consecutive result registers
+    // ---- O^T += V^T P^T : two k-steps of 32 keys; P^T fragment = the results of two neighbouring key tiles, a V^T
+    // fragment serves both query tiles
 #pragma unroll
-    for (int t32 = 0; t32 < 2; ++t32)
+    for (int w = 0; w < 2; ++w) {
+      u32x4 pf[2];
 #pragma unroll
-      for (int ks = 0; ks < 2; ++ks) {
-        u32x4 pf;
+      for (int u = 0; u < 2; ++u) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) pf[i] = pack2<BF16>(st[t32][8 * ks + 2 * i], st[t32][8 * ks + 2 * i + 1]);
-        const int chunk = (t32 * 2 + ks) * 2 + half;  // this lane's 8 keys of the step, in stored order
+        for (int t = 0; t < 2; ++t) {
+          float4v& p = st[u][2 * w + t];
 #pragma unroll
-        for (int t = 0; t < DT; ++t) {
-          const u32x4 vf = *(const u32x4*)vt_addr(t * 32 + qcol, chunk);
-          o[t] = mfma32<BF16>(vf, pf, o[t]);
+          for (int e = 0; e < 4; ++e) {
+            p[e] = __builtin_amdgcn_exp2f(fmaf(p[e], a.scale_log2, neg_m[u]));
+            l_run[u] += p[e];   // (this lane's keys; the lanes of a query are added at the end)
+          }
+          pf[u][2 * t] = pack2<BF16>(p[0], p[1]);
+          pf[u][2 * t + 1] = pack2<BF16>(p[2], p[3]);
         }
       }
+#pragma unroll
+      for (int t = 0; t < DT; ++t) {
+        const uint2 v0 = read_v(stage, 2 * w, t), v1 = read_v(stage, 2 * w + 1, t);
+        const u32x4 vf = {v0.x, v0.y, v1.x, v1.y};
+#pragma unroll
+        for (int u = 0; u < 2; ++u) o[u][t] = mfma16<BF16>(vf, pf[u], o[u][t]);
+      }
+    }
   }
 
-  // ---- normalise and store: lane owns query my_q, rows d = 32 t + 8 (e/4) + 4 half + e%4
-  l_run += __shfl_xor(l_run, 32);   // each half-wave has summed its own keys
-  if (!q_live) return;
-  const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-  char* op = a.out + (int64_t)(s0 + my_q) * a.out_stride_b + (int64_t)head * D * 2;
+  // ---- normalise and store: lane owns queries my_q, rows d = 16 t + 4 quad + e
 #pragma unroll
-  for (int t = 0; t < DT; ++t)
+  for (int u = 0; u < 2; ++u) {
+    float l = l_run[u];
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+    if (my_q[u] >= qlen) continue;
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    char* op = a.out + (int64_t)(s0 + my_q[u]) * a.out_stride_b + (int64_t)head * D * 2 + quad * 8;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int d = 32 * t + 8 * g + 4 * half;
+    for (int t = 0; t < DT; ++t) {
       uint2 w;
-      w.x = pack2<BF16>(o[t][4 * g] * inv, o[t][4 * g + 1] * inv);
-      w.y = pack2<BF16>(o[t][4 * g + 2] * inv, o[t][4 * g + 3] * inv);
-      *(uint2*)(op + d * 2) = w;
+      w.x = pack2<BF16>(o[u][t][0] * inv, o[u][t][1] * inv);
+      w.y = pack2<BF16>(o[u][t][2] * inv, o[u][t][3] * inv);
+      *(uint2*)(op + t * 32) = w;
     }
+  }
 }
 
 }  // namespace
@@ -346,11 +359,9 @@ int launch_prefill(PrefillArgs& a, bool paged, int64_t num_seqs, int64_t max_seq
     src = kPaged16;
     a.groups_shift = __builtin_ctz((unsigned)a.block_size) - 4;
   }
-#define APS_LAUNCH_PF(B, D_, P) APS_LAUNCH((prefill_attention_kernel<B, D_, P>), grid, dim3(kThreads), 0, s, a)
-#define APS_LAUNCH_PF_D(B, P)                                        \
-  do {                                                               \
-    if (head_size == 64) APS_LAUNCH_PF(B, 64, P); else APS_LAUNCH_PF(B, 128, P); \
-  } while (0)
+#define APS_LAUNCH_PF(B, D_, P) \
+  APS_LAUNCH((prefill_attention_kernel<B, D_, P>), grid, dim3(kThreads), prefill_lds_bytes<D_>(), s, a)
+#define APS_LAUNCH_PF_D(B, P) do { if (head_size == 64) APS_LAUNCH_PF(B, 64, P); else APS_LAUNCH_PF(B, 128, P); } while (0)
 #define APS_LAUNCH_PF_S(P) do { if (dtype == APS_F16) APS_LAUNCH_PF_D(false, P); else APS_LAUNCH_PF_D(true, P); } while (0)
   if (src == kPacked) APS_LAUNCH_PF_S(kPacked);
   else if (src == kPaged16) APS_LAUNCH_PF_S(kPaged16);
