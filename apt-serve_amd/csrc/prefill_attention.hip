@@ -1,10 +1,10 @@
 // Causal attention over freshly projected, packed (varlen) q/k/v for gfx950 — the prompt step.
 //
-// One 256-thread workgroup owns 128 consecutive queries of one (sequence, head); each of its four
-// wavefronts owns 32 of them.  Keys/values are consumed 64 at a time through LDS.
+// One 256-thread workgroup owns 128 (64) consecutive queries of one (sequence, head); each of its four
+// wavefronts owns QT = 2 (1) tiles of 16 of them.  Keys/values are consumed 64 at a time through LDS.
 //
 // The score tile is computed transposed, S^T = K Q^T, with v_mfma_f32_16x16x32: in the result layout
-// a lane owns ONE query (column lane%16) of each of its wavefront's two query tiles and 4 of the 16 keys of
+// a lane owns ONE query (column lane%16) of each of its wavefront's query tiles and 4 of the 16 keys of
 // every key tile, so the running max / sum of the online softmax are per-lane scalars plus two exchanges
 // between the 16-lane rows.  The same registers, rounded to the operand dtype, are directly the B operand
 // (k = keys) of O^T = V^T P^T, provided V^T comes in the key order the result layout produces: the lane
@@ -30,7 +30,6 @@
 namespace aps {
 namespace {
 
-constexpr int BQ = 128;   // queries per workgroup
 constexpr int BKV = 64;   // keys per iteration
 constexpr int kThreads = 256;
 constexpr float kLog2e = 1.4426950408889634f;
@@ -71,11 +70,12 @@ __device__ __forceinline__ u32x4 raw_rsrc(const char* p, int64_t bytes) {   // m
 // of 16 on lie together in one block; the same key by key, for row pitches past 32 MiB and blocks of any other size.
 enum KeySource { kPacked, kPaged16, kPackedAny, kPagedAny };
 
-template <bool BF16, int D, int SRC>
+template <bool BF16, int D, int SRC, int QT>
 // Two wavefronts per SIMD: the kernel needs ~244 registers, and left to itself the compiler splits them into
 // 244 + 64 accumulation registers, which leaves room for one.
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_attention_kernel(
     const PrefillArgs a) {
+  constexpr int BQ = 64 * QT;         // queries per workgroup
   constexpr bool PAGED = SRC == kPaged16 || SRC == kPagedAny;
   constexpr int KS = D / 32;          // k-steps of the score product
   constexpr int KT = BKV / 16;        // key tiles of a score tile
@@ -107,25 +107,27 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   if (q0 >= qlen) return;
   const int tid = threadIdx.x & (kThreads - 1), wave = tid >> 6, lane = tid & 63;
   const int qcol = lane & 15, quad = lane >> 4;
-  int my_q[2];                                 // query index inside the sequence's new tokens (may be >= qlen)
+  int my_q[QT];                                 // query index inside the sequence's new tokens (may be >= qlen)
 #pragma unroll
-  for (int u = 0; u < 2; ++u) my_q[u] = q0 + wave * 32 + 16 * u + qcol;
+  for (int u = 0; u < QT; ++u) my_q[u] = q0 + wave * (16 * QT) + 16 * u + qcol;
 
   // Q^T fragments: B operand, lane = (query, 8 consecutive d of each 32-wide k-step)
-  u32x4 qf[2][KS];
+  u32x4 qf[QT][KS];
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
+  for (int u = 0; u < QT; ++u) {
     const char* qp = a.q + (int64_t)(s0 + min(my_q[u], qlen - 1)) * a.q_stride_b + (int64_t)head * D * 2;
 #pragma unroll
     for (int s = 0; s < KS; ++s) qf[u][s] = *(const u32x4*)(qp + (32 * s + 8 * quad) * 2);
   }
 
-  float4v o[2][DT];
+  float4v o[QT][DT];
 #pragma unroll
-  for (int u = 0; u < 2; ++u)
+  for (int u = 0; u < QT; ++u)
 #pragma unroll
     for (int t = 0; t < DT; ++t) o[u][t] = float4v{0.f, 0.f, 0.f, 0.f};
-  float m_run[2] = {-INFINITY, -INFINITY}, l_run[2] = {0.f, 0.f};
+  float m_run[QT], l_run[QT];
+#pragma unroll
+  for (int u = 0; u < QT; ++u) { m_run[u] = -INFINITY; l_run[u] = 0.f; }
 
   // Copies.  A wave-wide copy moves RPC = 64 / KCH key rows; wavefront w makes copies w, w + 4, ... of K's and of V's, so
   // that a lane always moves the same row of a group of 16 keys (and has one swizzle), and the group is wave-uniform.
@@ -216,10 +218,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   };
 
   const int kv_end = min(len, q0 + BQ + off);  // causal: keys beyond the tile's last query are never needed
-  const int wave_q0 = q0 + wave * 32 + off;    // last key the first query of this wavefront sees
+  const int wave_q0 = q0 + wave * (16 * QT) + off;    // last key the first query of this wavefront sees
   load_blocks(0);
 #pragma unroll
-  for (int u = 0; u < 2; ++u)   // the queries have arrived before the first copy is counted
+  for (int u = 0; u < QT; ++u)   // the queries have arrived before the first copy is counted
 #pragma unroll
     for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[u][s]));
   copy_tile(0, 0);
@@ -228,13 +230,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     APS_WAIT_VM(0);    // and this wavefront's copies of this tile have landed: past the barrier everyone's
     APS_BARRIER();
     if (kv0 + BKV < kv_end) copy_tile(kv0 + BKV, stage ^ 1);  // in flight while this tile is multiplied
-    if (kv0 > wave_q0 + 31) continue;                         // every key of the tile lies after this wavefront's queries
+    if (kv0 > wave_q0 + 16 * QT - 1) continue;                         // every key of the tile lies after this wavefront's queries
     const char* const k_lds = lds + stage * kStage;
 
     // ---- S^T = K Q^T: a K fragment serves both query tiles
-    float4v st[2][KT];
+    float4v st[QT][KT];
 #pragma unroll
-    for (int u = 0; u < 2; ++u)
+    for (int u = 0; u < QT; ++u)
 #pragma unroll
       for (int t = 0; t < KT; ++t) st[u][t] = float4v{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
@@ -244,7 +246,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         const int key = t * 16 + qcol, ch = 4 * s + quad;  // A operand row of this lane
         const u32x4 kf = *(const u32x4*)(k_lds + key * KROW + ((ch ^ k_swz(key)) * 16));
 #pragma unroll
-        for (int u = 0; u < 2; ++u) st[u][t] = mfma16<BF16>(kf, qf[u][s], st[u][t]);
+        for (int u = 0; u < QT; ++u) st[u][t] = mfma16<BF16>(kf, qf[u][s], st[u][t]);
       }
     // ---- online softmax for this lane's two queries (16 keys of each here, the others in lanes 16, 32, 48 apart)
     // Only a tile that reaches past the wavefront's first query or past the sequence needs the mask.
@@ -253,7 +255,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     const bool masked = kv0 + BKV - 1 > wave_q0 || kv0 + BKV > len;
     if (masked) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
+      for (int u = 0; u < QT; ++u) {
         const int last = min(my_q[u] + off, len - 1) - kv0 - 4 * quad;   // the last key of this lane's that is seen
 #pragma unroll
         for (int t = 0; t < KT; ++t)
@@ -262,10 +264,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             if (16 * t + e > last) st[u][t][e] = -INFINITY;
       }
     }
-    float mx[2], m_use[2], neg_m[2];
+    float mx[QT], m_use[QT], neg_m[QT];
     bool moved = false;
 #pragma unroll
-    for (int u = 0; u < 2; ++u) {
+    for (int u = 0; u < QT; ++u) {
       mx[u] = m_run[u];   // raw-score domain
 #pragma unroll
       for (int t = 0; t < KT; ++t)
@@ -284,7 +286,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     // needs it (a wave-uniform branch)
     if (__builtin_amdgcn_ballot_w64(moved) != 0) {
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
+      for (int u = 0; u < QT; ++u) {
         const float alpha = __builtin_amdgcn_exp2f((m_run[u] - m_use[u]) * a.scale_log2);
         l_run[u] *= alpha;
 #pragma unroll
@@ -296,9 +298,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     // fragment serves both query tiles
 #pragma unroll
     for (int w = 0; w < 2; ++w) {
-      u32x4 pf[2];
+      u32x4 pf[QT];
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
+      for (int u = 0; u < QT; ++u) {
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
           float4v& p = st[u][2 * w + t];
@@ -316,14 +318,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         const uint2 v0 = read_v(stage, 2 * w, t), v1 = read_v(stage, 2 * w + 1, t);
         const u32x4 vf = {v0.x, v0.y, v1.x, v1.y};
 #pragma unroll
-        for (int u = 0; u < 2; ++u) o[u][t] = mfma16<BF16>(vf, pf[u], o[u][t]);
+        for (int u = 0; u < QT; ++u) o[u][t] = mfma16<BF16>(vf, pf[u], o[u][t]);
       }
     }
   }
 
   // ---- normalise and store: lane owns queries my_q, rows d = 16 t + 4 quad + e
 #pragma unroll
-  for (int u = 0; u < 2; ++u) {
+  for (int u = 0; u < QT; ++u) {
     float l = l_run[u];
     l += __shfl_xor(l, 16);
     l += __shfl_xor(l, 32);
@@ -348,7 +350,12 @@ using namespace aps;
 namespace {
 int launch_prefill(PrefillArgs& a, bool paged, int64_t num_seqs, int64_t max_seqlen_q, int num_heads, int head_size,
                    int dtype, aps_stream_t stream) {
-  const int64_t q_tiles = (max_seqlen_q + BQ - 1) / BQ;
+  // Few workgroups: 64 queries each instead of 128.  A workgroup's time is its key tiles one after the other, 2.0 us each
+  // with 32 queries a wavefront and 1.5 with 16, so as long as the CUs are not full the shorter ones finish first (12
+  // heads, 2048 tokens: 34 -> 26 us; 40 heads, 361 tokens 11.1 -> 9.9, 4 x 50 on a prefix of 4000 61 -> 49); full CUs
+  // lose by reading every fragment for half the queries (40 heads, 1400 tokens 26 -> 28, 4 x 2048 221 -> 304).
+  const int qt = num_heads * (a.num_tokens / 128 + num_seqs) <= 384 ? 1 : 2;
+  const int64_t q_tiles = (max_seqlen_q + 64 * qt - 1) / (64 * qt);
   if (q_tiles > 65535 || num_seqs > 65535 || num_heads > 65535) return APS_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)num_heads, (unsigned)num_seqs, (unsigned)q_tiles);
   hipStream_t s = (hipStream_t)stream;
@@ -360,7 +367,12 @@ int launch_prefill(PrefillArgs& a, bool paged, int64_t num_seqs, int64_t max_seq
     a.groups_shift = __builtin_ctz((unsigned)a.block_size) - 4;
   }
 #define APS_LAUNCH_PF(B, D_, P) \
-  APS_LAUNCH((prefill_attention_kernel<B, D_, P>), grid, dim3(kThreads), prefill_lds_bytes<D_>(), s, a)
+  do {                                                                                                                \
+    if (qt == 2)                                                                                                      \
+      APS_LAUNCH((prefill_attention_kernel<B, D_, P, 2>), grid, dim3(kThreads), prefill_lds_bytes<D_>(), s, a);       \
+    else                                                                                                              \
+      APS_LAUNCH((prefill_attention_kernel<B, D_, P, 1>), grid, dim3(kThreads), prefill_lds_bytes<D_>(), s, a);       \
+  } while (0)
 #define APS_LAUNCH_PF_D(B, P) do { if (head_size == 64) APS_LAUNCH_PF(B, 64, P); else APS_LAUNCH_PF(B, 128, P); } while (0)
 #define APS_LAUNCH_PF_S(P) do { if (dtype == APS_F16) APS_LAUNCH_PF_D(false, P); else APS_LAUNCH_PF_D(true, P); } while (0)
   if (src == kPacked) APS_LAUNCH_PF_S(kPacked);

@@ -107,12 +107,30 @@ def test_prefix_attention_over_the_paged_cache(dev, H, D, dtype):
 
 
 @pytest.mark.parametrize("BS", [16, 32, 64, 128, 24, 48])   # powers of two from 16 on: addressing by groups of 16 keys
+@pytest.mark.parametrize("H", [2, 64])                     # 64- and 128-query workgroups
 @pytest.mark.parametrize("D,dtype", [(64, torch.bfloat16), (128, torch.float16)])
-def test_prefix_attention_block_sizes_and_block_remainders(dev, BS, D, dtype):
+def test_prefix_attention_block_sizes_and_block_remainders(dev, BS, D, dtype, H):
     """Last blocks filled by 1 .. all tokens, NaN behind them, last key groups of a tile wholly past the sequence."""
     klens = [1, 15, 16, 17, 48, 63, 64, 65, 113, 129, 200]
     qlens = [1, 15, 3, 17, 40, 63, 1, 65, 100, 129, 131]
-    run_prefix(dev, klens, qlens, 2, D, dtype, seed=7, BS=BS, poison=True)
+    run_prefix(dev, klens, qlens, H, D, dtype, seed=7, BS=BS, poison=True)
+
+
+@pytest.mark.parametrize("H,D", [(2, 64), (200, 64), (2, 128), (200, 128)])
+def test_packed_remainders_of_both_workgroup_sizes(dev, H, D):
+    """64 queries a workgroup (2 heads) and 128 (200 heads): every remainder class of the query and key tiles."""
+    lens = [1, 15, 17, 33, 64, 65, 97, 128, 129, 191, 200]
+    T = sum(lens)
+    q, k, v = (randn((T, H, D), 40 + i) for i in range(3))
+    cu = torch.tensor([0] + list(np.cumsum(lens)), dtype=torch.int32)
+    out = ops.flash_attn_varlen_func(q.to(dev), k.to(dev), v.to(dev), cu_seqlens_q=cu.to(dev), max_seqlen_q=max(lens),
+                                     softmax_scale=D ** -0.5).float().cpu()
+    for b, n in enumerate(lens):
+        s = slice(int(cu[b]), int(cu[b]) + n)
+        sc = torch.einsum("qhd,khd->hqk", q[s].float(), k[s].float()) * D ** -0.5
+        sc = sc.masked_fill(torch.ones(n, n, dtype=torch.bool).triu(1), float("-inf"))
+        ref = torch.einsum("hqk,khd->qhd", sc.softmax(-1), v[s].float())
+        assert torch.allclose(out[s], ref, atol=5e-3, rtol=5e-3), (n, (out[s] - ref).abs().max().item())
 
 
 def test_packed_rows_past_the_sequence_and_wide_row_pitch(dev):
