@@ -902,7 +902,7 @@ __global__ __launch_bounds__(kScThreads) void weight_ksplit_kernel(const GemmArg
     if (r < m) {
       const int slot = 64 * jg + lane;
       const int piece = (slot & ~15) | ((slot ^ r) & 15);
-      asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"
+      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"   // (m0 needs one wait state)
                    :
                    : "s"(__builtin_amdgcn_readfirstlane(lds_base + (uint32_t)(r * kRowBytes + jg * 1024))),
                      "v"((uint32_t)(r * g.lda_b) + (uint32_t)(piece * 16)), "s"(rsrc)
