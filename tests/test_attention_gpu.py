@@ -71,6 +71,17 @@ def test_decode_attention_small(dev, D, dtype, partition_size):
     check(out, ref, dtype)
 
 
+@pytest.mark.parametrize("B", [63, 64, 65, 257, 511, 512, 513])
+def test_sequences_taken_longest_first_each_exactly_once(dev, B):
+    """Enough (sequence, head) pairs that workgroups look their sequence up by the rank of its length: many equal
+    lengths, empty and negative ones, whole and broken groups of 64 sequences, up to the limit and past it."""
+    lens = np.random.default_rng(B).choice([-3, 0, 0, 1, 16, 31, 31, 31, 64, 150], B).tolist()
+    lens[B // 2] = 160
+    c = make_case(B, 16, 64, 16, lens, B)
+    out, ref = run_both(c, dev, 32)       # 5 partitions of the longest: 16 x 5 x B wavefronts
+    check(out, ref)
+
+
 @pytest.mark.parametrize("BS", [16, 32])
 def test_decode_attention_block_sizes_and_many_partitions(dev, BS):
     lens = [700, 1, 257, 512, 31]
