@@ -1107,17 +1107,22 @@ extern "C" {
 // Tile rows / 64 and K split of a product beyond the row-streaming kernels' range: the pair with the least time by
 // this account (us), fitted to the 13B layer shapes at 20 row counts from 49 to 16384:
 //   rounds of workgroups over the CUs x (k-tiles of a workgroup x time of a k-tile + 5), and for a split 6 (the second
-//   launch and its workspace) + the fp32 parts written and read once at 4.2 TB/s.
-// A k-tile takes 0.85 / 1.0 / 1.3 / 1.5 us with 64 / 128 / 192 / 256 tile rows: 256 rows are the cheapest per row, the
+//   launch and its workspace) + the fp32 parts written and read once at 4.6 TB/s.
+// A k-tile takes 0.85 / 0.95 / 1.35 / 1.5 us with 64 / 128 / 192 / 256 tile rows: 256 rows are the cheapest per row, the
 // 128-row tile, whose 48 KiB stages fit the LDS three times, beats 192 rows wherever it does not need another round
 // (361 x 5120 on 20480 weight rows: 84 us; 192 rows 118, 256 rows 110).  More than 8 parts were slower than 8 at every
 // size (5120 x 5120, 64 rows: 22 us with 8, 27 with 12).
+// With weight rows a multiple of 4 KiB apart (fc2's 40 KiB, unpadded) the pieces of a k-tile meet in few memory channels
+// and a k-tile takes 1.3 / 1.36 / 1.8 / 1.85 us instead (361 x 20480 on 5120 weight rows: 126 us as 256 rows x 6 parts,
+// 140 as 128 rows x 4; at a longer pitch 95 and 91).
 struct TilePlan { int mi, splits; };
 static TailPlan tail_of(int mi, int64_t m, int64_t n, int64_t nk) {
   return mi == 4 ? plan_tail(((m + BM - 1) / BM) * (n / BN), nk) : TailPlan{0, 1, 0, 0};
 }
-static TilePlan tile_plan(int64_t m, int64_t n, int64_t k, bool may_split) {
-  static constexpr double kTileUs[4] = {0.85, 1.0, 1.3, 1.5};
+static bool pitch_4k(int64_t w_stride) { return w_stride * 2 % 4096 == 0; }
+static TilePlan tile_plan(int64_t m, int64_t n, int64_t k, bool may_split, bool few_channels) {
+  static constexpr double kUs[2][4] = {{0.85, 0.95, 1.35, 1.5}, {1.3, 1.36, 1.8, 1.85}};
+  const double* kTileUs = kUs[few_channels];
   const int64_t nk = k / BK;
   TilePlan best{4, 1};
   double least = 1e300;
@@ -1133,7 +1138,7 @@ static TilePlan tile_plan(int64_t m, int64_t n, int64_t k, bool may_split) {
         rounds += ways > 1 ? 1.0 / ways + 0.1 : 1.0;
       }
       double us = rounds * ((double)((nk + s - 1) / s) * kTileUs[mi - 1] + 5.0);
-      if (s > 1) us += 6.0 + (double)s * m * n * 8 / 4.2e6;
+      if (s > 1) us += 6.0 + (double)s * m * n * 8 / 4.6e6;
       if (us < least) { least = us; best = {mi, s}; }
     }
   }
@@ -1146,20 +1151,21 @@ int aps_linear_nt_splits(int64_t m, int64_t n, int64_t k) {
   if (m <= kRsMaxRows) return 1;  // streamed in one launch
   if (APS_KSPLIT && ksplit_covers(m, n, k)) return 1;   // K split inside the workgroups
   if (m <= kWsMaxRows) return weight_stream_plan(m, n, k).parts;
-  return tile_plan(m, n, k, true).splits;
+  // (the pitch of the weight rows is known at the launch only: room for either plan)
+  return std::max(tile_plan(m, n, k, true, false).splits, pitch_4k(k) ? tile_plan(m, n, k, true, true).splits : 1);
 }
 
 // Tail plan of a product, or none: only full-size tiles without a uniform K split are cut.
-static TailPlan tail_plan_of(int64_t m, int64_t n, int64_t k) {
+static TailPlan tail_plan_of(int64_t m, int64_t n, int64_t k, bool few_channels) {
   if (m <= kWsMaxRows || n <= 0 || k <= 0 || n % BN != 0 || k % BK != 0) return TailPlan{0, 1, 0, 0};
-  const TilePlan tp = tile_plan(m, n, k, true);
+  const TilePlan tp = tile_plan(m, n, k, true, few_channels);
   return tp.splits > 1 ? TailPlan{0, 1, 0, 0} : tail_of(tp.mi, m, n, k / BK);
 }
 
 int64_t aps_linear_nt_workspace_bytes(int64_t m, int64_t n, int64_t k) {
   const int s = aps_linear_nt_splits(m, n, k);
   if (s > 1) return (int64_t)s * m * n * 4;
-  return tail_plan_of(m, n, k).bytes;
+  return std::max(tail_plan_of(m, n, k, false).bytes, pitch_4k(k) ? tail_plan_of(m, n, k, true).bytes : 0);
 }
 
 // Where the rows of a gathered A operand live (see GemmArgs::row_src).
@@ -1189,7 +1195,8 @@ static int launch_gemm(const void* x, const void* weight, const void* bias, cons
   g.lda_b = x_stride * 2; g.ldw_b = w_stride * 2;
   g.m = m; g.n = n; g.k = k;
   const bool may_split = workspace && !(gs && m <= kWsMaxRows);  // (the split plan of few rows belongs to the streams)
-  const TilePlan plan = tile_plan(m, n, k, may_split);
+  const bool few_channels = pitch_4k(k) && pitch_4k(w_stride);
+  const TilePlan plan = tile_plan(m, n, k, may_split, few_channels);
   const int mi = plan.mi;
   g.tiles_m = (int)((m + 64 * mi - 1) / (64 * mi)); g.tiles_n = (int)(n / BN);
   g.out = om;
@@ -1256,7 +1263,7 @@ static int launch_gemm(const void* x, const void* weight, const void* bias, cons
   dim3 grid((unsigned)(per_xcd * kNumXcd), (unsigned)splits);
   g.tail_ways = 1;
   if (workspace && splits == 1) {
-    const TailPlan tp = tail_plan_of(m, n, k);
+    const TailPlan tp = tail_plan_of(m, n, k, few_channels);
     if (tp.ways > 1) {
       if (workspace_bytes < tp.bytes || (addr(workspace) & 15)) return APS_ERR_WORKSPACE;
       g.tail_partial = (float*)workspace;
