@@ -1124,23 +1124,26 @@ static TailPlan tail_of(int mi, int64_t m, int64_t n, int64_t nk) {
 static bool pitch_4k(int64_t w_stride) { return w_stride * 2 % 4096 == 0; }
 static TilePlan tile_plan(int64_t m, int64_t n, int64_t k, bool may_split, bool few_channels) {
   static constexpr double kUs[2][4] = {{0.85, 0.95, 1.35, 1.5}, {1.3, 1.36, 1.8, 1.85}};
-  const double* kTileUs = kUs[few_channels];
-  const int64_t nk = k / BK;
+  const int nk = (int)std::min<int64_t>(k / BK, 1 << 20);
+  const double part_us = (double)m * n * (8 / 4.6e6);
   TilePlan best{4, 1};
   double least = 1e300;
   for (int mi = 4; mi >= 1; --mi) {
     const int64_t bm = 64 * mi, tiles = ((m + bm - 1) / bm) * (n / BN);
-    const int max_splits = may_split ? (int)std::max<int64_t>(1, std::min<int64_t>(8, kNumCus / tiles)) : 1;
-    for (int s = 1; s <= max_splits; ++s) {
-      if (s > 1 && nk / s < 4) break;
-      const int64_t full = tiles * s / kNumCus, rest = tiles * s % kNumCus;
-      double rounds = (double)full;
-      if (rest) {
-        const int ways = may_split && s == 1 ? tail_of(mi, m, n, nk).ways : 1;
+    const double kt_us = kUs[few_channels][mi - 1];
+    if (!may_split || 2 * tiles > kNumCus) {   // no split: at least half of the CUs have a tile
+      double rounds = (double)(tiles / kNumCus);
+      if (tiles % kNumCus) {
+        const int ways = may_split ? tail_of(mi, m, n, nk).ways : 1;
         rounds += ways > 1 ? 1.0 / ways + 0.1 : 1.0;
       }
-      double us = rounds * ((double)((nk + s - 1) / s) * kTileUs[mi - 1] + 5.0);
-      if (s > 1) us += 6.0 + (double)s * m * n * 8 / 4.6e6;
+      const double us = rounds * (nk * kt_us + 5.0);
+      if (us < least) { least = us; best = {mi, 1}; }
+      continue;
+    }
+    const int most = std::min(8, kNumCus / (int)tiles);   // one round of workgroups
+    for (int s = 1; s <= most && (s == 1 || nk >= 4 * s); ++s) {
+      const double us = ((nk + s - 1) / s) * kt_us + 5.0 + (s > 1 ? 6.0 + s * part_us : 0.0);
       if (us < least) { least = us; best = {mi, s}; }
     }
   }
@@ -1157,17 +1160,19 @@ int aps_linear_nt_splits(int64_t m, int64_t n, int64_t k) {
   return std::max(tile_plan(m, n, k, true, false).splits, pitch_4k(k) ? tile_plan(m, n, k, true, true).splits : 1);
 }
 
-// Tail plan of a product, or none: only full-size tiles without a uniform K split are cut.
-static TailPlan tail_plan_of(int64_t m, int64_t n, int64_t k, bool few_channels) {
-  if (m <= kWsMaxRows || n <= 0 || k <= 0 || n % BN != 0 || k % BK != 0) return TailPlan{0, 1, 0, 0};
-  const TilePlan tp = tile_plan(m, n, k, true, few_channels);
-  return tp.splits > 1 ? TailPlan{0, 1, 0, 0} : tail_of(tp.mi, m, n, k / BK);
-}
-
 int64_t aps_linear_nt_workspace_bytes(int64_t m, int64_t n, int64_t k) {
-  const int s = aps_linear_nt_splits(m, n, k);
-  if (s > 1) return (int64_t)s * m * n * 4;
-  return std::max(tail_plan_of(m, n, k, false).bytes, pitch_4k(k) ? tail_plan_of(m, n, k, true).bytes : 0);
+  if (m <= kWsMaxRows || n <= 0 || k <= 0 || n % BN != 0 || k % BK != 0) {
+    const int s = aps_linear_nt_splits(m, n, k);
+    return s > 1 ? (int64_t)s * m * n * 4 : 0;
+  }
+  int s = 1;
+  int64_t tail = 0;
+  for (int few = 0; few <= (pitch_4k(k) ? 1 : 0); ++few) {
+    const TilePlan tp = tile_plan(m, n, k, true, few);
+    s = std::max(s, tp.splits);
+    if (tp.splits == 1) tail = std::max(tail, tail_of(tp.mi, m, n, k / BK).bytes);   // only unsplit tiles are cut
+  }
+  return s > 1 ? (int64_t)s * m * n * 4 : tail;
 }
 
 // Where the rows of a gathered A operand live (see GemmArgs::row_src).
@@ -1196,11 +1201,6 @@ static int launch_gemm(const void* x, const void* weight, const void* bias, cons
   g.a = (const char*)x; g.w = (const char*)weight; g.bias = bias;
   g.lda_b = x_stride * 2; g.ldw_b = w_stride * 2;
   g.m = m; g.n = n; g.k = k;
-  const bool may_split = workspace && !(gs && m <= kWsMaxRows);  // (the split plan of few rows belongs to the streams)
-  const bool few_channels = pitch_4k(k) && pitch_4k(w_stride);
-  const TilePlan plan = tile_plan(m, n, k, may_split, few_channels);
-  const int mi = plan.mi;
-  g.tiles_m = (int)((m + 64 * mi - 1) / (64 * mi)); g.tiles_n = (int)(n / BN);
   g.out = om;
   hipStream_t s = (hipStream_t)stream;
   if (gs) {   // only the tile kernel reads its A rows through a row map
@@ -1250,6 +1250,10 @@ static int launch_gemm(const void* x, const void* weight, const void* bias, cons
       APS_LAUNCH(skinny_nt_kernel<false>, grid, dim3(kSkWaves * 64), 0, s, g, per_wave);
     return launch_status();
   }
+  const bool may_split = workspace && !(gs && m <= kWsMaxRows);  // (the split plan of few rows belongs to the streams)
+  const TilePlan plan = tile_plan(m, n, k, may_split, pitch_4k(k) && pitch_4k(w_stride));
+  const int mi = plan.mi;
+  g.tiles_m = (int)((m + 64 * mi - 1) / (64 * mi)); g.tiles_n = (int)(n / BN);
   const int64_t total = (int64_t)g.tiles_m * g.tiles_n;
   if (total >= ((int64_t)1 << 30)) return APS_ERR_UNSUPPORTED;
   const int64_t per_xcd = (total + kNumXcd - 1) / kNumXcd;
@@ -1265,7 +1269,7 @@ static int launch_gemm(const void* x, const void* weight, const void* bias, cons
   dim3 grid((unsigned)(per_xcd * kNumXcd), (unsigned)splits);
   g.tail_ways = 1;
   if (workspace && splits == 1) {
-    const TailPlan tp = tail_plan_of(m, n, k, few_channels);
+    const TailPlan tp = m > kWsMaxRows ? tail_of(mi, m, n, nk_all) : TailPlan{0, 1, 0, 0};
     if (tp.ways > 1) {
       if (workspace_bytes < tp.bytes || (addr(workspace) & 15)) return APS_ERR_WORKSPACE;
       g.tail_partial = (float*)workspace;
