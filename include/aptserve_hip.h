@@ -488,7 +488,8 @@ int aps_build_prefill_metadata(
  * workspace (nullable): fp32 scratch of aps_linear_nt_workspace_bytes(m,n,k)
  * bytes, 16-byte aligned, owned by the caller.  With it, a problem whose output
  * tiles leave CUs idle (a decode step's rows: anything from 3 rows up to a few
- * hundred) is split along K into aps_linear_nt_splits(m,n,k) partial products
+ * hundred) is split along K into at most aps_linear_nt_splits(m,n,k) partial
+ * products (fewer when the pitch of the weight rows calls for other tiles)
  * that a second kernel adds (in fp32, then bias, then one rounding); without it
  * a single-launch kernel runs.  A workspace that is passed but too small or
  * misaligned is an error (APS_ERR_WORKSPACE), never a silent fallback.
