@@ -52,20 +52,6 @@ struct PrefillArgs {
 template <int D>
 constexpr int prefill_lds_bytes() { return 2 * 2 * BKV * D * 2; }
 
-// One 1 KiB copy global -> LDS: lane l's 16 bytes at offset voff + soff of the buffer land at lds + 16 l.  From assembly:
-// the compiler, seeing a copy into LDS, waits for every load in flight before the next LDS read of any stage.
-__device__ __forceinline__ void copy_to_lds(uint32_t lds, const u32x4& rsrc, uint32_t voff, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
-               : "memory");
-}
-__device__ __forceinline__ u32x4 raw_rsrc(const char* p, int64_t bytes) {   // make_rsrc for the assembly
-  const uint64_t a = (uint64_t)p;
-  const uint32_t n = bytes <= 0 ? 0u : (bytes > 0xffffffffll ? 0xffffffffu : (uint32_t)bytes);
-  return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)),
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)n), 0x00020000u};
-}
-
 // Where the keys come from: packed rows; blocks of 16, 32, 64, ... tokens, so that 16 consecutive keys from a multiple
 // of 16 on lie together in one block; the same key by key, for row pitches past 32 MiB and blocks of any other size.
 enum KeySource { kPacked, kPaged16, kPackedAny, kPagedAny };
@@ -175,8 +161,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       const u32x4 rv = raw_rsrc(v_base + kv0 * a.v_stride_b, left * a.v_stride_b + D * 2);
 #pragma unroll
       for (int j = 0; j < PER; ++j) {
-        copy_to_lds(dst + j * 4096, rk, k_lane, j * 4 * RPC * (uint32_t)a.k_stride_b);
-        copy_to_lds(dst + kTile + j * 4096, rv, v_lane, j * 4 * RPC * (uint32_t)a.v_stride_b);
+        copy2_to_lds(dst + j * 4096, rk, k_lane, dst + kTile + j * 4096, rv, v_lane, j * 4 * RPC * (uint32_t)a.k_stride_b,
+                     j * 4 * RPC * (uint32_t)a.v_stride_b);
       }
     } else if constexpr (SRC == kPaged16) {
 #pragma unroll
@@ -187,6 +173,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
         // what a block holds past its sequence may be anything, and a zero probability does not cancel a NaN: the buffer
         // ends with the sequence's last row and the others read as zeros
         const int64_t bytes = min(15, len - 1 - 16 * g) * a.k_stride_b + D * 2;
+        // (one copy at a time: both descriptors before the first copy cost 2 to 3 % more)
         copy_to_lds(dst + j * 4096, raw_rsrc(k_base + start, bytes), k_lane, 0);
         copy_to_lds(dst + kTile + j * 4096, raw_rsrc(v_base + start, bytes), v_lane, 0);
       }

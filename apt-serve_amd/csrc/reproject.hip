@@ -890,12 +890,7 @@ __global__ __launch_bounds__(kScThreads) void weight_ksplit_kernel(const GemmArg
   // (The copies are issued from assembly: the compiler, seeing a copy into LDS and a later LDS read, waits for
   // every load in flight before the first read, weight rows included; it cannot know which bytes the copy wrote.)
   const int64_t head_off = g.head_rows ? (n0 / g.head_rows) * g.x_head_stride_b : 0;
-  const uint64_t xa = (uint64_t)(g.a + head_off);
-  u32x4 rsrc;   // buffer descriptor over the m rows of x
-  rsrc[0] = __builtin_amdgcn_readfirstlane((uint32_t)xa);
-  rsrc[1] = __builtin_amdgcn_readfirstlane((uint32_t)(xa >> 32));
-  rsrc[2] = __builtin_amdgcn_readfirstlane((uint32_t)((m - 1) * g.lda_b + g.k * 2));
-  rsrc[3] = 0x00020000u;
+  const u32x4 rsrc = raw_rsrc(g.a + head_off, (m - 1) * g.lda_b + g.k * 2);   // the m rows of x
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
 #pragma unroll
   for (int j = 0; j < P; ++j) {   // (8 rows x P copies / 8 wavefronts = P copies per wavefront at most)
@@ -904,11 +899,8 @@ __global__ __launch_bounds__(kScThreads) void weight_ksplit_kernel(const GemmArg
     if (r < m) {
       const int slot = 64 * jg + lane;
       const int piece = (slot & ~15) | ((slot ^ r) & 15);
-      asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds"   // (m0 needs one wait state)
-                   :
-                   : "s"(__builtin_amdgcn_readfirstlane(lds_base + (uint32_t)(r * kRowBytes + jg * 1024))),
-                     "v"((uint32_t)(r * g.lda_b) + (uint32_t)(piece * 16)), "s"(rsrc)
-                   : "memory");
+      copy_to_lds(__builtin_amdgcn_readfirstlane(lds_base + (uint32_t)(r * kRowBytes + jg * 1024)), rsrc,
+                  (uint32_t)(r * g.lda_b) + (uint32_t)(piece * 16), 0);
     }
   }
   __builtin_amdgcn_sched_barrier(0);

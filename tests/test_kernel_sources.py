@@ -1,0 +1,38 @@
+"""Rules of the kernel sources that a compiler does not check (host only)."""
+import re
+from pathlib import Path
+
+import pytest
+
+CSRC = Path(__file__).resolve().parent.parent / "apt-serve_amd" / "csrc"
+SOURCES = sorted(p for p in CSRC.rglob("*") if p.suffix in (".hip", ".h"))
+
+
+def asm_statements(text):
+    """(instructions, rest of the statement) of every inline assembly statement."""
+    text = re.sub(r"//[^\n]*", "", text)
+    for m in re.finditer(r'\basm\s+volatile\s*\(((?:[^()"]|"(?:\\.|[^"\\])*"|\((?:[^()"]|"(?:\\.|[^"\\])*"|\([^()]*\))*\))*)\)\s*;', text):
+        body = m.group(1)
+        code = re.match(r'\s*((?:"(?:\\.|[^"\\])*"\s*)+)', body)
+        if code:
+            yield "".join(re.findall(r'"((?:\\.|[^"\\])*)"', code.group(1))), body[code.end():]
+
+
+def test_assembly_that_writes_m0_says_so_and_waits():
+    """A copy global -> LDS takes its LDS address from m0 and its descriptor from scalar registers.  The compiler keeps
+    m0 for its own use unless the statement names it, and it cannot put wait states inside a statement: one is needed
+    between a write of m0 and the copy, five between a scalar register written by a vector instruction and the copy."""
+    found = 0
+    for p in SOURCES:
+        for code, rest in asm_statements(p.read_text()):
+            ins = [i.strip() for i in re.split(r"\\n|;", code) if i.replace("\\t", "").strip()]
+            ins = [i.replace("\\t", " ").strip() for i in ins]
+            writes = [i for i, x in enumerate(ins) if re.match(r"s_mov_b32 m0\b", x)]
+            if not writes:
+                continue
+            found += 1
+            assert '"m0"' in rest.rsplit(":", 1)[-1], f"{p.name}: m0 is not in the clobber list of {code!r}"
+            load = next(i for i, x in enumerate(ins) if x.startswith("buffer_load") or x.startswith("global_load"))
+            states = sum(int(x.split()[1]) + 1 if x.startswith("s_nop") else 1 for x in ins[:load])
+            assert states >= 5, f"{p.name}: {states} wait states before the copy in {code!r}"
+    assert found >= 1
