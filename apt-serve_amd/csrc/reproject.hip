@@ -289,7 +289,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       for (int j = 0; j < 4; ++j) acc[i][j] = mfma16<BF16>(af[i], wf[j], acc[i][j]);
   };
   auto interleave = [&]() {  // scheduling hint: the 12 LDS reads spread over the 32 MFMA of a k-step
-    if constexpr (MI != 4) return;  // the small tiles are bound by the weight stream: the compiler's order will do
+    if constexpr (MI != 4) return;  // the smaller tiles keep the compiler's order: reads and products of a k-step one after the other
 #pragma unroll
     for (int r = 0; r < 8; ++r) {
       __builtin_amdgcn_sched_group_barrier(0x008, 3, 0); __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
@@ -1099,44 +1099,49 @@ using namespace aps;
 extern "C" {
 
 // Tile rows / 64 and K split of a product beyond the row-streaming kernels' range: the pair with the least time by
-// this account (us), fitted to the 13B layer shapes at 20 row counts from 49 to 16384:
-//   rounds of workgroups over the CUs x (k-tiles of a workgroup x time of a k-tile + 5), and for a split 6 (the second
-//   launch and its workspace) + the fp32 parts written and read once at 4.6 TB/s.
-// A k-tile takes 0.85 / 0.95 / 1.35 / 1.5 us with 64 / 128 / 192 / 256 tile rows: 256 rows are the cheapest per row, the
-// 128-row tile, whose 48 KiB stages fit the LDS three times, beats 192 rows wherever it does not need another round
-// (361 x 5120 on 20480 weight rows: 84 us; 192 rows 118, 256 rows 110).  More than 8 parts were slower than 8 at every
-// size (5120 x 5120, 64 rows: 22 us with 8, 27 with 12).
-// With weight rows a multiple of 4 KiB apart (fc2's 40 KiB, unpadded) the pieces of a k-tile meet in few memory channels
-// and a k-tile takes 1.3 / 1.36 / 1.8 / 1.85 us instead (361 x 20480 on 5120 weight rows: 126 us as 256 rows x 6 parts,
-// 140 as 128 rows x 4; at a longer pitch 95 and 91).
+// this account (us).  Its numbers are fitted, as a whole, to every tile size and K split timed on 23 weight shapes (256 to
+// 20480 rows of 768 to 65536, close and padded) at 36 row counts from 49 to 8192; the pair it picks takes 1.2 % longer than
+// the fastest one measured on average, more than 10 % longer at 31 of 1188 products:
+//   rounds of workgroups x (k-tiles of a workgroup x time of a k-tile + 3),
+//   for a split 4 + 0.65 per part (the second launch reads them one after the other) + the fp32 parts written and read
+//   once at 3.8 TB/s, for a cut last round its short k-range, 2, and its parts at the same rate.
+// The parts of a tile run on one XCD, so a round takes ceil(tiles / 8) x parts <= 32: 20 tiles x 12 parts are two rounds
+// though 240 are fewer than the CUs (5120 x 20480, 64 rows: 66 us; with 10 parts 48).  Few tiles of a long K take many
+// parts (256 weight rows of 20480, 64 rows: 22 us with 32 parts, 46 with 8).
+// Of the tile sizes the 128-row one, whose 48 KiB stages fit the LDS three times, beats 192 rows wherever it does not need
+// another round (361 x 5120 on 20480 weight rows: 82 us; 192 rows 111, 256 rows 109); 256 rows are the cheapest per row.
+// Where the weight rows lie a multiple of 2 KiB apart that is not a power of two, the 128-byte pieces that a k-tile takes of
+// many rows meet in fewer memory channels: a little slower for an odd multiple (10 KiB: 8 %), up to 60 % for a multiple of
+// 4 KiB (361 rows, 128-row tiles, us per k-tile: 12 KiB 1.06, 24 KiB 1.17, 40 KiB 1.29; 4, 8, 16, 32 KiB and every pitch
+// 128 bytes longer 0.78 to 0.9).  fc2 of 361 rows (40 KiB): 131 us as 192 rows x 6 parts, 127 as 256 x 6, 139 as 128 x 4;
+// at the longer pitch 100, 96 and 92.
+enum RowPitch { kPitchFree, kPitch2K, kPitch4K };
+static RowPitch row_pitch(int64_t stride) {
+  const int64_t b = stride * 2;
+  return b % 2048 != 0 || (b & (b - 1)) == 0 ? kPitchFree : (b % 4096 == 0 ? kPitch4K : kPitch2K);
+}
 struct TilePlan { int mi, splits; };
 static TailPlan tail_of(int mi, int64_t m, int64_t n, int64_t nk) {
   return mi == 4 ? plan_tail(((m + BM - 1) / BM) * (n / BN), nk) : TailPlan{0, 1, 0, 0};
 }
-static bool pitch_4k(int64_t w_stride) { return w_stride * 2 % 4096 == 0; }
-static TilePlan tile_plan(int64_t m, int64_t n, int64_t k, bool may_split, bool few_channels) {
-  static constexpr double kUs[2][4] = {{0.85, 0.95, 1.35, 1.5}, {1.3, 1.36, 1.8, 1.85}};
+static TilePlan tile_plan(int64_t m, int64_t n, int64_t k, bool may_split, RowPitch pitch) {
+  static constexpr double kUs[3][4] = {{0.91, 1.13, 1.63, 1.79}, {0.94, 1.15, 1.57, 1.7}, {1.9, 2.13, 2.62, 3.4}};
+  static constexpr int kXcdCus = kNumCus / kNumXcd;
   const int nk = (int)std::min<int64_t>(k / BK, 1 << 20);
-  const double part_us = (double)m * n * (8 / 4.6e6);
+  const double us_per_byte = 0.26e-6, part_us = (double)m * n * 8 * us_per_byte;
   TilePlan best{4, 1};
   double least = 1e300;
   for (int mi = 4; mi >= 1; --mi) {
-    const int64_t bm = 64 * mi, tiles = ((m + bm - 1) / bm) * (n / BN);
-    const double kt_us = kUs[few_channels][mi - 1];
-    if (!may_split || 2 * tiles > kNumCus) {   // no split: at least half of the CUs have a tile
-      double rounds = (double)(tiles / kNumCus);
-      if (tiles % kNumCus) {
-        const int ways = may_split ? tail_of(mi, m, n, nk).ways : 1;
-        rounds += ways > 1 ? 1.0 / ways + 0.1 : 1.0;
-      }
-      const double us = rounds * (nk * kt_us + 5.0);
-      if (us < least) { least = us; best = {mi, 1}; }
-      continue;
-    }
-    const int most = std::min(8, kNumCus / (int)tiles);   // one round of workgroups
-    for (int s = 1; s <= most && (s == 1 || nk >= 4 * s); ++s) {
-      const double us = ((nk + s - 1) / s) * kt_us + 5.0 + (s > 1 ? 6.0 + s * part_us : 0.0);
-      if (us < least) { least = us; best = {mi, s}; }
+    const int64_t bm = 64 * mi, tiles = ((m + bm - 1) / bm) * (n / BN), per_xcd = (tiles + kNumXcd - 1) / kNumXcd;
+    const double kt_us = kUs[pitch][mi - 1], round_us = nk * kt_us + 3.0;
+    double us = (double)((per_xcd + kXcdCus - 1) / kXcdCus) * round_us;
+    const TailPlan tp = may_split ? tail_of(mi, m, n, nk) : TailPlan{0, 1, 0, 0};
+    if (tp.ways > 1) us = (double)(tp.from / kNumCus) * round_us + tp.kt * kt_us + 5.0 + tp.bytes * 2 * us_per_byte;
+    if (us < least) { least = us; best = {mi, 1}; }
+    const int most = may_split ? (int)std::min<int64_t>(kXcdCus / per_xcd, nk / 4) : 1;   // one round, 4 k-tiles a part
+    for (int s = 2; s <= most; ++s) {
+      const double split_us = ((nk + s - 1) / s) * kt_us + 7.0 + s * (0.65 + part_us);
+      if (split_us < least) { least = split_us; best = {mi, s}; }
     }
   }
   return best;
@@ -1148,8 +1153,8 @@ int aps_linear_nt_splits(int64_t m, int64_t n, int64_t k) {
   if (m <= kRsMaxRows) return 1;  // streamed in one launch
   if (APS_KSPLIT && ksplit_covers(m, n, k)) return 1;   // K split inside the workgroups
   if (m <= kWsMaxRows) return weight_stream_plan(m, n, k).parts;
-  // (the pitch of the weight rows is known at the launch only: room for either plan)
-  return std::max(tile_plan(m, n, k, true, false).splits, pitch_4k(k) ? tile_plan(m, n, k, true, true).splits : 1);
+  // (the pitch of the weight rows is known at the launch only: room for close rows and for padded ones)
+  return std::max(tile_plan(m, n, k, true, kPitchFree).splits, tile_plan(m, n, k, true, row_pitch(k)).splits);
 }
 
 int64_t aps_linear_nt_workspace_bytes(int64_t m, int64_t n, int64_t k) {
@@ -1157,14 +1162,13 @@ int64_t aps_linear_nt_workspace_bytes(int64_t m, int64_t n, int64_t k) {
     const int s = aps_linear_nt_splits(m, n, k);
     return s > 1 ? (int64_t)s * m * n * 4 : 0;
   }
-  int s = 1;
-  int64_t tail = 0;
-  for (int few = 0; few <= (pitch_4k(k) ? 1 : 0); ++few) {
-    const TilePlan tp = tile_plan(m, n, k, true, few);
-    s = std::max(s, tp.splits);
-    if (tp.splits == 1) tail = std::max(tail, tail_of(tp.mi, m, n, k / BK).bytes);   // only unsplit tiles are cut
+  int64_t bytes = 0;
+  for (const RowPitch pitch : {kPitchFree, row_pitch(k)}) {
+    const TilePlan tp = tile_plan(m, n, k, true, pitch);
+    // (only unsplit tiles are cut)
+    bytes = std::max(bytes, tp.splits > 1 ? (int64_t)tp.splits * m * n * 4 : tail_of(tp.mi, m, n, k / BK).bytes);
   }
-  return s > 1 ? (int64_t)s * m * n * 4 : tail;
+  return bytes;
 }
 
 // Where the rows of a gathered A operand live (see GemmArgs::row_src).
@@ -1243,7 +1247,8 @@ static int launch_gemm(const void* x, const void* weight, const void* bias, cons
     return launch_status();
   }
   const bool may_split = workspace && !(gs && m <= kWsMaxRows);  // (the split plan of few rows belongs to the streams)
-  const TilePlan plan = tile_plan(m, n, k, may_split, pitch_4k(k) && pitch_4k(w_stride));
+  const RowPitch pitch = row_pitch(w_stride) == row_pitch(k) ? row_pitch(k) : kPitchFree;   // (what the workspace allows for)
+  const TilePlan plan = tile_plan(m, n, k, may_split, pitch);
   const int mi = plan.mi;
   g.tiles_m = (int)((m + 64 * mi - 1) / (64 * mi)); g.tiles_n = (int)(n / BN);
   const int64_t total = (int64_t)g.tiles_m * g.tiles_n;

@@ -154,6 +154,19 @@ def test_linear_workspace_planning_is_host_only_and_consistent():
     assert lib.aps_linear_nt_splits(0, 5120, 5120) == 1 and lib.aps_linear_nt_workspace_bytes(0, 5120, 5120) == 0
 
 
+def test_linear_k_split_fills_one_round_of_the_xcds():
+    """Few output tiles of a long K are split until the CUs are busy, and never into more parts than one round holds:
+    the parts of a tile run on one XCD, 32 CUs, and tiles are dealt to the 8 XCDs evenly."""
+    lib = _lib.load()
+    for m in (49, 64):                                          # 64-row tiles: n / 256 of them
+        assert lib.aps_linear_nt_splits(m, 256, 20480) >= 16
+        for n, k in [(256, 20480), (512, 8192), (2048, 8192), (5120, 5120), (5120, 20480), (4096, 16384)]:
+            s = lib.aps_linear_nt_splits(m, n, k)
+            assert s > 1 and s * -(-(n // 256) // 8) <= 32
+    # 384 tiles of 256 rows: the parts of a cut last round cost more than 512 tiles of 192 rows in two whole ones
+    assert lib.aps_linear_nt_workspace_bytes(3000, 8192, 2048) == 0
+
+
 def test_absorbed_attention_workspace_planning_is_host_only():
     """The workspace of the attention on hidden rows covers at least its named buffers (query image and context
     rows: n*H*Hd 16-bit each; fp32 scores over the padded longest sequence; a row of zeros), grows with the

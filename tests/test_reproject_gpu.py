@@ -57,6 +57,24 @@ def test_linear_nt_ring_of_k_tiles(dev, M, nk, dtype):
     check(ops.linear_nt(x.to(dev), w.to(dev), b.to(dev)), OR._linear_fp32(x, w, b), dtype)
 
 
+@pytest.mark.parametrize("M", [64, 100, 200, 361, 512])       # split 64-, 128-, 192- and 256-row tiles
+@pytest.mark.parametrize("N,K", [(5120, 20480), (5120, 20544), (256, 20480), (1024, 6144)])
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+def test_linear_nt_k_split_of_tiles_at_both_row_pitches(dev, M, N, K, dtype):
+    """K splits (last parts shorter where the k-tiles do not divide) with rows close together, where K of 20480 and 6144
+    has a plan of its own, and 128 bytes further apart: sampled rows against 64 bits, and the two against each other."""
+    assert ops._lib.load().aps_linear_nt_splits(M, N, K) > 1
+    g = torch.Generator(device=dev).manual_seed(M + K)
+    x, w, b = (torch.randn(*s, generator=g, device=dev).mul_(a).to(dtype) for s, a in (((M, K), 1), ((N, K), 0.02), ((N,), 0.2)))
+    rows = torch.tensor(sorted({0, 1, 15, M // 3, M // 2, M - 2, M - 1}), device=dev)
+    ref = (x[rows].double() @ w.double().t() + b.double()).float().cpu()
+
+    def pitched(t):
+        return torch.empty(t.size(0), K + 64, dtype=dtype, device=dev)[:, :K].copy_(t)
+    for xx, ww in ((x, w), (x, pitched(w)), (pitched(x), pitched(w))):
+        check(ops.linear_nt(xx, ww, b)[rows], ref, dtype)
+
+
 @pytest.mark.parametrize("M", [3, 8, 16, 17, 32, 33, 48])
 @pytest.mark.parametrize("N,K", [(256, 64), (512, 1600), (1024, 2048), (2560, 5120), (16896, 1024), (20992, 512)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
