@@ -69,7 +69,11 @@ __device__ __forceinline__ void copy_to_lds(uint32_t lds, const u32x4& rsrc, uin
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
                : "memory", "m0");
 }
-// Two of them under one wait: the packed prompt attention runs as long as without it (4 x 2048 tokens 240 us).
+// The same with an address per lane.
+__device__ __forceinline__ void copy_lanes_to_lds(uint32_t lds, const char* p) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory", "m0");
+}
+// Two of copy_to_lds under one wait: the packed prompt attention runs as long as without it (4 x 2048 tokens 240 us).
 __device__ __forceinline__ void copy2_to_lds(uint32_t lds0, const u32x4& rsrc0, uint32_t voff0, uint32_t lds1, const u32x4& rsrc1,
                                              uint32_t voff1, uint32_t soff0, uint32_t soff1) {
   asm volatile(

@@ -117,7 +117,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
   // Copies.  A wave-wide copy moves RPC = 64 / KCH key rows; wavefront w makes copies w, w + 4, ... of K's and of V's, so
   // that a lane always moves the same row of a group of 16 keys (and has one swizzle), and the group is wave-uniform.
-  // A lane keeps its offset inside a tile; the tile's (kPacked) or the group's (kPaged16) start is scalar work.  (Every
+  // A lane keeps its offset inside a tile; the tile's (kPacked) or the group's (kPaged16) start is scalar work.  (Key by key,
+  // every lane makes its addresses; the block numbers are loaded a tile ahead too.  Blocks of 48: 4 x 200 tokens on 4000
+  // cached of 40 x 128 heads 57.6 -> 48.5 us against copies through the builtin, 8 x 1000 on 1000 564 -> 533.)  (Every
   // lane multiplying out 64-bit offsets of twelve rows a tile, 130 quarter-rate multiplications with the divisions of a
   // block table, cost as much as the softmax: 274 against 251 us for 4 x 2048 tokens.)
   constexpr int RPC = 64 / KCH, PER = BKV / RPC / 4;   // key rows of a copy; copies per wavefront and operand
@@ -133,20 +135,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     const int64_t b = blk < 0 ? 0 : (blk >= a.num_blocks ? a.num_blocks - 1 : (int64_t)blk);
     return b * a.block_stride_b;
   };
-  // kPackedAny, kPagedAny: byte offset of key gk of the sequence from k_base / v_base
-  auto key_off = [&](int gk, int64_t stride_b) -> int64_t {
-    if constexpr (!PAGED) return (int64_t)gk * stride_b;
-    const int bi = gk / a.block_size;
-    return block_start(a.block_tables[(int64_t)seq * a.table_stride + bi]) + (int64_t)(gk - bi * a.block_size) * stride_b;
-  };
-  // kPaged16: the blocks of the wavefront's groups of the next tile to be copied (past the sequence: its last group)
+  // kPaged16: the blocks of the wavefront's groups of the next tile to be copied (past the sequence: its last group).
+  // kPagedAny: those of the lane's keys, and their places in them (past the sequence: its last key).
   const int last_group = (len - 1) >> 4;
   auto group_of = [&](int kv0, int j) { return min((kv0 >> 4) + (KCH == 16 ? j : (wave_u >> 1) + 2 * j), last_group); };
-  int blocks[PER];
+  auto key_of = [&](int kv0, int j) { return min(kv0 + key0 + j * 4 * RPC, len - 1); };
+  int blocks[PER], in_block[PER];
   auto load_blocks = [&](int kv0) {
-    if constexpr (SRC == kPaged16) {
 #pragma unroll
-      for (int j = 0; j < PER; ++j) blocks[j] = table[group_of(kv0, j) >> a.groups_shift];
+    for (int j = 0; j < PER; ++j) {
+      if constexpr (SRC == kPaged16) blocks[j] = table[group_of(kv0, j) >> a.groups_shift];
+      if constexpr (SRC == kPagedAny) {
+        const int bi = key_of(kv0, j) / a.block_size;
+        blocks[j] = a.block_tables[(int64_t)seq * a.table_stride + bi];
+        in_block[j] = key_of(kv0, j) - bi * a.block_size;
+      }
     }
   };
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
@@ -179,17 +182,24 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
       }
       load_blocks(kv0 + BKV);
     } else {
+      if constexpr (PAGED) {   // the block numbers have arrived before the first copy is counted
+#pragma unroll
+        for (int j = 0; j < PER; ++j) asm volatile("" : "+v"(blocks[j]));
+      }
 #pragma unroll
       for (int j = 0; j < PER; ++j) {
-        const int gk = min(kv0 + key0 + j * 4 * RPC, len - 1);
-        char* const l = lds + stage * kStage + (wave_u + 4 * j) * 1024;
-        __builtin_amdgcn_global_load_lds(
-            (const __attribute__((address_space(1))) void*)(k_base + key_off(gk, a.k_stride_b) + (slot ^ k_swz(key0)) * 16),
-            (__attribute__((address_space(3))) void*)l, 16, 0, 0);
-        __builtin_amdgcn_global_load_lds(
-            (const __attribute__((address_space(1))) void*)(v_base + key_off(gk, a.v_stride_b) + (slot ^ v_swz(key0)) * 16),
-            (__attribute__((address_space(3))) void*)(l + kTile), 16, 0, 0);
+        int64_t k_off, v_off;
+        if constexpr (PAGED) {
+          k_off = block_start(blocks[j]) + (int64_t)in_block[j] * a.k_stride_b;
+          v_off = k_off;   // (both caches have the same strides)
+        } else {
+          k_off = (int64_t)key_of(kv0, j) * a.k_stride_b;
+          v_off = (int64_t)key_of(kv0, j) * a.v_stride_b;
+        }
+        copy_lanes_to_lds(dst + j * 4096, k_base + k_off + (slot ^ k_swz(key0)) * 16);
+        copy_lanes_to_lds(dst + kTile + j * 4096, v_base + v_off + (slot ^ v_swz(key0)) * 16);
       }
+      load_blocks(kv0 + BKV);
     }
   };
   // V^T fragment (16 d of tile t, keys of this lane's quad in key tile kt): the lane gives the address of its share of the

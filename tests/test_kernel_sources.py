@@ -2,8 +2,6 @@
 import re
 from pathlib import Path
 
-import pytest
-
 CSRC = Path(__file__).resolve().parent.parent / "apt-serve_amd" / "csrc"
 SOURCES = sorted(p for p in CSRC.rglob("*") if p.suffix in (".hip", ".h"))
 
@@ -36,3 +34,10 @@ def test_assembly_that_writes_m0_says_so_and_waits():
             states = sum(int(x.split()[1]) + 1 if x.startswith("s_nop") else 1 for x in ins[:load])
             assert states >= 5, f"{p.name}: {states} wait states before the copy in {code!r}"
     assert found >= 1
+
+
+def test_prompt_attention_copies_a_tile_ahead():
+    """Its copies into LDS are in flight while the tile before is multiplied.  Issued through the compiler's builtin they
+    are waited for before the next LDS read of any stage, so every path issues them from assembly."""
+    code = re.sub(r"//[^\n]*", "", (CSRC / "prefill_attention.hip").read_text())
+    assert not re.search(r"__builtin_amdgcn_\w*load\w*_lds", code)
