@@ -351,7 +351,8 @@ int launch_prefill(PrefillArgs& a, bool paged, int64_t num_seqs, int64_t max_seq
   // with 32 queries a wavefront and 1.5 with 16, so as long as the CUs are not full the shorter ones finish first (12
   // heads, 2048 tokens: 34 -> 26 us; 40 heads, 361 tokens 11.1 -> 9.9, 4 x 50 on a prefix of 4000 61 -> 49); full CUs
   // lose by reading every fragment for half the queries (40 heads, 1400 tokens 26 -> 28, 4 x 2048 221 -> 304).
-  const int qt = num_heads * (a.num_tokens / 128 + num_seqs) <= 384 ? 1 : 2;
+  // (A longest sequence stated far beyond the tokens, within the grid's limit at 128 queries only, is taken at 128.)
+  const int qt = num_heads * (a.num_tokens / 128 + num_seqs) <= 384 && max_seqlen_q <= 65535 * 64 ? 1 : 2;
   const int64_t q_tiles = (max_seqlen_q + 64 * qt - 1) / (64 * qt);
   if (q_tiles > 65535 || num_seqs > 65535 || num_heads > 65535) return APS_ERR_UNSUPPORTED;
   const dim3 grid((unsigned)num_heads, (unsigned)num_seqs, (unsigned)q_tiles);

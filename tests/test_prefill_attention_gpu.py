@@ -157,6 +157,18 @@ def test_packed_rows_past_the_sequence_and_wide_row_pitch(dev):
     assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("max_seqlen", [65535 * 64, 65535 * 64 + 1, 65535 * 128])
+def test_longest_sequence_stated_beyond_the_tokens(dev, max_seqlen):
+    """The longest length is a bound: a small step accepts any that the grid takes with 128 queries a workgroup."""
+    H, D, n = 2, 64, 70
+    q, k, v = (randn((n, H, D), 23 + i).to(dev) for i in range(3))
+    cu = torch.tensor([0, n], dtype=torch.int32, device=dev)
+    a, b = (ops.flash_attn_varlen_func(q, k, v, cu_seqlens_q=cu, max_seqlen_q=m, softmax_scale=0.125) for m in (n, max_seqlen))
+    assert torch.allclose(a.float(), b.float(), atol=2e-3, rtol=2e-3)   # (64 and 128 queries a workgroup: other key order)
+    with pytest.raises(RuntimeError):
+        ops.flash_attn_varlen_func(q, k, v, cu_seqlens_q=cu, max_seqlen_q=65535 * 128 + 1, softmax_scale=0.125)
+
+
 def test_prefix_attention_block_size_32_and_argument_errors(dev):
     run_prefix(dev, [100, 45], [33, 45], 4, 64, BS=32, seed=3)
     from test_oracle_attention import build_paged
