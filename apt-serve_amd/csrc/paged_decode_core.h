@@ -371,13 +371,12 @@ __global__ __launch_bounds__(64) void paged_decode_kernel(const AttnArgs a) {
   }
 }
 
-constexpr int kRankInKernelMax = 512;  // up to this many sequences a wavefront finds its sequence itself
+constexpr int kRankInKernelMax = 512;  // up to this many sequences a workgroup finds its sequence itself
 
 // The sequence of rank `rank` (0: the longest; ties by index) among the first `batch`, and its length: a search for the
-// length by its bits, in which a wavefront holds all lengths in registers and counts with ballots: 31 x batch / 64
-// compares, where ranking every sequence against every other in LDS took batch^2 / 64 a workgroup, 5 us at 128 sequences
-// before its first load, and as long in the workgroups of empty sequences.  40 heads of 128, f16: 256 sequences, half of
-// them empty, 343 -> 322 us, 200 of 300 tokens 220 -> 212, 128 of 680 tokens 289 -> 285; fp8 cache 156 -> 153.
+// length by its bits, in which a wavefront holds all lengths in registers and counts with ballots, some 16 counts for
+// lengths of a few thousand, where ranking every sequence against every other in LDS took batch^2 / 64 compares a
+// workgroup, 5 us at 128 sequences before its first load, and as long in the workgroups of empty sequences.
 __device__ __forceinline__ int sequence_of_rank(const int32_t* seq_lens, int batch, int rank, int lane, int& seq_len) {
   constexpr int kSlots = kRankInKernelMax / 64;
   int len[kSlots];
@@ -387,14 +386,24 @@ __device__ __forceinline__ int sequence_of_rank(const int32_t* seq_lens, int bat
     len[i] = j < batch ? max(seq_lens[j], 0) : -1;
   }
   auto count = [&](auto pred) {
-    int c = 0;
-#pragma unroll
-    for (int i = 0; i < kSlots; ++i)
-      if (i * 64 < batch) c += __popcll(__builtin_amdgcn_ballot_w64(pred(len[i])));
+    auto ones = [&](int i) { return (int)__popcll(__builtin_amdgcn_ballot_w64(pred(len[i]))); };
+    int c = ones(0);
+    if (batch > 64) {
+      c += ones(1);
+      if (batch > 128) {
+        c += ones(2) + ones(3);
+        if (batch > 256) c += ones(4) + ones(5) + ones(6) + ones(7);
+      }
+    }
     return c;
   };
+  static_assert(kSlots == 8, "count() goes over the slots by hand");
+  int top = 0;   // the highest bit of any length
+#pragma unroll
+  for (int w = 16; w > 0; w >>= 1)
+    if (count([&](int x) { return (x >> (top + w)) > 0; }) != 0) top += w;
   int value = 0;   // the largest value that more than `rank` lengths reach
-  for (int bit = 30; bit >= 0; --bit) {
+  for (int bit = top; bit >= 0; --bit) {
     const int trial = value | (1 << bit);
     if (count([&](int x) { return x >= trial; }) > rank) value = trial;
   }
@@ -402,6 +411,7 @@ __device__ __forceinline__ int sequence_of_rank(const int32_t* seq_lens, int bat
   int seq = 0;
 #pragma unroll
   for (int i = 0; i < kSlots; ++i) {
+    if (i > 0 && i * 64 >= batch) break;
     const uint64_t same = __builtin_amdgcn_ballot_w64(len[i] == value);
     const int n = __popcll(same);
     if (skip >= 0 && skip < n) {
@@ -418,12 +428,12 @@ __device__ __forceinline__ int sequence_of_rank(const int32_t* seq_lens, int bat
 // wavefront that finishes last merges the partial results through LDS: no partials in HBM, no second launch.
 // Wavefronts whose partition is empty leave at once (their registers and wave slot are free from then on).
 // Workgroup rows are dealt out longest sequence first (list scheduling): the order comes from seq_order, or,
-// for batches up to kRankInKernelMax, from a search in every wavefront (sequence_of_rank).
+// for batches up to kRankInKernelMax, from a search in the first wavefront (sequence_of_rank).
 // (the body takes its place in the grid as arguments: head group bx, workgroup row by)
 template <int QT, int KV, int D, int HPW, int DEPTH, int WAVES>
 __device__ __forceinline__ void paged_decode_group_body(const AttnArgs& a, const int bx, const int by) {
   constexpr int EPL = Unpack<KV>::EPL, LPT = D / EPL, LPR = LPT * HPW;
-  __shared__ int s_arrived;
+  __shared__ int s_arrived, s_seq, s_len;
   __shared__ float s_part[WAVES][LPR][EPL + 2];
   const int tid = threadIdx.x;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -431,12 +441,22 @@ __device__ __forceinline__ void paged_decode_group_body(const AttnArgs& a, const
   if (tid == 0) s_arrived = 0;
   int seq, seq_len;
   if (a.rank_in_kernel) {
-    seq = sequence_of_rank(a.seq_lens, a.batch, by, lane, seq_len);
+    // One wavefront searches, the others wait: with a search in each, workgroups of short sequences were bound by its
+    // instructions (f16, ranked in LDS / a search in each / in one: 40 heads of 128, 32 sequences of 20 tokens
+    // 12.9 / 22.4 / 10.4 us, 256 of 20 115 / 44.5 / 34.7, 64 of 700 198 / 194 / 193; 12 heads of 64, 96 of 40
+    // 13.3 / 18.3 / 7.7).
+    if (wave == 0) {
+      seq = sequence_of_rank(a.seq_lens, a.batch, by, lane, seq_len);
+      if (lane == 0) { s_seq = seq; s_len = seq_len; }
+    }
+    __syncthreads();
+    seq = __builtin_amdgcn_readfirstlane(s_seq);
+    seq_len = __builtin_amdgcn_readfirstlane(s_len);
   } else {
     seq = a.seq_order ? a.seq_order[by] : by;
     seq_len = a.seq_lens[seq];
+    __syncthreads();
   }
-  __syncthreads();
   int np = (seq_len + a.partition_size - 1) / a.partition_size;
   np = np < 1 ? 1 : (np > WAVES ? WAVES : np);
   if (wave >= np) return;

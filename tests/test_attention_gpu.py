@@ -82,6 +82,16 @@ def test_sequences_taken_longest_first_each_exactly_once(dev, B):
     check(out, ref)
 
 
+@pytest.mark.parametrize("B", [127, 128, 129, 255, 256])    # the groups of 64 lengths counted together
+def test_sequences_of_few_and_of_many_bits(dev, B):
+    """One sequence whose length has more bits than the others', equal ones of 2^k and 2^k - 1 around it."""
+    lens = np.random.default_rng(B).choice([0, 1, 2, 3, 4, 7, 8, 127, 128], B).tolist()
+    lens[B // 3] = 4097
+    c = make_case(B, 16, 64, 16, lens, B)
+    out, ref = run_both(c, dev, 1024)     # 5 partitions of the longest
+    check(out, ref)
+
+
 @pytest.mark.parametrize("BS", [16, 32])
 def test_decode_attention_block_sizes_and_many_partitions(dev, BS):
     lens = [700, 1, 257, 512, 31]

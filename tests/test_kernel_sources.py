@@ -41,3 +41,11 @@ def test_prompt_attention_copies_a_tile_ahead():
     are waited for before the next LDS read of any stage, so every path issues them from assembly."""
     code = re.sub(r"//[^\n]*", "", (CSRC / "prefill_attention.hip").read_text())
     assert not re.search(r"__builtin_amdgcn_\w*load\w*_lds", code)
+
+
+def test_one_wavefront_of_a_workgroup_looks_the_sequence_up():
+    """The search by rank is some hundred instructions that do not depend on the wavefront: in every wavefront of
+    workgroups whose sequences are short it took longer than the attention."""
+    text = re.sub(r"//[^\n]*", "", (CSRC / "paged_decode_core.h").read_text())
+    calls = [m.start() for m in re.finditer(r"=\s*sequence_of_rank\(", text)]
+    assert len(calls) == 1 and re.search(r"if \(wave == 0\) \{\s*seq $", text[:calls[0]])
