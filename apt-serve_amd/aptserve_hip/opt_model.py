@@ -42,24 +42,41 @@ class OPTConfig:
         return OPTConfig(768, 12, 12, 3072, 50272, 2048)
 
 
-#: Bytes added to the row pitch of a matrix whose rows are a multiple of 2 KiB long.  At such a pitch the 128-byte
-#: pieces that a k-tile takes of many rows meet in few channels of the memory side: fc2 of 361 rows (rows of 40 KiB)
-#: takes 123 us, 106 with its weight at the longer pitch and 99 with the activations as well; fc1 86 and 80, qkv 82
-#: and 77 (rows of 10 KiB).  Products of at most 48 rows stream whole rows and do not care.
+#: Bytes added to the row pitch of a matrix whose rows are a multiple of 2 KiB long, but not a power of two.  At such a
+#: pitch the 128-byte pieces that a k-tile takes of many rows meet in few channels of the memory side: fc2 of 361 rows
+#: (rows of 40 KiB) takes 131 us, 107 with its weight at the longer pitch and 92 with the activations as well, fc1 86 and
+#: 82, qkv 83 and 78 (rows of 10 KiB), a whole prompt step of 361 tokens 14.15 ms and 12.62.  Rows of 4, 8 or 16 KiB are read
+#: no faster at a longer pitch.  Products of at most 48 rows stream whole rows and care little: fc2 of 5 rows 37.5 us and
+#: 38.2, a decode step of 5 sequences 7.28 ms and 7.29, of 16 (20 layers) 4.72 and 4.64.
 _PITCH_PAD = 128
+
+
+def _row_pitch(k: int, dtype) -> int:
+    row = k * dtype.itemsize
+    return k + (_PITCH_PAD // dtype.itemsize if row % 2048 == 0 and row & (row - 1) else 0)
 
 
 def row_pitched(n: int, k: int, dtype, device) -> torch.Tensor:
     """An uninitialised ``[n, k]`` matrix at the row pitch the products of this library read fastest (a view of a
     wider one where that is not ``k``); every operator takes it in place of a contiguous matrix."""
-    esz = torch.empty(0, dtype=dtype).element_size()
-    return torch.empty(n, k + (_PITCH_PAD // esz if k * esz % 2048 == 0 else 0), dtype=dtype, device=device)[:, :k]
+    return torch.empty(n, _row_pitch(k, dtype), dtype=dtype, device=device)[:, :k]
+
+
+def lay_out_weights(weights: Dict[str, torch.Tensor]) -> Dict[str, torch.Tensor]:
+    """Puts the layers' matrices at the pitch of :func:`row_pitched`: to be called once, on loaded (contiguous) weights
+    and before a model is built from them.  Works in the given dict, one matrix at a time, and returns it; what holds on
+    to a replaced tensor keeps the old memory.  A loader that fills :func:`row_pitched` matrices has no need of it."""
+    for name, w in weights.items():
+        if name.startswith("layers.") and w.dim() == 2 and w.stride() == (w.size(1), 1) and w.size(1) != _row_pitch(
+                w.size(1), w.dtype):
+            weights[name] = row_pitched(*w.shape, w.dtype, w.device).copy_(w.detach())
+    return weights
 
 
 def random_weights(cfg: OPTConfig, seed: int, device, dtype=torch.float16, layers: Optional[int] = None
                    ) -> Dict[str, torch.Tensor]:
     """N(0, 0.02) matrices, N(0, 0.02) biases, LayerNorm gains near 1 — generated on ``device``; the layers'
-    matrices lie at the pitch of :func:`row_pitched`."""
+    matrices lie at the pitch of :func:`row_pitched`, as a loader would put them (or :func:`lay_out_weights`)."""
     g = torch.Generator(device=device).manual_seed(seed)
     Hd, F_, L = cfg.hidden_size, cfg.ffn_dim, cfg.num_hidden_layers if layers is None else layers
 
@@ -122,6 +139,8 @@ class HybridOPTDecoderLayer:
 
 
 class HybridOPTModel:
+    """``weights`` are used as they lie: matrices at the pitch of :func:`row_pitched` make prompt steps faster."""
+
     def __init__(self, cfg: OPTConfig, weights: Dict[str, torch.Tensor], num_layers: Optional[int] = None,
                  fused_norm: bool = True, **attn_kw) -> None:
         self.cfg, self.w, self.fused_norm = cfg, weights, fused_norm
