@@ -57,9 +57,10 @@ def _row_pitch(k: int, dtype) -> int:
 
 
 def row_pitched(n: int, k: int, dtype, device) -> torch.Tensor:
-    """An uninitialised ``[n, k]`` matrix at the row pitch the products of this library read fastest (a view of a
-    wider one where that is not ``k``); every operator takes it in place of a contiguous matrix."""
-    return torch.empty(n, _row_pitch(k, dtype), dtype=dtype, device=device)[:, :k]
+    """An uninitialised ``[n, k]`` matrix at the row pitch the products of this library read fastest; every operator
+    takes it in place of a contiguous matrix.  (One call, as ``torch.empty`` is: prompt steps of small models are bound by
+    the host.)"""
+    return torch.empty_strided((n, k), (_row_pitch(k, dtype), 1), dtype=dtype, device=device)
 
 
 def lay_out_weights(weights: Dict[str, torch.Tensor]) -> Dict[str, torch.Tensor]:
