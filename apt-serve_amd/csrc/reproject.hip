@@ -1101,9 +1101,9 @@ extern "C" {
 // Tile rows / 64 and K split of a product beyond the row-streaming kernels' range: the pair with the least time by
 // this account (us).  Its numbers are fitted, as a whole, to every tile size and K split timed on 23 weight shapes (256 to
 // 20480 rows of 768 to 65536, close and padded) at 36 row counts from 49 to 8192; the pair it picks takes 1.2 % longer than
-// the fastest one measured on average, more than 10 % longer at 31 of 1188 products:
+// the fastest one measured on average, more than 10 % longer at 33 of 1188 products:
 //   rounds of workgroups x (k-tiles of a workgroup x time of a k-tile + 3),
-//   for a split 4 + 0.65 per part (the second launch reads them one after the other) + the fp32 parts written and read
+//   for a split 4.2 + 0.65 per part (the second launch reads them one after the other) + the fp32 parts written and read
 //   once at 3.8 TB/s, for a cut last round its short k-range, 2, and its parts at the same rate.
 // The parts of a tile run on one XCD, so a round takes ceil(tiles / 8) x parts <= 32: 20 tiles x 12 parts are two rounds
 // though 240 are fewer than the CUs (5120 x 20480, 64 rows: 66 us; with 10 parts 48).  Few tiles of a long K take many
@@ -1140,7 +1140,7 @@ static TilePlan tile_plan(int64_t m, int64_t n, int64_t k, bool may_split, RowPi
     if (us < least) { least = us; best = {mi, 1}; }
     const int most = may_split ? (int)std::min<int64_t>(kXcdCus / per_xcd, nk / 4) : 1;   // one round, 4 k-tiles a part
     for (int s = 2; s <= most; ++s) {
-      const double split_us = ((nk + s - 1) / s) * kt_us + 7.0 + s * (0.65 + part_us);
+      const double split_us = ((nk + s - 1) / s) * kt_us + 7.2 + s * (0.65 + part_us);
       if (split_us < least) { least = split_us; best = {mi, s}; }
     }
   }
