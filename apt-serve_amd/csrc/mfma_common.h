@@ -62,7 +62,7 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
 // The compiler puts no wait states into a statement: the copy needs one after the write of m0, and five after a vector
 // instruction (v_readfirstlane) that wrote a register of the descriptor, so s_mov + s_nop 3 stand before it.  m0 is in the
 // clobber list so that the compiler does not keep a value of its own in it (it warns that it does not save m0, either).
-// The longer wait costs prompts on a cached prefix 1 to 2 % (200 x 4 tokens on 4000 of 40 x 128 heads: 52.0 -> 52.9 us).
+// The longer wait costs prompts on a cached prefix 1 to 2 % (4 sequences, 200 tokens in all on 4000 cached, 40 x 128 heads: 52.0 -> 52.9 us).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
 __device__ __forceinline__ void copy_to_lds(uint32_t lds, const u32x4& rsrc, uint32_t voff, uint32_t soff) {

@@ -58,7 +58,8 @@ enum KeySource { kPacked, kPaged16, kPackedAny, kPagedAny };
 
 template <bool BF16, int D, int SRC, int QT>
 // Two workgroups per CU (64 KiB of LDS each at head size 128) are two wavefronts per SIMD: the compiler may use the
-// registers that leaves (202 at 128 queries a workgroup).
+// registers that leaves (202 at 128 queries a workgroup).  Head size 64 has the same bound, though its 32 KiB would leave room
+// for more.
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void prefill_attention_kernel(
     const PrefillArgs a) {
   constexpr int BQ = 64 * QT;         // queries per workgroup
@@ -118,8 +119,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   // Copies.  A wave-wide copy moves RPC = 64 / KCH key rows; wavefront w makes copies w, w + 4, ... of K's and of V's, so
   // that a lane always moves the same row of a group of 16 keys (and has one swizzle), and the group is wave-uniform.
   // A lane keeps its offset inside a tile; the tile's (kPacked) or the group's (kPaged16) start is scalar work.  (Key by key,
-  // every lane makes its addresses; the block numbers are loaded a tile ahead too.  Blocks of 48: 4 x 200 tokens on 4000
-  // cached of 40 x 128 heads 57.6 -> 48.5 us against copies through the builtin, 8 x 1000 on 1000 564 -> 533.)  (Every
+  // every lane makes its addresses; the block numbers are loaded a tile ahead too.  Blocks of 48: 4 sequences, 200 tokens on 4000
+  // cached, of 40 x 128 heads 57.6 -> 48.5 us against copies through the builtin, 8 sequences, 8000 on 8000 564 -> 533.)  (Every
   // lane multiplying out 64-bit offsets of twelve rows a tile, 130 quarter-rate multiplications with the divisions of a
   // block table, cost as much as the softmax: 274 against 251 us for 4 x 2048 tokens.)
   constexpr int RPC = 64 / KCH, PER = BKV / RPC / 4;   // key rows of a copy; copies per wavefront and operand
@@ -350,7 +351,8 @@ int launch_prefill(PrefillArgs& a, bool paged, int64_t num_seqs, int64_t max_seq
   // Few workgroups: 64 queries each instead of 128.  A workgroup's time is its key tiles one after the other, 2.0 us each
   // with 32 queries a wavefront and 1.5 with 16, so as long as the CUs are not full the shorter ones finish first (12
   // heads, 2048 tokens: 34 -> 26 us; 40 heads, 361 tokens 11.1 -> 9.9, 4 x 50 on a prefix of 4000 61 -> 49); full CUs
-  // lose by reading every fragment for half the queries (40 heads, 1400 tokens 26 -> 28, 4 x 2048 221 -> 304).
+  // lose by reading every fragment for half the queries (40 heads, 1400 tokens 26 -> 28, 4 x 2048 243 -> 312).  The count
+  // looks at queries alone (16 chunks, 1000 new on 8000 cached tokens, 40 heads: 91 us, 89 with 64).
   // (A longest sequence stated far beyond the tokens, within the grid's limit at 128 queries only, is taken at 128.)
   const int qt = num_heads * (a.num_tokens / 128 + num_seqs) <= 384 && max_seqlen_q <= 65535 * 64 ? 1 : 2;
   const int64_t q_tiles = (max_seqlen_q + 64 * qt - 1) / (64 * qt);
