@@ -16,7 +16,7 @@
 // needs less energy per flop than 32x32x16 (16): alone, with operands in
 // registers, they sustain 1.8 against 1.4-1.6 PFLOP/s (aps_mfma_probe).
 // The K loop moves BK = 64 at a time through an LDS ring of two stages (2 x (32 + 32)
-// KiB of the 160 KiB per CU; three and four stages for the smaller tiles of 128 and
+// KiB of the 160 KiB per CU; three stages for the smaller tiles of 128 and
 // 64 rows; 144 KiB with the epilogue images): tile t+1 is
 // copied global -> LDS by buffer_load ... lds (no VGPR round trip) while the
 // matrix cores consume tile t.
@@ -63,10 +63,11 @@ struct TileShape {
   static constexpr int kWm = 32 * MI, kBm = 2 * kWm;
   static constexpr int kATileBytes = kBm * BK * 2;
   static constexpr int kStageBytes = kATileBytes + kWTileBytes;
-  // As many stages as the LDS of a CU holds: with two, a tile's loads have one k-tile's time to arrive, and the 64-
+  // Three stages where the LDS of a CU holds them: with two, a tile's loads have one k-tile's time to arrive, and the 64-
   // and 128-row tiles, whose k-tiles are short, waited for them (512 x 5120 on 15360 weight rows: 84 us with three
-  // stages of the 128-row tile, 111 with two of the 192-row one).
-  static constexpr int kStages = MI <= 2 ? 5 - MI : 2;
+  // stages of the 128-row tile, 111 with two of the 192-row one).  The 64-row tile has room for four, which take longer to
+  // fill and bring nothing (49 x 768 rows on 1536 8.8 us, with three 8.6; 49 x 5120 on 5120 20.05 with either, 22.7 with two).
+  static constexpr int kStages = MI <= 2 ? 3 : 2;
   static constexpr int kEpiWaveBytes = kWm * kEpiPitch;
   static constexpr int kLdsBytes =
       kWaves * kEpiWaveBytes > kStages * kStageBytes ? kWaves * kEpiWaveBytes : kStages * kStageBytes;
@@ -306,10 +307,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   issue_loads(0, 0);
   if (ahead > 0) issue_loads(1, 1);
   if (S > 2 && ahead > 1) issue_loads(2, 2);
-  if (S > 3 && ahead > 2) issue_loads(3, 3);
   auto wait_tiles = [&](int tiles) {   // until at most `tiles` tiles are in flight
-    if (S > 3 && tiles >= 3) wait_vm<3 * kLoads>();
-    else if (S > 2 && tiles == 2) wait_vm<2 * kLoads>();
+    if (S > 2 && tiles >= 2) wait_vm<2 * kLoads>();
     else if (tiles == 1) wait_vm<kLoads>();
     else wait_vm<0>();
   };

@@ -47,7 +47,7 @@ def test_linear_nt_small(dev, M, N, K, dtype):
 @pytest.mark.parametrize("M", [64, 200, 380, 500])       # 64-, 128-, 192- and 256-row tiles at this N
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_linear_nt_ring_of_k_tiles(dev, M, nk, dtype):
-    """The LDS ring of every tile size (four, three, two stages) around its fill and drain: fewer k-tiles than
+    """The LDS ring of every tile size (three and two stages) around its fill and drain: fewer k-tiles than
     stages, as many, one more, and several rounds, on enough tiles that the plan neither splits K nor changes size."""
     N, K = 25600, 64 * nk
     assert ops._lib.load().aps_linear_nt_splits(M, N, K) == 1
