@@ -57,39 +57,37 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
   else return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, half2p));
 }
 
+// A buffer descriptor that scalar instructions wrote: base + off, last_row + row_bytes bytes long (all wave-uniform).  A copy
+// from assembly may follow at once; after a vector instruction (v_readfirstlane) wrote a register of its descriptor it would
+// need five wait states, which the compiler does not put into or before an assembly statement.  (The kernels that use it
+// spill no scalar registers; a reload would be such an instruction.)  40 x 128 heads, 4 sequences, 200 tokens on 4000 cached:
+// 48.1 us, with five wait states before every copy 52.9, with neither 51.7; 4 prompts, 8192 tokens 240, 243 and 248.
+struct ScalarRsrc { u32x4 words; };
+__device__ __forceinline__ ScalarRsrc scalar_rsrc(const char* base, int64_t off, uint32_t last_row, uint32_t row_bytes) {
+  uint32_t lo, hi, n;
+  asm("s_add_u32 %0, %3, %4\n\ts_addc_u32 %1, %5, %6\n\ts_add_u32 %2, %7, %8"
+      : "=&s"(lo), "=&s"(hi), "=&s"(n)
+      : "s"((uint32_t)(uint64_t)base), "s"((uint32_t)(uint64_t)off), "s"((uint32_t)((uint64_t)base >> 32)),
+        "s"((uint32_t)((uint64_t)off >> 32)), "s"(last_row), "s"(row_bytes)
+      : "scc");
+  return ScalarRsrc{u32x4{lo, hi, n, 0x00020000u}};
+}
 // One 1 KiB copy global -> LDS: lane l's 16 bytes at offset voff + soff of the buffer land at lds + 16 l.  From assembly:
-// the compiler, seeing a copy into LDS, waits for every load in flight before the next LDS read of any stage.
-// The compiler puts no wait states into a statement: the copy needs one after the write of m0, and five after a vector
-// instruction (v_readfirstlane) that wrote a register of the descriptor, so s_mov + s_nop 3 stand before it.  m0 is in the
-// clobber list so that the compiler does not keep a value of its own in it (it warns that it does not save m0, either).
-// The longer wait costs prompts on a cached prefix 1 to 2 % (4 sequences, 200 tokens in all on 4000 cached, 40 x 128 heads: 52.0 -> 52.9 us).
+// the compiler, seeing a copy into LDS, waits for every load in flight before the next LDS read of any stage.  The s_nop is
+// the wait state between a write of m0 and the copy; m0 is in the clobber list so that the compiler does not keep a value of
+// its own in it (it warns that it does not save m0, either).
 #pragma clang diagnostic push
 #pragma clang diagnostic ignored "-Winline-asm"
-__device__ __forceinline__ void copy_to_lds(uint32_t lds, const u32x4& rsrc, uint32_t voff, uint32_t soff) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc), "s"(soff)
+__device__ __forceinline__ void copy_to_lds(uint32_t lds, const ScalarRsrc& rsrc, uint32_t voff, uint32_t soff) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(voff), "s"(rsrc.words),
+               "s"(soff)
                : "memory", "m0");
 }
 // The same with an address per lane.
 __device__ __forceinline__ void copy_lanes_to_lds(uint32_t lds, const char* p) {
-  asm volatile("s_mov_b32 m0, %0\n\ts_nop 3\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory", "m0");
-}
-// Two of copy_to_lds under one wait: the packed prompt attention runs as long as without it (4 x 2048 tokens 240 us).
-__device__ __forceinline__ void copy2_to_lds(uint32_t lds0, const u32x4& rsrc0, uint32_t voff0, uint32_t lds1, const u32x4& rsrc1,
-                                             uint32_t voff1, uint32_t soff0, uint32_t soff1) {
-  asm volatile(
-      "s_mov_b32 m0, %0\n\ts_nop 3\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\t"
-      "s_mov_b32 m0, %4\n\ts_nop 0\n\tbuffer_load_dwordx4 %5, %6, %7 offen lds" ::"s"(lds0),
-      "v"(voff0), "s"(rsrc0), "s"(soff0), "s"(lds1), "v"(voff1), "s"(rsrc1), "s"(soff1)
-      : "memory", "m0");
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, off" ::"s"(lds), "v"(p) : "memory", "m0");
 }
 #pragma clang diagnostic pop
-__device__ __forceinline__ u32x4 raw_rsrc(const char* p, int64_t bytes) {   // make_rsrc for the assembly
-  const uint64_t a = (uint64_t)p;
-  const uint32_t n = bytes <= 0 ? 0u : (bytes > 0xffffffffll ? 0xffffffffu : (uint32_t)bytes);
-  return u32x4{(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a),
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32)),
-               (uint32_t)__builtin_amdgcn_readfirstlane((int)n), 0x00020000u};
-}
 
 // Hand-placed wait points: a __syncthreads() would add fences that wait for every outstanding DMA load.
 #define APS_WAIT_VM(n) asm volatile("s_waitcnt vmcnt(" #n ")" ::: "memory")

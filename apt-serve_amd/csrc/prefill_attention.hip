@@ -160,13 +160,13 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   auto copy_tile = [&](int kv0, int stage) {
     const uint32_t dst = lds_base + stage * kStage + wave_u * 1024;   // copy i of an operand: bytes [1024 i, 1024 i + 1024)
     if constexpr (SRC == kPacked) {   // rows past the sequence read as zeros; the mask removes their scores
-      const int64_t left = len - kv0 - 1;
-      const u32x4 rk = raw_rsrc(k_base + kv0 * a.k_stride_b, left * a.k_stride_b + D * 2);
-      const u32x4 rv = raw_rsrc(v_base + kv0 * a.v_stride_b, left * a.v_stride_b + D * 2);
+      const uint32_t last = (uint32_t)min(BKV - 1, len - kv0 - 1);
+      const ScalarRsrc rk = scalar_rsrc(k_base, kv0 * a.k_stride_b, last * (uint32_t)a.k_stride_b, D * 2);
+      const ScalarRsrc rv = scalar_rsrc(v_base, kv0 * a.v_stride_b, last * (uint32_t)a.v_stride_b, D * 2);
 #pragma unroll
       for (int j = 0; j < PER; ++j) {
-        copy2_to_lds(dst + j * 4096, rk, k_lane, dst + kTile + j * 4096, rv, v_lane, j * 4 * RPC * (uint32_t)a.k_stride_b,
-                     j * 4 * RPC * (uint32_t)a.v_stride_b);
+        copy_to_lds(dst + j * 4096, rk, k_lane, j * 4 * RPC * (uint32_t)a.k_stride_b);
+        copy_to_lds(dst + kTile + j * 4096, rv, v_lane, j * 4 * RPC * (uint32_t)a.v_stride_b);
       }
     } else if constexpr (SRC == kPaged16) {
 #pragma unroll
@@ -176,10 +176,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
             block_start(blocks[j]) + (int64_t)((g & ((1 << a.groups_shift) - 1)) * 16) * a.k_stride_b;
         // what a block holds past its sequence may be anything, and a zero probability does not cancel a NaN: the buffer
         // ends with the sequence's last row and the others read as zeros
-        const int64_t bytes = min(15, len - 1 - 16 * g) * a.k_stride_b + D * 2;
-        // (one copy at a time: both descriptors before the first copy cost 2 to 3 % more)
-        copy_to_lds(dst + j * 4096, raw_rsrc(k_base + start, bytes), k_lane, 0);
-        copy_to_lds(dst + kTile + j * 4096, raw_rsrc(v_base + start, bytes), v_lane, 0);
+        const uint32_t last = (uint32_t)min(15, len - 1 - 16 * g) * (uint32_t)a.k_stride_b;
+        copy_to_lds(dst + j * 4096, scalar_rsrc(k_base, start, last, D * 2), k_lane, 0);
+        copy_to_lds(dst + kTile + j * 4096, scalar_rsrc(v_base, start, last, D * 2), v_lane, 0);
       }
       load_blocks(kv0 + BKV);
     } else {

@@ -889,7 +889,7 @@ __global__ __launch_bounds__(kScThreads) void weight_ksplit_kernel(const GemmArg
   // (The copies are issued from assembly: the compiler, seeing a copy into LDS and a later LDS read, waits for
   // every load in flight before the first read, weight rows included; it cannot know which bytes the copy wrote.)
   const int64_t head_off = g.head_rows ? (n0 / g.head_rows) * g.x_head_stride_b : 0;
-  const u32x4 rsrc = raw_rsrc(g.a + head_off, (m - 1) * g.lda_b + g.k * 2);   // the m rows of x
+  const ScalarRsrc rsrc = scalar_rsrc(g.a, head_off, (uint32_t)((m - 1) * g.lda_b), (uint32_t)(g.k * 2));   // the m rows of x
   const uint32_t lds_base = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) char*)lds;
 #pragma unroll
   for (int j = 0; j < P; ++j) {   // (8 rows x P copies / 8 wavefronts = P copies per wavefront at most)

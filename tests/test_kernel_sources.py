@@ -16,24 +16,41 @@ def asm_statements(text):
             yield "".join(re.findall(r'"((?:\\.|[^"\\])*)"', code.group(1))), body[code.end():]
 
 
+def instructions(code):
+    return [i.strip() for i in re.split(r"\\n|;", code.replace("\\t", " ")) if i.strip()]
+
+
 def test_assembly_that_writes_m0_says_so_and_waits():
-    """A copy global -> LDS takes its LDS address from m0 and its descriptor from scalar registers.  The compiler keeps
-    m0 for its own use unless the statement names it, and it cannot put wait states inside a statement: one is needed
-    between a write of m0 and the copy, five between a scalar register written by a vector instruction and the copy."""
+    """A copy global -> LDS takes its LDS address from m0.  The compiler keeps m0 for its own use unless the statement
+    names it, and it cannot put the wait state between a write of m0 and the copy into a statement."""
     found = 0
     for p in SOURCES:
         for code, rest in asm_statements(p.read_text()):
-            ins = [i.strip() for i in re.split(r"\\n|;", code) if i.replace("\\t", "").strip()]
-            ins = [i.replace("\\t", " ").strip() for i in ins]
-            writes = [i for i, x in enumerate(ins) if re.match(r"s_mov_b32 m0\b", x)]
-            if not writes:
-                continue
-            found += 1
-            assert '"m0"' in rest.rsplit(":", 1)[-1], f"{p.name}: m0 is not in the clobber list of {code!r}"
-            load = next(i for i, x in enumerate(ins) if x.startswith("buffer_load") or x.startswith("global_load"))
-            states = sum(int(x.split()[1]) + 1 if x.startswith("s_nop") else 1 for x in ins[:load])
-            assert states >= 5, f"{p.name}: {states} wait states before the copy in {code!r}"
+            ins = instructions(code)
+            for i, x in enumerate(ins):
+                if re.match(r"s_mov_b32 m0\b", x):
+                    found += 1
+                    assert '"m0"' in rest.rsplit(":", 1)[-1], f"{p.name}: m0 is not in the clobber list of {code!r}"
+                    load = next(j for j, y in enumerate(ins) if j > i and re.match(r"(buffer|global)_load", y))
+                    assert load > i + 1, f"{p.name}: no wait state after the write of m0 in {code!r}"
     assert found >= 1
+
+
+def test_copies_from_assembly_take_descriptors_that_scalar_instructions_wrote():
+    """Five wait states lie between a vector instruction that writes a scalar register and a memory instruction that reads
+    it; the compiler puts none in front of a statement.  Descriptors of copies come from scalar_rsrc alone, which ends
+    in scalar instructions."""
+    text = {p.name: re.sub(r"//[^\n]*", "", p.read_text()) for p in SOURCES}
+    for name, t in text.items():
+        for code, rest in asm_statements(t):
+            if any(x.startswith("buffer_") for x in instructions(code)):
+                assert '"s"(rsrc.words)' in rest, f"{name}: {code!r}"
+    made = [(name, m.start()) for name, t in text.items() for m in re.finditer(r"\bScalarRsrc\s*\{\s*u32x4\s*\{", t)]
+    assert [name for name, _ in made] == ["mfma_common.h"]
+    body = text["mfma_common.h"]
+    body = body[body.index("ScalarRsrc scalar_rsrc("):made[0][1]]
+    code = "".join(re.findall(r'asm\("((?:\\.|[^"\\])*)"', body))
+    assert code and all(x.startswith("s_") for x in instructions(code))
 
 
 def test_prompt_attention_copies_a_tile_ahead():
