@@ -81,11 +81,14 @@ def random_weights(cfg: OPTConfig, seed: int, device, dtype=torch.float16, layer
     g = torch.Generator(device=device).manual_seed(seed)
     Hd, F_, L = cfg.hidden_size, cfg.ffn_dim, cfg.num_hidden_layers if layers is None else layers
 
-    def n(*shape, std=0.02, mean=0.0):
-        return (torch.randn(*shape, generator=g, device=device, dtype=torch.float32) * std + mean).to(dtype)
+    def values(*shape, std=0.02, mean=0.0):
+        return torch.randn(*shape, generator=g, device=device, dtype=torch.float32) * std + mean
+
+    def n(*shape, **kw):
+        return values(*shape, **kw).to(dtype)
 
     def m(*shape):
-        return row_pitched(*shape, dtype, device).copy_(n(*shape))
+        return row_pitched(*shape, dtype, device).copy_(values(*shape))
     w = {"embed_tokens": n(cfg.vocab_size, Hd), "embed_positions": n(cfg.max_position_embeddings + 2, Hd),
          "final_ln_w": n(Hd, std=0.02, mean=1.0), "final_ln_b": n(Hd)}
     for i in range(L):
