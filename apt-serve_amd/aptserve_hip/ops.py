@@ -846,12 +846,18 @@ def flash_attn_varlen_func(q, k, v, cu_seqlens_q=None, cu_seqlens_k=None, max_se
         _need(block_table.dtype == torch.int32 and block_table.dim() == 2 and block_table.size(0) == n_seq and
               block_table.device == dev and (block_table.size(1) <= 1 or block_table.stride(1) == 1),
               "block_table must be int32 [seqs, width] with contiguous rows on the same GPU")
+        lib = _lib.load()
+        max_k = block_table.size(1) * k.size(1)
+        if max_seqlen_k is not None:
+            max_k = min(max_k, int(max_seqlen_k))
+        need = lib.aps_paged_prefill_attention_workspace_bytes(n_seq, T, max_len, max_k, H, D)
+        ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None     # (few tokens on long prefixes)
         with _on(dev):
-            st = _lib.load().aps_paged_prefill_attention(
+            st = lib.aps_paged_prefill_attention_split(
                 out.data_ptr() if T else None, q.data_ptr() if T else None, k.data_ptr(), v.data_ptr(),
                 _ptr(block_table), _ptr(cu_seqlens_q), _ptr(cu_seqlens_k), n_seq if T else 0, T, max_len, H, D,
                 k.size(1), block_table.stride(0), block_table.size(1), q.stride(0), out.stride(0), k.stride(0),
-                k.size(0), float(softmax_scale), _DTYPE_CODE[q.dtype], _stream(q))
+                k.size(0), float(softmax_scale), _DTYPE_CODE[q.dtype], max_k, _ptr(ws), need, _stream(q))
         _lib.check(st, "flash_attn_varlen_func (prefix branch)")
         return out
     _need(cu_seqlens_k is None or cu_seqlens_k is cu_seqlens_q or torch.equal(cu_seqlens_k, cu_seqlens_q),

@@ -46,7 +46,24 @@ struct PrefillArgs {
   int64_t table_stride, table_width, block_stride_b, num_blocks;
   int block_size;
   int groups_shift;   // kPaged16: block_size = 16 << groups_shift
+  // PAGED, key parts: a workgroup multiplies one of at most `parts` runs of key tiles of its queries, as many as runs of `part_tiles`
+  // tiles take; with more than one of them fp32 sums, maxima and weights go to `partial` (one unit per workgroup: the O^T
+  // registers as they lie, then max and sum per query) and prefill_combine_kernel adds them.
+  int parts, part_tiles;
+  float* partial;
 };
+
+// Key tiles of each part of a query tile that meets n key tiles (the last part may have fewer)
+__device__ __forceinline__ int tiles_per_part(int n, int parts, int part_tiles) {
+  const int p = min(parts, (n + part_tiles - 1) / part_tiles);
+  return (n + p - 1) / p;
+}
+template <int D>
+__host__ __device__ constexpr int64_t unit_floats(int qt) { return 64 * qt * (D + 2); }
+// Units of a query tile: tiles before it are counted as if each sequence began a new one behind the tokens in front of it
+__device__ __forceinline__ int64_t first_unit(int s0, int seq, int q_tile, int bq, int heads, int head, int parts) {
+  return ((int64_t)(s0 / bq + seq + q_tile) * heads + head) * parts;
+}
 
 // Two stages of a K and a V tile
 template <int D>
@@ -90,8 +107,15 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     if (len < qlen || (int64_t)(len + a.block_size - 1) / a.block_size > a.table_width) return;
   }
   const int off = len - qlen;        // query i sees keys 0 .. i + off
-  const int q0 = (int)(gridDim.z - 1 - blockIdx.z) * BQ;
+  // (a packed prompt has one part: every tile of it is there, and its many query tiles fill the CUs)
+  const unsigned parts = PAGED ? (unsigned)a.parts : 1;
+  const int part = PAGED ? (int)(blockIdx.z % parts) : 0;
+  const int q_tile = (int)((gridDim.z - 1 - blockIdx.z) / parts), q0 = q_tile * BQ;
   if (q0 >= qlen) return;
+  const int kv_all = min(len, q0 + BQ + off);  // causal: keys beyond the tile's last query are never needed
+  const int n_tiles = (kv_all + BKV - 1) / BKV, per_part = PAGED ? tiles_per_part(n_tiles, a.parts, a.part_tiles) : n_tiles;
+  if (part >= (n_tiles + per_part - 1) / per_part) return;
+  const int kv_begin = part * per_part * BKV, kv_end = min(kv_all, kv_begin + per_part * BKV);
   const int tid = threadIdx.x & (kThreads - 1), wave = tid >> 6, lane = tid & 63;
   const int qcol = lane & 15, quad = lane >> 4;
   int my_q[QT];                                 // query index inside the sequence's new tokens (may be >= qlen)
@@ -214,15 +238,14 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
                                          (__attribute__((address_space(3))) short4v*)(lds + at)));
   };
 
-  const int kv_end = min(len, q0 + BQ + off);  // causal: keys beyond the tile's last query are never needed
   const int wave_q0 = q0 + wave * (16 * QT) + off;    // last key the first query of this wavefront sees
-  load_blocks(0);
+  load_blocks(kv_begin);
 #pragma unroll
   for (int u = 0; u < QT; ++u)   // the queries have arrived before the first copy is counted
 #pragma unroll
     for (int s = 0; s < KS; ++s) asm volatile("" : "+v"(qf[u][s]));
-  copy_tile(0, 0);
-  for (int kv0 = 0, stage = 0; kv0 < kv_end; kv0 += BKV, stage ^= 1) {
+  copy_tile(kv_begin, 0);
+  for (int kv0 = kv_begin, stage = 0; kv0 < kv_end; kv0 += BKV, stage ^= 1) {
     APS_WAIT_LGKM0();  // no fragment read of the previous tile is under way,
     APS_WAIT_VM(0);    // and this wavefront's copies of this tile have landed: past the barrier everyone's
     APS_BARRIER();
@@ -320,6 +343,21 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
     }
   }
 
+  // ---- one of several key parts: sums as they are
+  if (PAGED && per_part < n_tiles) {
+    float* const unit = a.partial + (first_unit(s0, seq, q_tile, BQ, a.num_heads, head, a.parts) + part) * unit_floats<D>(QT);
+    float* const ml = unit + BQ * D + wave * (16 * QT) + qcol;
+#pragma unroll
+    for (int u = 0; u < QT; ++u) {
+#pragma unroll
+      for (int t = 0; t < DT; ++t) ((float4v*)unit)[(u * DT + t) * kThreads + tid] = o[u][t];
+      float l = l_run[u];
+      l += __shfl_xor(l, 16);
+      l += __shfl_xor(l, 32);
+      if (quad == 0) { ml[16 * u] = m_run[u]; ml[BQ + 16 * u] = l; }
+    }
+    return;
+  }
   // ---- normalise and store: lane owns queries my_q, rows d = 16 t + 4 quad + e
 #pragma unroll
   for (int u = 0; u < QT; ++u) {
@@ -339,24 +377,106 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
   }
 }
 
+// out = sum of the key parts of a query tile, each weighted with exp2 of its maximum against the largest, over the sum of
+// their weights: the same sums in fp32, rounded once.  Same grid (without the parts) and same lanes as the kernel above, so
+// that units are written and read 1 KiB a wavefront.
+template <bool BF16, int D, int QT>
+__global__ __launch_bounds__(kThreads) void prefill_combine_kernel(const PrefillArgs a) {
+  constexpr int BQ = 64 * QT, DT = D / 16;
+  const int seq = blockIdx.y, head = blockIdx.x, q_tile = blockIdx.z, q0 = q_tile * BQ;
+  const int s0 = a.cu_seqlens[seq], s1 = a.cu_seqlens[seq + 1];
+  if (s0 < 0 || s1 < s0 || s1 > a.num_tokens) return;
+  const int qlen = s1 - s0;
+  const int len = a.cu_seqlens_k[seq + 1] - a.cu_seqlens_k[seq];
+  if (len < qlen || (int64_t)(len + a.block_size - 1) / a.block_size > a.table_width || q0 >= qlen) return;
+  const int n_tiles = (min(len, q0 + BQ + len - qlen) + BKV - 1) / BKV;
+  const int per_part = tiles_per_part(n_tiles, a.parts, a.part_tiles), parts = (n_tiles + per_part - 1) / per_part;
+  if (parts == 1) return;   // stored by its workgroup
+  const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, qcol = lane & 15, quad = lane >> 4;
+  const float* const units = a.partial + first_unit(s0, seq, q_tile, BQ, a.num_heads, head, a.parts) * unit_floats<D>(QT);
+#pragma unroll
+  for (int u = 0; u < QT; ++u) {
+    const int row = wave * (16 * QT) + 16 * u + qcol;
+    float m = -INFINITY;
+    for (int p = 0; p < parts; ++p) m = fmaxf(m, units[p * unit_floats<D>(QT) + BQ * D + row]);
+    const float m_use = m == -INFINITY ? 0.f : m;
+    float4v o[DT];
+#pragma unroll
+    for (int t = 0; t < DT; ++t) o[t] = float4v{0.f, 0.f, 0.f, 0.f};
+    float l = 0.f;
+    for (int p = 0; p < parts; ++p) {
+      const float* const unit = units + p * unit_floats<D>(QT);
+      const float w = __builtin_amdgcn_exp2f((unit[BQ * D + row] - m_use) * a.scale_log2);
+      l += w * unit[BQ * D + BQ + row];
+#pragma unroll
+      for (int t = 0; t < DT; ++t) {
+        const float4v v = ((const float4v*)unit)[(u * DT + t) * kThreads + tid];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[t][e] = fmaf(w, v[e], o[t][e]);
+      }
+    }
+    if (q0 + row >= qlen) continue;
+    const float inv = l > 0.f ? 1.f / l : 0.f;
+    char* op = a.out + (int64_t)(s0 + q0 + row) * a.out_stride_b + (int64_t)head * D * 2 + quad * 8;
+#pragma unroll
+    for (int t = 0; t < DT; ++t) {
+      uint2 w;
+      w.x = pack2<BF16>(o[t][0] * inv, o[t][1] * inv);
+      w.y = pack2<BF16>(o[t][2] * inv, o[t][3] * inv);
+      *(uint2*)(op + t * 32) = w;
+    }
+  }
+}
+
 }  // namespace
 }  // namespace aps
 
 using namespace aps;
 
 namespace {
-int launch_prefill(PrefillArgs& a, bool paged, int64_t num_seqs, int64_t max_seqlen_q, int num_heads, int head_size,
-                   int dtype, aps_stream_t stream) {
-  // Few workgroups: 64 queries each instead of 128.  A workgroup's time is its key tiles one after the other, 2.0 us each
-  // with 32 queries a wavefront and 1.5 with 16, so as long as the CUs are not full the shorter ones finish first (12
-  // heads, 2048 tokens: 34 -> 26 us; 40 heads, 361 tokens 11.1 -> 9.9, 4 x 50 on a prefix of 4000 61 -> 49); full CUs
-  // lose by reading every fragment for half the queries (40 heads, 1400 tokens 26 -> 28, 4 x 2048 243 -> 312).  The count
-  // looks at queries alone (16 chunks, 1000 new on 8000 cached tokens, 40 heads: 91 us, 89 with 64).
-  // (A longest sequence stated far beyond the tokens, within the grid's limit at 128 queries only, is taken at 128.)
-  const int qt = num_heads * (a.num_tokens / 128 + num_seqs) <= 384 && max_seqlen_q <= 65535 * 64 ? 1 : 2;
+// Few workgroups: 64 queries each instead of 128.  A workgroup's time is its key tiles one after the other, 2.0 us each
+// with 32 queries a wavefront and 1.5 with 16, so as long as the CUs are not full the shorter ones finish first (12
+// heads, 2048 tokens: 34 -> 26 us; 40 heads, 361 tokens 11.1 -> 9.9, 4 x 50 on a prefix of 4000 61 -> 49); full CUs
+// lose by reading every fragment for half the queries (40 heads, 1400 tokens 26 -> 28, 4 x 2048 243 -> 312).  The count
+// looks at queries alone (16 chunks, 1000 new on 8000 cached tokens, 40 heads: 91 us, 89 with 64).
+// (A longest sequence stated far beyond the tokens, within the grid's limit at 128 queries only, is taken at 128.)
+int query_tiles(int64_t num_seqs, int64_t num_tokens, int64_t max_seqlen_q, int num_heads) {
+  return num_heads * (num_tokens / 128 + num_seqs) <= 384 && max_seqlen_q <= 65535 * 64 ? 1 : 2;
+}
+// Key parts of a step on cached prefixes.  Few new tokens on a long prefix leave CUs idle while each workgroup walks its key
+// tiles: the tiles are dealt over as many workgroups as 512 places (two a CU) take, about (tokens / tile + half a tile per
+// sequence) x heads of them being wanted without parts, and at least 8 tiles each, below which writing and adding the
+// parts costs what it saves; and from about 25 us on, since the second launch takes the host 4 (12 x 64 heads, 26 tokens on
+// 1000 cached 20, in two parts 23.5).  Measured (us; 1 part, then as planned): 40 x 128 heads, 1 sequence, 64 tokens on 8000 cached
+// 163, 55; 128 on 1900 48, 33; 4 sequences, 64 on 4000 45, 34; 200 on 4000 48, 39; 8, 64 on 8000 58, 43; 12 x 64 heads, 64 on
+// 8000 103, 25; 4 sequences, 1000 on 4000 35, 25.  Full places lose: 1 sequence, 512 on 1500 52, in two parts 56; 6 sequences,
+// 2048 on 4200 99, in parts of 8 tiles 119; prompts without a prefix (1 x 1500 44, in two parts 52).
+struct KeyParts { int parts, part_tiles; int64_t bytes; };
+KeyParts key_parts(int64_t num_seqs, int64_t num_tokens, int64_t max_seqlen_q, int64_t max_seqlen_k, int num_heads,
+                   int head_size) {
+  const int qt = query_tiles(num_seqs, num_tokens, max_seqlen_q, num_heads);
+  const int64_t bq = 64 * qt, q_tiles = (max_seqlen_q + bq - 1) / bq, tiles = (max_seqlen_k + BKV - 1) / BKV;
+  const int64_t wanted = (2 * num_tokens / bq + num_seqs) * num_heads / 2;
+  const int64_t most = std::min<int64_t>(512 / std::max<int64_t>(wanted, 1), tiles / 8);
+  if (most < 2 || tiles < (head_size == 64 ? 24 : 16) || q_tiles * most > 65535) return KeyParts{1, INT32_MAX / 2, 0};
+  const int part_tiles = (int)std::min<int64_t>((tiles + most - 1) / most, INT32_MAX / 2);
+  return KeyParts{(int)most, part_tiles,
+                  (num_tokens / bq + num_seqs) * num_heads * most *
+                      (head_size == 64 ? unit_floats<64>(qt) : unit_floats<128>(qt)) * 4};
+}
+
+int launch_prefill(PrefillArgs& a, bool paged, int64_t num_seqs, int64_t max_seqlen_q, int64_t max_seqlen_k, int num_heads,
+                   int head_size, int dtype, void* workspace, int64_t workspace_bytes, aps_stream_t stream) {
+  const int qt = query_tiles(num_seqs, a.num_tokens, max_seqlen_q, num_heads);
   const int64_t q_tiles = (max_seqlen_q + 64 * qt - 1) / (64 * qt);
   if (q_tiles > 65535 || num_seqs > 65535 || num_heads > 65535) return APS_ERR_UNSUPPORTED;
-  const dim3 grid((unsigned)num_heads, (unsigned)num_seqs, (unsigned)q_tiles);
+  a.parts = 1; a.part_tiles = INT32_MAX / 2;
+  if (paged && workspace && max_seqlen_k > 0) {
+    const KeyParts kp = key_parts(num_seqs, a.num_tokens, max_seqlen_q, max_seqlen_k, num_heads, head_size);
+    if (workspace_bytes < kp.bytes || (addr(workspace) & 15)) return APS_ERR_WORKSPACE;
+    a.parts = kp.parts; a.part_tiles = kp.part_tiles; a.partial = (float*)workspace;
+  }
+  const dim3 grid((unsigned)num_heads, (unsigned)num_seqs, (unsigned)(q_tiles * a.parts));
   hipStream_t s = (hipStream_t)stream;
   // 64 rows within 32-bit offsets; 16 << shift tokens a block and a row pitch that a 24-bit product takes
   int src = paged ? kPagedAny : kPackedAny;
@@ -381,11 +501,31 @@ int launch_prefill(PrefillArgs& a, bool paged, int64_t num_seqs, int64_t max_seq
 #undef APS_LAUNCH_PF_S
 #undef APS_LAUNCH_PF_D
 #undef APS_LAUNCH_PF
+  const int st = launch_status();
+  if (st != APS_OK || a.parts == 1) return st;
+  const dim3 cgrid((unsigned)num_heads, (unsigned)num_seqs, (unsigned)q_tiles);
+#define APS_LAUNCH_PC(B, D_)                                                                              \
+  do {                                                                                                    \
+    if (qt == 2) APS_LAUNCH((prefill_combine_kernel<B, D_, 2>), cgrid, dim3(kThreads), 0, s, a);          \
+    else APS_LAUNCH((prefill_combine_kernel<B, D_, 1>), cgrid, dim3(kThreads), 0, s, a);                  \
+  } while (0)
+#define APS_LAUNCH_PC_D(B) do { if (head_size == 64) APS_LAUNCH_PC(B, 64); else APS_LAUNCH_PC(B, 128); } while (0)
+  if (dtype == APS_F16) APS_LAUNCH_PC_D(false); else APS_LAUNCH_PC_D(true);
+#undef APS_LAUNCH_PC_D
+#undef APS_LAUNCH_PC
   return launch_status();
 }
 }  // namespace
 
 extern "C" {
+
+int64_t aps_paged_prefill_attention_workspace_bytes(int64_t num_seqs, int64_t num_q_tokens, int64_t max_seqlen_q,
+                                                    int64_t max_seqlen_k, int num_heads, int head_size) {
+  if (num_seqs <= 0 || num_q_tokens <= 0 || max_seqlen_q <= 0 || max_seqlen_k <= 0 || num_heads <= 0 || num_heads > 65535 ||
+      (head_size != 64 && head_size != 128))
+    return 0;
+  return key_parts(num_seqs, num_q_tokens, max_seqlen_q, max_seqlen_k, num_heads, head_size).bytes;
+}
 
 int aps_varlen_prefill_attention(void* out, const void* q, const void* k, const void* v, const int32_t* cu_seqlens,
                                  int64_t num_seqs, int64_t num_tokens, int64_t max_seqlen, int num_heads,
@@ -411,16 +551,16 @@ int aps_varlen_prefill_attention(void* out, const void* q, const void* k, const 
   a.num_heads = num_heads;
   a.num_tokens = num_tokens;
   a.scale_log2 = softmax_scale * kLog2e;
-  return launch_prefill(a, false, num_seqs, max_seqlen, num_heads, head_size, dtype, stream);
+  return launch_prefill(a, false, num_seqs, max_seqlen, max_seqlen, num_heads, head_size, dtype, nullptr, 0, stream);
 }
 
-int aps_paged_prefill_attention(void* out, const void* q, const void* k_cache, const void* v_cache,
+int aps_paged_prefill_attention_split(void* out, const void* q, const void* k_cache, const void* v_cache,
                                 const int32_t* block_tables, const int32_t* cu_seqlens_q,
                                 const int32_t* cu_seqlens_k, int64_t num_seqs, int64_t num_q_tokens,
                                 int64_t max_seqlen_q, int num_heads, int head_size, int block_size,
                                 int64_t table_stride, int64_t table_width, int64_t q_stride, int64_t out_stride,
                                 int64_t cache_block_stride, int64_t num_cache_blocks, float softmax_scale, int dtype,
-                                aps_stream_t stream) {
+                                int64_t max_seqlen_k, void* workspace, int64_t workspace_bytes, aps_stream_t stream) {
   if (num_seqs < 0 || num_q_tokens < 0 || max_seqlen_q < 0 || num_heads <= 0 || head_size <= 0 || block_size <= 0 ||
       table_width < 0 || num_cache_blocks < 0)
     return APS_ERR_INVALID_ARG;
@@ -446,7 +586,21 @@ int aps_paged_prefill_attention(void* out, const void* q, const void* k_cache, c
   a.num_heads = num_heads;
   a.num_tokens = num_q_tokens;
   a.scale_log2 = softmax_scale * kLog2e;
-  return launch_prefill(a, true, num_seqs, max_seqlen_q, num_heads, head_size, dtype, stream);
+  return launch_prefill(a, true, num_seqs, max_seqlen_q, max_seqlen_k, num_heads, head_size, dtype, workspace, workspace_bytes,
+                        stream);
+}
+
+int aps_paged_prefill_attention(void* out, const void* q, const void* k_cache, const void* v_cache,
+                                const int32_t* block_tables, const int32_t* cu_seqlens_q,
+                                const int32_t* cu_seqlens_k, int64_t num_seqs, int64_t num_q_tokens,
+                                int64_t max_seqlen_q, int num_heads, int head_size, int block_size,
+                                int64_t table_stride, int64_t table_width, int64_t q_stride, int64_t out_stride,
+                                int64_t cache_block_stride, int64_t num_cache_blocks, float softmax_scale, int dtype,
+                                aps_stream_t stream) {
+  return aps_paged_prefill_attention_split(out, q, k_cache, v_cache, block_tables, cu_seqlens_q, cu_seqlens_k, num_seqs,
+                                           num_q_tokens, max_seqlen_q, num_heads, head_size, block_size, table_stride,
+                                           table_width, q_stride, out_stride, cache_block_stride, num_cache_blocks,
+                                           softmax_scale, dtype, 0, nullptr, 0, stream);
 }
 
 }  // extern "C"

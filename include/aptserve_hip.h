@@ -398,6 +398,26 @@ int aps_paged_prefill_attention(
     int64_t out_stride, int64_t cache_block_stride, int64_t num_cache_blocks,
     float softmax_scale, int dtype, aps_stream_t stream);
 
+/* The same with the keys of a sequence dealt over several workgroups, whose fp32
+ * sums go through `workspace` (16-byte aligned) and are added by a second launch.
+ * It pays where few new tokens continue long prefixes; how many parts, and that
+ * there is more than one at all, follows from the sizes:
+ * aps_paged_prefill_attention_workspace_bytes says what the call needs (0: one
+ * part).  max_seqlen_k sizes the parts only: a sequence may be longer.  A null
+ * workspace means one part; one too small is APS_ERR_WORKSPACE. */
+int64_t aps_paged_prefill_attention_workspace_bytes(
+    int64_t num_seqs, int64_t num_q_tokens, int64_t max_seqlen_q,
+    int64_t max_seqlen_k, int num_heads, int head_size);
+int aps_paged_prefill_attention_split(
+    void* out, const void* q, const void* k_cache, const void* v_cache,
+    const int32_t* block_tables, const int32_t* cu_seqlens_q,
+    const int32_t* cu_seqlens_k, int64_t num_seqs, int64_t num_q_tokens,
+    int64_t max_seqlen_q, int num_heads, int head_size, int block_size,
+    int64_t table_stride, int64_t table_width, int64_t q_stride,
+    int64_t out_stride, int64_t cache_block_stride, int64_t num_cache_blocks,
+    float softmax_scale, int dtype, int64_t max_seqlen_k, void* workspace,
+    int64_t workspace_bytes, aps_stream_t stream);
+
 /* ------------------------------------------------------------------------
  * Ragged-batch metadata, built on the GPU from a per-sequence description.
  * ref: worker/aptserve_model_runner.py:240-842 (_prepare_model_input), hybrid

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 import torch
 
-from aptserve_hip import ops
+from aptserve_hip import _lib, ops
 from oracle import attention as OA
 from util import randn
 
@@ -167,6 +167,53 @@ def test_longest_sequence_stated_beyond_the_tokens(dev, max_seqlen):
     assert torch.allclose(a.float(), b.float(), atol=2e-3, rtol=2e-3)   # (64 and 128 queries a workgroup: other key order)
     with pytest.raises(RuntimeError):
         ops.flash_attn_varlen_func(q, k, v, cu_seqlens_q=cu, max_seqlen_q=65535 * 128 + 1, softmax_scale=0.125)
+
+
+@pytest.mark.parametrize("H,D,BS,dtype", [(2, 64, 16, torch.float16), (2, 128, 48, torch.bfloat16), (80, 128, 16, torch.float16),
+                                          (80, 64, 32, torch.bfloat16)])
+def test_prefix_attention_in_key_parts(dev, H, D, BS, dtype):
+    """Few new tokens on long prefixes: the keys of a sequence in parts (64 queries a workgroup with 2 heads, 128 with 80).
+    Lengths on and about the edges of the parts, one that fits a single part, queries that see nothing of the last part;
+    NaN behind every sequence.  A null workspace means one part, whose 16-bit probabilities are rounded against another
+    maximum: each may differ by 2 u of itself (u = 2^-11, bf16 2^-8) and, below fp16's normal numbers, by 2^-24, so the
+    weighted mean of V by (2 u + 2^-24 keys) max |V|; and the result is rounded once."""
+    from test_oracle_attention import build_paged
+    lib = _lib.load()
+    klens, qlens = [1538, 833, 64, 1025], [70, 1, 3, 64]
+    T, mq, mk = sum(qlens), max(qlens), max(klens)
+    need = lib.aps_paged_prefill_attention_workspace_bytes(4, T, mq, mk, H, D)
+    assert need > 0
+    run_prefix(dev, klens, qlens, H, D, dtype, BS=BS, poison=True)
+    kc, vc, bt, _, _ = (x.to(dev) if isinstance(x, torch.Tensor) else x for x in build_paged(4, H, D, BS, klens, 3, dtype=dtype))
+    q = randn((T, H, D), 4, dtype).to(dev)
+    cu_q, cu_k = (torch.tensor([0] + list(np.cumsum(n)), dtype=torch.int32, device=dev) for n in (qlens, klens))
+    outs = []
+    for ws in (torch.empty(need, dtype=torch.uint8, device=dev), None):
+        out = torch.full_like(q, float("nan"))
+
+        def call(nbytes):
+            return lib.aps_paged_prefill_attention_split(
+                out.data_ptr(), q.data_ptr(), kc.data_ptr(), vc.data_ptr(), bt.data_ptr(), cu_q.data_ptr(), cu_k.data_ptr(),
+                4, T, mq, H, D, BS, bt.stride(0), bt.size(1), q.stride(0), out.stride(0), kc.stride(0), kc.size(0), D ** -0.5,
+                0 if dtype == torch.float16 else 1, mk, None if ws is None else ws.data_ptr(), nbytes,
+                torch.cuda.current_stream(dev).cuda_stream)
+        assert call(need) == 0
+        if ws is not None:
+            assert call(need - 1) == -3
+        outs.append(out.double())
+    ulp = 2.0 ** (-10 if dtype == torch.float16 else -7)
+    mean = (ulp + (max(klens) * 2.0 ** -24 if dtype == torch.float16 else 0.0)) * vc.abs().max().item()
+    assert ((outs[0] - outs[1]).abs() <= mean + ulp * outs[1].abs()).all()
+
+
+def test_prefix_attention_parts_only_where_workgroups_are_few():
+    lib = _lib.load()
+    need = lib.aps_paged_prefill_attention_workspace_bytes
+    assert need(1, 64, 64, 8064, 40, 128) == 2 * 40 * 8 * 64 * 130 * 4
+    assert need(6, 2048, 807, 2461, 40, 128) == 0       # the CUs are full
+    assert need(1, 64, 64, 960, 40, 128) == 0 < need(1, 64, 64, 961, 40, 128)       # parts of fewer than 8 key tiles
+    assert need(1, 64, 64, 1472, 12, 64) == 0 < need(1, 64, 64, 1473, 12, 64)       # too short for a second launch
+    assert need(0, 0, 0, 0, 40, 128) == 0 and need(1, 64, 64, 0, 40, 128) == 0 and need(1, 64, 64, 8064, 40, 96) == 0
 
 
 def test_prefix_attention_block_size_32_and_argument_errors(dev):
