@@ -17,6 +17,7 @@ that scales with the number of cached tokens.
 from __future__ import annotations
 
 import contextlib
+import ctypes
 import itertools
 from dataclasses import dataclass
 from typing import List, Optional, Sequence
@@ -153,20 +154,22 @@ class _Staging:
             self.bufs[i] = torch.empty(max(n, 4096), dtype=torch.int32, pin_memory=True)
         return i, self.bufs[i][:n]
 
-    def upload(self, i: int, host: torch.Tensor, device, stream) -> torch.Tensor:
-        dev = host.to(device, non_blocking=True)
+    def mark(self, i: int, stream) -> None:
+        """Buffer ``i`` is free once ``stream`` has come this far."""
         ev = torch.cuda.Event()
         ev.record(stream)
         self.events[i] = ev
+
+    def upload(self, i: int, host: torch.Tensor, device, stream) -> torch.Tensor:
+        dev = host.to(device, non_blocking=True)
+        self.mark(i, stream)
         return dev
 
 
     def upload_into(self, i: int, host: torch.Tensor, dst: torch.Tensor, stream) -> torch.Tensor:
         """Like ``upload`` into device memory the caller keeps (same address in every step)."""
         dst.copy_(host, non_blocking=True)
-        ev = torch.cuda.Event()
-        ev.record(stream)
-        self.events[i] = ev
+        self.mark(i, stream)
         return dst
 
 
@@ -256,6 +259,68 @@ def _pack_tables(tables, lens: np.ndarray, out: np.ndarray, rows: Optional[np.nd
     out[rows, cols] = flat
 
 
+def _packed_rows(tables, batch: int) -> bool:
+    """Whether ``tables`` is a packed int32 array whose rows native code can walk (contiguous entries, rows in order)."""
+    return (type(tables) is np.ndarray and tables.ndim == 2 and tables.shape[0] == batch and tables.dtype == np.int32
+            and tables.shape[1] > 0 and tables.strides[1] == 4 and tables.strides[0] % 4 == 0
+            and tables.strides[0] >= 4 * tables.shape[1])
+
+
+def _build_decode_packed(lens: np.ndarray, hid: np.ndarray, tables: np.ndarray, shared: np.ndarray, block_size: int,
+                         device, check_totals: bool) -> Optional[HybridAttentionMetadata]:
+    """Decode step from packed tables in two native calls, one for the sizes and one that packs, uploads and launches.
+    ``None`` where the general path has to say what is wrong."""
+    B = len(lens)
+    lib = _lib.load()
+    stats = (ctypes.c_int64 * 6)()
+    lens_ptr, hid_ptr = lens.ctypes.data, hid.ctypes.data
+    if lib.aps_decode_batch_stats(lens_ptr, hid_ptr, B, ctypes.addressof(stats)) != 0:
+        return None
+    min_len, max_len, n_hs, n_hr, max_hid_len, max_kv_len = stats
+    W, Ws = -(-max_len // block_size), -(-max_hid_len // block_size)
+    if min_len <= 0 or max_len > 0x7fffffff or W > tables.shape[1] or Ws > shared.shape[1]:
+        return None
+    n_kv = B - n_hs
+    num_tot = n_hr + n_kv
+    stream = torch.cuda.current_stream(device)
+    on_device = (contextlib.nullcontext() if torch.cuda.current_device() == stream.device_index
+                 else torch.cuda.device(device))
+    stg = _staging.setdefault(device, _Staging())
+    slot, host = stg.take(2 * B + B * (W + Ws))
+    packed = torch.empty(2 * B + B * (W + Ws), dtype=torch.int32, device=device)
+    sizes64 = [num_tot, n_hr, n_hr, n_kv, n_hs, n_hs, B, num_tot - B, B, 4, num_tot, num_tot, n_hr, n_hs + 1, n_kv, B]
+    buf64 = torch.empty(sum(sizes64), dtype=torch.int64, device=device)
+    sizes32 = [B * W, B + 1, B + 1, B, B, (B * W + 3) // 4 if n_hs else 0]
+    buf32 = torch.empty(sum(sizes32), dtype=torch.int32, device=device)
+    with on_device:
+        st = lib.aps_build_decode_metadata_from_host(
+            lens_ptr, hid_ptr, B, block_size, tables.ctypes.data, tables.strides[0] // 4, W, shared.ctypes.data,
+            shared.strides[0] // 4, Ws, n_hs, n_hr, host.data_ptr(), packed.data_ptr(), buf64.data_ptr(), buf32.data_ptr(),
+            stream.cuda_stream)
+    stg.mark(slot, stream)
+    _lib.check(st, "build_decode_metadata")
+    (slot_mapping, slot_mapping_shared, use_tot, kv_use, use_input, store_tot, upd, pull, positions, totals, holder_src,
+     kv_dest, hidden_slots, hidden_seq_start, kv_use_input, new_token_slot) = torch.split(buf64, sizes64)
+    bt_out, seq_start, query_start, ctx, kv_seq_lens, types32 = torch.split(buf32, sizes32)
+    d_lens, _, d_bt, _ = torch.split(packed, [B, B, B * W, B * Ws])
+    if check_totals:
+        got = totals.tolist()
+        if got != [num_tot, n_hr, n_hs, n_kv]:
+            raise RuntimeError(f"device totals {got} disagree with the host's {[num_tot, n_hr, n_hs, n_kv]}")
+    return HybridAttentionMetadata(
+        num_prefills=0, num_prefill_tokens=0, num_decode_tokens=B, num_hidden_cache_tokens=n_hs, num_tot_tokens=num_tot,
+        slot_mapping=slot_mapping, slot_mapping_shared=slot_mapping_shared, hidden_cache_use_tot=use_tot,
+        kv_cache_use_tot=kv_use, hidden_cache_use_input=use_input, hidden_cache_store_tot=store_tot, hidden_holder_upd=upd,
+        hidden_holder_pull=pull, seq_lens=lens.tolist(), seq_lens_tensor=d_lens, max_query_len=1, max_prefill_seq_len=0,
+        max_decode_seq_len=max_len, query_start_loc=query_start, seq_start_loc=seq_start, context_lens_tensor=ctx,
+        block_tables=bt_out.view(B, W), use_cuda_graph=False, input_positions=positions,
+        # per-block source for the hybrid attention: every block of a hidden sequence is a workspace block
+        block_types=types32.view(torch.uint8)[:B * W].view(B, W) if n_hs else None, holder_src=holder_src,
+        kv_dest=kv_dest, hidden_slots=hidden_slots, hidden_seq_start=hidden_seq_start, max_hidden_seq_len=max_hid_len,
+        kv_cache_use_input=kv_use_input, new_token_slot=new_token_slot, kv_seq_lens=kv_seq_lens,
+        max_kv_seq_len=max_kv_len, private_block_tables=d_bt.view(B, W))
+
+
 def build_metadata(is_prompt: bool, seq_lens: Sequence[int], use_hidden: Sequence[bool],
                    block_tables: Sequence[Sequence[int]], block_tables_4_shared: Sequence[Sequence[int]],
                    block_size: int, device, context_lens: Optional[Sequence[int]] = None,
@@ -285,6 +350,12 @@ def build_metadata(is_prompt: bool, seq_lens: Sequence[int], use_hidden: Sequenc
     hid = np.asarray(use_hidden, dtype=bool)
     if len(hid) != B or len(block_tables) != B:
         raise ValueError("seq_lens, use_hidden and block_tables must have one entry per sequence")
+    if (not is_prompt and static is None and block_size > 0 and lens.ndim == 1 and hid.ndim == 1
+            and _packed_rows(block_tables, B) and _packed_rows(block_tables_4_shared, B)):
+        md = _build_decode_packed(np.ascontiguousarray(lens), np.ascontiguousarray(hid), block_tables,
+                                  block_tables_4_shared, block_size, device, check_totals)
+        if md is not None:
+            return md
     if np.any(lens <= 0):
         raise ValueError("sequence lengths must be positive")
     need_blocks = -(-lens // block_size)
@@ -383,7 +454,7 @@ def build_metadata(is_prompt: bool, seq_lens: Sequence[int], use_hidden: Sequenc
                 kv_use.data_ptr() if n_kv else None, use_input.data_ptr() if n_hs else None,
                 store_tot.data_ptr() if n_hs else None, upd.data_ptr(), pull.data_ptr() if num_tot > B else None,
                 holder_src.data_ptr(), kv_dest.data_ptr(), hidden_slots.data_ptr() if n_hr else None,
-                hidden_seq_start.data_ptr() if n_hs else None, kv_use_input.data_ptr() if n_kv else None,
+                hidden_seq_start.data_ptr(), kv_use_input.data_ptr() if n_kv else None,
                 new_token_slot.data_ptr(), kv_seq_lens.data_ptr(), num_tot, n_hr, n_hs, n_kv,
                 bt_out.data_ptr() if Wo else None, Wo, Wo,
                 None if block_types is None else block_types.data_ptr(), seq_start.data_ptr(),

@@ -474,6 +474,34 @@ int aps_build_decode_metadata(
     int32_t* query_start_loc, int32_t* context_lens, int64_t* input_positions,
     int64_t* totals, aps_stream_t stream);
 
+/* The same from the host's arrays in one call: packs lengths, flags and tables
+ * into `staging` (pinned; 2 batch + batch (width + shared_width) words), copies it
+ * to `packed` (device, as many) and launches the builder.  block_tables /
+ * block_tables_shared are HOST arrays, 0-padded rows table_stride / shared_stride
+ * entries apart of which width / shared_width <= width count; rows of the shared
+ * table of K/V-cached sequences are taken as empty.  out64 holds, one behind the
+ * other (tot = hidden_rows + K/V-cached sequences, kv = those): slot_mapping[tot],
+ * slot_mapping_shared and hidden_cache_use_tot[hidden_rows], kv_cache_use_tot[kv],
+ * hidden_cache_use_input and hidden_cache_store_tot[hidden_seqs],
+ * hidden_holder_upd[batch], hidden_holder_pull[tot - batch], input_positions[batch],
+ * totals[4], holder_src and kv_dest[tot], hidden_slots[hidden_rows],
+ * hidden_seq_start[hidden_seqs + 1], kv_cache_use_input[kv], new_token_slot[batch];
+ * out32 block_tables_out[batch, width], seq_start_loc and query_start_loc[batch + 1],
+ * context_lens and kv_seq_lens[batch], block_types_out[batch, width] bytes.  Lengths
+ * are positive int32 values; hidden_seqs and hidden_rows are checked against the
+ * arrays.  staging may be written again once the stream has passed the copy. */
+int aps_build_decode_metadata_from_host(
+    const int64_t* seq_lens, const uint8_t* use_hidden, int64_t batch,
+    int block_size, const int32_t* block_tables, int64_t table_stride,
+    int64_t width, const int32_t* block_tables_shared, int64_t shared_stride,
+    int64_t shared_width, int64_t hidden_seqs, int64_t hidden_rows,
+    int32_t* staging, int32_t* packed, int64_t* out64, int32_t* out32,
+    aps_stream_t stream);
+/* stats[6] (host): shortest and longest length, hidden-cached sequences, their
+ * tokens, the longest of them, the longest K/V-cached sequence (0: none). */
+int aps_decode_batch_stats(const int64_t* seq_lens, const uint8_t* use_hidden,
+                           int64_t batch, int64_t* stats);
+
 /* Prompt step (:542-552, :648-666).  Row space = token space; token i of a
  * sequence (i in [context_len, seq_len)) gets slot table[i/BS]*BS + i%BS, or
  * -1 when table_width is 0.  hidden_cache_use_input = tokens of hidden-cached

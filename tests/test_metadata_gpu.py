@@ -65,6 +65,56 @@ def test_packed_tables_give_the_same_metadata_as_lists(dev, frac, prompt):
     assert_same(md, oracle_metadata(batch))
 
 
+@pytest.mark.parametrize("frac", [0.0, 0.4, 1.0])
+@pytest.mark.parametrize("n,bs", [(1, 16), (11, 16), (257, 32)])
+def test_native_packing_equals_the_general_path(dev, frac, n, bs):
+    """Packed int32 tables are packed, uploaded and expanded by one native call: every field, tensors and numbers alike,
+    equals what the general path makes of the same batch (lists; int64, transposed and reversed arrays take it too), for
+    close rows, row slices, wider rows and lengths and flags that are strided."""
+    import dataclasses
+    batch = workloads.small_decode_batch(7, n, 300, frac, 400 * (n // 11 + 1), bs)
+    bt, bts = batch.packed_tables()
+    if bts.shape[1] == 0:
+        bts = np.zeros((n, 1), dtype=np.int32)
+    lens, hid = np.asarray(batch.seq_lens), np.asarray(batch.use_hidden, dtype=bool)
+    general = metadata.build_from_batch(batch, dev)
+    wide = lambda a: np.concatenate([a, np.full((n, 5), 99, dtype=a.dtype)], axis=1)
+    reverse = lambda a: a[::-1].copy()[::-1]
+    forms = [(bt, bts, lens, hid), (wide(bt), wide(bts)[:, :bts.shape[1]], lens, hid),
+             (np.repeat(bt, 2, 0)[::2], bts, np.repeat(lens, 2)[::2], np.repeat(hid, 2)[::2]),
+             (bt.astype(np.int64), bts, lens, hid), (np.asfortranarray(bt), np.asfortranarray(bts), lens, hid),
+             (reverse(bt), reverse(bts), reverse(lens), reverse(hid))]
+    native = [metadata._packed_rows(f[0], n) and metadata._packed_rows(f[1], n) for f in forms]
+    assert native[:4] == [True, True, True, False] and (n == 1 or native[5] is False)
+    for f in forms:
+        md = metadata.build_metadata(False, f[2], f[3], f[0], f[1], bs, dev, check_totals=True)
+        for field in dataclasses.fields(md):
+            a, b = getattr(md, field.name), getattr(general, field.name)
+            if isinstance(b, torch.Tensor):
+                assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b), field.name
+            else:
+                assert a == b and type(a) is type(b), field.name
+
+
+def test_native_packing_checks_its_sizes():
+    """Host only: the reductions, and sizes that disagree with the arrays are refused before anything is launched."""
+    from aptserve_hip import _lib
+    lib = _lib.load()
+    lens, hid = np.array([5, 40, 17], dtype=np.int64), np.array([True, False, True])
+    stats = np.zeros(6, dtype=np.int64)
+    assert lib.aps_decode_batch_stats(lens.ctypes.data, hid.ctypes.data, 3, stats.ctypes.data) == 0
+    assert stats.tolist() == [5, 40, 2, 22, 17, 40]
+    bt, out = np.ones((3, 3), dtype=np.int32), np.zeros(256, dtype=np.int64)
+
+    def call(n_hs=2, n_hr=22, width=3, stride=3, swidth=2, lens=lens):
+        p = out.ctypes.data
+        return lib.aps_build_decode_metadata_from_host(lens.ctypes.data, hid.ctypes.data, 3, 16, bt.ctypes.data, stride, width,
+                                                       bt.ctypes.data, 3, swidth, n_hs, n_hr, p, p, p, p, None)
+    for bad in (dict(n_hs=1), dict(n_hr=21), dict(stride=2), dict(swidth=4), dict(n_hs=4), dict(lens=np.array([5, 0, 17])),
+                dict(lens=np.array([5, 1 << 31, 17]))):
+        assert call(**bad) == -1, bad
+
+
 def test_packed_tables_wider_than_needed_and_too_narrow(dev):
     """Packed tables may be wider than the longest sequence needs (a runner keeps them at a fixed width): the
     extra columns are ignored.  Tables narrower than ceil(seq_len / block_size) are refused, the private one
