@@ -333,12 +333,17 @@ class HybridOPTAttention:
                                           md.hidden_cache_use_input, md.max_hidden_seq_len, w[s:2 * s], w[2 * s:],
                                           None if b is None else b[2 * s:], self.scaling, attn_output, kv_job=kv_job,
                                           store_job=store_job)
-        with phase("projections"):
-            return ops.linear_nt(attn_output, self.out_weight, self.out_bias)
+        return attn_output
 
     def forward(self, hidden_states, kv_cache, shared_cache, attn_metadata: HybridAttentionMetadata,
                 hidden_cache=None):
-        """``hidden_cache``: where hidden rows are cached when it is not ``kv_cache`` itself — a separate
+        """:meth:`attend` and the out projection."""
+        attn_output = self.attend(hidden_states, kv_cache, shared_cache, attn_metadata, hidden_cache)
+        with phase("projections"):
+            return ops.linear_nt(attn_output, self.out_weight, self.out_bias)
+
+    def attend(self, hidden_states, kv_cache, shared_cache, attn_metadata: HybridAttentionMetadata, hidden_cache=None):
+        """Everything up to the out projection.  ``hidden_cache``: where hidden rows are cached when it is not ``kv_cache`` itself — a separate
         ``(2, N, BS, H, D)`` tensor in the activation dtype, needed with an fp8 K/V cache (whose bytes cannot hold
         16-bit hidden rows)."""
         md = attn_metadata
@@ -367,8 +372,7 @@ class HybridOPTAttention:
                                                   kv_cache[0], kv_cache[1], md.kv_dest)
                     with phase("attention"):
                         attn_output = self.attn.forward(q, None, None, kv_cache, shared_cache, md, kv_written=True)
-                    with phase("projections"):
-                        return ops.linear_nt(attn_output, self.out_weight, self.out_bias)
+                    return attn_output
                 if self.fused and md.holder_src is not None:
                     holder = torch.empty(md.num_tot_tokens, hidden_states.shape[1], device=hidden_states.device,
                                          dtype=hidden_states.dtype)
@@ -392,8 +396,7 @@ class HybridOPTAttention:
                                                   shared_cache[1], kv_cache[0], kv_cache[1], md.kv_dest)
                     with phase("attention"):
                         attn_output = self.attn.forward(q, None, None, kv_cache, shared_cache, md, kv_written=True)
-                    with phase("projections"):
-                        return ops.linear_nt(attn_output, self.out_weight, self.out_bias)
+                    return attn_output
                 else:
                     kv, _ = self.qkv_proj(holder, q_only=False, kv_only=True)
                     k, v = kv.chunk(chunks=2, dim=-1)
@@ -406,7 +409,7 @@ class HybridOPTAttention:
                                             self.attn.kv_cache_dtype, self.attn.k_scale, self.attn.v_scale,
                                             hidden_cache=hidden_cache)
                 attn_output = self.attn.forward(q, k, v, kv_cache, shared_cache, md, kv_written=True)
-                return ops.linear_nt(attn_output, self.out_weight, self.out_bias)
+                return attn_output
             else:                                                                   # :125-127
                 ops.hidden_to_cache(hidden_states, hc, md.slot_mapping, md.hidden_cache_use_input,
                                     md.hidden_cache_store_tot)
@@ -415,8 +418,7 @@ class HybridOPTAttention:
         else:                                                                       # :128-130
             qkv, _ = self.qkv_proj(hidden_states)
             q, k, v = qkv.chunk(chunks=3, dim=-1)
-        attn_output = self.attn.forward(q, k, v, kv_cache, shared_cache, md)
-        return ops.linear_nt(attn_output, self.out_weight, self.out_bias)
+        return self.attn.forward(q, k, v, kv_cache, shared_cache, md)
 
     __call__ = forward
 

@@ -982,6 +982,40 @@ def add_layer_norm(x, residual, weight, bias, eps: float = 1e-5, out=None, sum_o
     return out, (x if residual is None else sum_out)
 
 
+def linear_add_layer_norm(x, weight, bias, residual, ln_weight, ln_bias, eps: float = 1e-5):
+    """:func:`linear_nt` and :func:`add_layer_norm` of its result in one call, with the same results: the out projection
+    and ``fc2`` of a layer with the residual add and the norm behind them
+    (additional_designs/model_executor/models/aptserve_opt.py:186-211).  Where the product is split along K, the norm's
+    launch adds the parts.  Returns ``(normed, sum)``."""
+    dev = x.device
+    _check_data("x", x, dev)
+    _check_data("weight", weight, dev)
+    _check_data("residual", residual, dev)
+    _need(x.dim() == 2 and weight.dim() == 2 and x.size(1) == weight.size(1), "x [M,K] and weight [N,K] expected")
+    _need(x.dtype == weight.dtype and x.dtype in (torch.float16, torch.bfloat16), "f16 or bf16 operands expected")
+    M, K = x.shape
+    N = weight.size(0)
+    _need(ln_weight is not None, "ln_weight is required")
+    for n, t in (("bias", bias), ("ln_weight", ln_weight), ("ln_bias", ln_bias)):
+        if t is not None:
+            _check_data(n, t, dev)
+            _need(t.dim() == 1 and t.numel() == N and t.dtype == x.dtype and t.is_contiguous(),
+                  f"{n} must be a contiguous [N] vector of the operand dtype")
+    _need(residual.shape == (M, N) and residual.dtype == x.dtype, "residual must look like the product")
+    normed, total, product = (torch.empty(M, N, dtype=x.dtype, device=dev) for _ in range(3))
+    lib = _lib.load()
+    need = lib.aps_linear_nt_workspace_bytes(M, N, K)
+    workspace = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
+    with _on(dev):
+        st = lib.aps_linear_add_layer_norm(
+            normed.data_ptr(), total.data_ptr(), product.data_ptr(), x.data_ptr(), weight.data_ptr(), _ptr(bias),
+            residual.data_ptr(), ln_weight.data_ptr(), _ptr(ln_bias), M, N, K, x.stride(0), weight.stride(0),
+            residual.stride(0), float(eps), _DTYPE_CODE[x.dtype], _ptr(workspace), need,
+            _tile_counters(dev).data_ptr() if need else None, _stream(x))
+    _lib.check(st, "linear_add_layer_norm")
+    return normed, total
+
+
 # ------------------------------------------------------------------ block maintenance
 
 _LAYER_BASES = {}

@@ -107,14 +107,16 @@ class HybridOPTDecoderLayer:
         self.self_attn = HybridOPTAttention(cfg.hidden_size, cfg.num_attention_heads, w[prefix + "qkv_w"],
                                             w[prefix + "qkv_b"], w[prefix + "out_w"], w[prefix + "out_b"], **attn_kw)
 
-    def _mlp(self, x):
-        """fc1 with its ReLU (stored by fc1's own epilogue), then fc2."""
+    def _fc1(self, x):
+        """fc1 with its ReLU (stored by fc1's own epilogue)."""
         w, p = self.w, self.p
+        # more rows than the weight-streaming products take: the tile kernel reads x by k-tiles too
+        out = row_pitched(x.size(0), w[p + "fc1_w"].size(0), x.dtype, x.device) if x.size(0) > 48 else None
+        return ops.linear_nt(x, w[p + "fc1_w"], w[p + "fc1_b"], out=out, relu=True)
+
+    def _mlp(self, x):
         with phase("projections"):
-            # more rows than the weight-streaming products take: the tile kernel reads x by k-tiles too
-            out = row_pitched(x.size(0), w[p + "fc1_w"].size(0), x.dtype, x.device) if x.size(0) > 48 else None
-            x = ops.linear_nt(x, w[p + "fc1_w"], w[p + "fc1_b"], out=out, relu=True)
-            return ops.linear_nt(x, w[p + "fc2_w"], w[p + "fc2_b"])
+            return ops.linear_nt(self._fc1(x), self.w[self.p + "fc2_w"], self.w[self.p + "fc2_b"])
 
     def forward(self, hidden_states, kv_cache, shared_cache, md: HybridAttentionMetadata):
         """additional_designs/model_executor/models/aptserve_opt.py:179-212 with plain element-wise ops."""
@@ -128,15 +130,19 @@ class HybridOPTDecoderLayer:
         return residual + self._mlp(hidden_states)
 
     def forward_fused_norm(self, residual, normed, kv_cache, shared_cache, md, next_ln_w, next_ln_b):
-        """The same layer with every (residual add, LayerNorm) pair in one launch.  ``normed`` is this layer's
+        """The same layer with every (residual add, LayerNorm) pair in one launch, which also adds the K parts of the
+        product in front of it where there are any.  ``normed`` is this layer's
         ``self_attn_layer_norm`` of ``residual`` (computed by the previous layer's last launch); returns the
         layer's output and the NEXT norm of it (the next layer's ``self_attn_layer_norm``, or the decoder's
         final one)."""
         w, p = self.w, self.p
-        attn = self.self_attn(normed, kv_cache, shared_cache, md)
-        normed, residual = ops.add_layer_norm(attn, residual, w[p + "final_ln_w"], w[p + "final_ln_b"])
-        mlp = self._mlp(normed)
-        normed, residual = ops.add_layer_norm(mlp, residual, next_ln_w, next_ln_b)
+        a = self.self_attn
+        attn = a.attend(normed, kv_cache, shared_cache, md)
+        with phase("projections"):
+            normed, residual = ops.linear_add_layer_norm(attn, a.out_weight, a.out_bias, residual, w[p + "final_ln_w"],
+                                                         w[p + "final_ln_b"])
+            normed, residual = ops.linear_add_layer_norm(self._fc1(normed), w[p + "fc2_w"], w[p + "fc2_b"], residual,
+                                                         next_ln_w, next_ln_b)
         return residual, normed
 
     __call__ = forward

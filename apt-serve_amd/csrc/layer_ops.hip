@@ -20,6 +20,10 @@ struct AddLnArgs {
   int64_t x_stride_b, res_stride_b, normed_stride_b, sum_stride_b;
   int width;
   float eps;
+  // PARTS: x is a product in K parts, fp32 planes [rows][width] that are added in order, plus its bias (nullable), rounded once
+  const float* partial; const char* lin_bias;
+  int64_t plane;
+  int parts;
 };
 
 __device__ __forceinline__ float block_sum(float v, float* red) {
@@ -41,7 +45,53 @@ __device__ __forceinline__ uint32_t to16(float v) {
   return BF16 ? f32_to_bf16_bits(v) : f32_to_f16_bits(v);
 }
 
+// The thread's vectors of a row of the product, rounded: parts in order, those of all vectors in flight together (a vector at a
+// time 7.2 us for 5 rows of 4 parts, 10.8 for 361; so 4.9 and 9.7), then the bias.  Past the row's end: its last vector.
 template <bool BF16, int VECS>
+__device__ __forceinline__ void product_vecs(const AddLnArgs& g, int64_t row, int nvec, u32x4 (&a)[VECS]) {
+  constexpr int ZC = VECS <= 3 ? 3 : 1;
+  const float* p[VECS];
+  float4v s[VECS][2];
+  u32x4 c[VECS];
+#pragma unroll
+  for (int j = 0; j < VECS; ++j) {
+    const int i = min((int)threadIdx.x + j * kLnThreads, nvec - 1);
+    p[j] = g.partial + row * g.width + (int64_t)i * 8;
+    s[j][0] = *(const float4v*)p[j]; s[j][1] = *(const float4v*)(p[j] + 4);
+    c[j] = g.lin_bias ? *(const u32x4*)(g.lin_bias + (int64_t)i * 16) : u32x4{0u, 0u, 0u, 0u};
+  }
+  for (int z0 = 1; z0 < g.parts; z0 += ZC) {
+    float4v t[ZC][VECS][2];
+#pragma unroll
+    for (int z = 0; z < ZC; ++z)
+#pragma unroll
+      for (int j = 0; j < VECS; ++j) {
+        const float* q = p[j] + (int64_t)min(z0 + z, g.parts - 1) * g.plane;
+        t[z][j][0] = *(const float4v*)q; t[z][j][1] = *(const float4v*)(q + 4);
+      }
+#pragma unroll
+    for (int z = 0; z < ZC; ++z)
+      if (z0 + z < g.parts) {
+#pragma unroll
+        for (int j = 0; j < VECS; ++j)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { s[j][0][e] += t[z][j][0][e]; s[j][1][e] += t[z][j][1][e]; }
+      }
+  }
+#pragma unroll
+  for (int j = 0; j < VECS; ++j)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      float lo = s[j][e >> 1][2 * (e & 1)], hi = s[j][e >> 1][2 * (e & 1) + 1];
+      if (g.lin_bias) { lo += from16<BF16>(c[j][e] & 0xffffu); hi += from16<BF16>(c[j][e] >> 16); }
+      a[j][e] = to16<BF16>(lo) | (to16<BF16>(hi) << 16);
+    }
+}
+
+// PARTS: the sum over a product's K parts is taken here instead of in a launch of its own that writes the product for this
+// one to read (361 rows of 5120 in 4 parts: 9.7 us for 7.0 + 6.5 and the gap between them; 5 rows 4.9, and the product in front
+// of it, which no longer adds its parts by itself, 35.3 instead of 39.1).
+template <bool BF16, int VECS, bool PARTS>
 __global__ __launch_bounds__(kLnThreads) void add_layer_norm_kernel(const AddLnArgs g) {
   __shared__ float red[4];
   const int64_t row = blockIdx.x;
@@ -59,13 +109,20 @@ __global__ __launch_bounds__(kLnThreads) void add_layer_norm_kernel(const AddLnA
     gw[j] = *(const u32x4*)(g.gamma + (int64_t)i * 16);
     gb[j] = g.beta ? *(const u32x4*)(g.beta + (int64_t)i * 16) : u32x4{0u, 0u, 0u, 0u};
   }
+  // (past the row's end: its last vector, loaded and not used, so that no load stands behind a branch)
+  u32x4 pa[VECS], pb[VECS];
+#pragma unroll
+  for (int j = 0; j < VECS; ++j) {
+    const int i = min((int)threadIdx.x + j * kLnThreads, nvec - 1);
+    if constexpr (!PARTS) pa[j] = *(const u32x4*)(x + (int64_t)i * 16);
+    pb[j] = r ? *(const u32x4*)(r + (int64_t)i * 16) : u32x4{0u, 0u, 0u, 0u};
+  }
+  if constexpr (PARTS) product_vecs<BF16, VECS>(g, row, nvec, pa);
 #pragma unroll
   for (int j = 0; j < VECS; ++j) {
     const int i = threadIdx.x + j * kLnThreads;
     if (i < nvec) {
-      const u32x4 a = *(const u32x4*)(x + (int64_t)i * 16);
-      u32x4 b = {0u, 0u, 0u, 0u};
-      if (r) b = *(const u32x4*)(r + (int64_t)i * 16);
+      const u32x4 a = pa[j], b = pb[j];
       u32x4 s16;
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
@@ -117,6 +174,24 @@ __global__ __launch_bounds__(kLnThreads) void add_layer_norm_kernel(const AddLnA
 
 using namespace aps;
 
+namespace {
+template <bool PARTS>
+int launch_add_layer_norm(const AddLnArgs& g, int64_t rows, int dtype, aps_stream_t stream) {
+  const dim3 grid((unsigned)rows);
+  // rows of up to 3 * 256 * 8 = 6144 elements (every OPT up to 13B) keep 3 vectors per thread, wider ones 8
+  const bool narrow = g.width <= 3 * kLnThreads * 8;
+  hipStream_t s = (hipStream_t)stream;
+  if (dtype == APS_BF16) {
+    if (narrow) APS_LAUNCH((add_layer_norm_kernel<true, 3, PARTS>), grid, dim3(kLnThreads), 0, s, g);
+    else APS_LAUNCH((add_layer_norm_kernel<true, kLnVecs, PARTS>), grid, dim3(kLnThreads), 0, s, g);
+  } else {
+    if (narrow) APS_LAUNCH((add_layer_norm_kernel<false, 3, PARTS>), grid, dim3(kLnThreads), 0, s, g);
+    else APS_LAUNCH((add_layer_norm_kernel<false, kLnVecs, PARTS>), grid, dim3(kLnThreads), 0, s, g);
+  }
+  return launch_status();
+}
+}  // namespace
+
 extern "C" int aps_add_layer_norm(void* normed, void* sum, const void* x, const void* residual, const void* gamma,
                                   const void* beta, int64_t rows, int64_t width, int64_t x_stride,
                                   int64_t residual_stride, int64_t normed_stride, int64_t sum_stride, float eps,
@@ -134,17 +209,16 @@ extern "C" int aps_add_layer_norm(void* normed, void* sum, const void* x, const 
                         (uint64_t)sum_stride * 2}) != 16)
     return APS_ERR_UNSUPPORTED;
   AddLnArgs g{(char*)normed, (char*)sum, (const char*)x, (const char*)residual, (const char*)gamma,
-              (const char*)beta, x_stride * 2, residual_stride * 2, normed_stride * 2, sum_stride * 2, (int)width, eps};
-  const dim3 grid((unsigned)rows);
-  // rows of up to 3 * 256 * 8 = 6144 elements (every OPT up to 13B) keep 3 vectors per thread, wider ones 8
-  const bool narrow = width <= 3 * kLnThreads * 8;
-  hipStream_t s = (hipStream_t)stream;
-  if (dtype == APS_BF16) {
-    if (narrow) APS_LAUNCH((add_layer_norm_kernel<true, 3>), grid, dim3(kLnThreads), 0, s, g);
-    else APS_LAUNCH((add_layer_norm_kernel<true, kLnVecs>), grid, dim3(kLnThreads), 0, s, g);
-  } else {
-    if (narrow) APS_LAUNCH((add_layer_norm_kernel<false, 3>), grid, dim3(kLnThreads), 0, s, g);
-    else APS_LAUNCH((add_layer_norm_kernel<false, kLnVecs>), grid, dim3(kLnThreads), 0, s, g);
-  }
-  return launch_status();
+              (const char*)beta, x_stride * 2, residual_stride * 2, normed_stride * 2, sum_stride * 2, (int)width, eps,
+              nullptr, nullptr, 0, 1};
+  return launch_add_layer_norm<false>(g, rows, dtype, stream);
+}
+
+// The same of a product's parts (see PARTS); pointers and width as aps_add_layer_norm wants them, rows `width` apart.
+__attribute__((visibility("hidden"))) int aps_internal_parts_add_layer_norm(
+    void* normed, void* sum, const float* partial, int parts, const void* lin_bias, const void* residual, const void* gamma,
+    const void* beta, int64_t rows, int64_t width, int64_t residual_stride, float eps, int dtype, aps_stream_t stream) {
+  AddLnArgs g{(char*)normed, (char*)sum, nullptr, (const char*)residual, (const char*)gamma, (const char*)beta, 0,
+              residual_stride * 2, width * 2, width * 2, (int)width, eps, partial, (const char*)lin_bias, rows * width, parts};
+  return launch_add_layer_norm<true>(g, rows, dtype, stream);
 }

@@ -1095,6 +1095,12 @@ inline TailPlan plan_tail(int64_t tiles, int64_t nk) {
 
 using namespace aps;
 
+// (layer_ops.hip)
+int aps_internal_parts_add_layer_norm(void* normed, void* sum, const float* partial, int parts, const void* lin_bias,
+                                      const void* residual, const void* gamma, const void* beta, int64_t rows, int64_t width,
+                                      int64_t residual_stride, float eps, int dtype, aps_stream_t stream);
+static constexpr int64_t kLnMaxWidth = 16384;   // what a workgroup of the norm keeps in registers
+
 extern "C" {
 
 // Tile rows / 64 and K split of a product beyond the row-streaming kernels' range: the pair with the least time by
@@ -1170,6 +1176,10 @@ int64_t aps_linear_nt_workspace_bytes(int64_t m, int64_t n, int64_t k) {
   return bytes;
 }
 
+// A row's workgroup adds the parts of a product that its norm reads; with more of them the sum wants a launch of its own, whose
+// workgroups are not bound to rows (49 rows in 32 parts: 640 KB a row).
+constexpr int kMaxPartsLeft = 8;
+
 // Where the rows of a gathered A operand live (see GemmArgs::row_src).
 struct GatherSrc {
   const int64_t* row_src;
@@ -1180,7 +1190,9 @@ struct GatherSrc {
 static int launch_gemm(const void* x, const void* weight, const void* bias, const OutMap& om, int64_t m, int64_t n,
                        int64_t k, int64_t x_stride, int64_t w_stride, int dtype, void* workspace,
                        int64_t workspace_bytes, aps_stream_t stream, const GatherSrc* gs = nullptr,
-                       int32_t* tile_counters = nullptr) {
+                       int32_t* tile_counters = nullptr, int* parts_left = nullptr) {
+  // parts_left: a caller that adds the K parts itself, where there are at most kMaxPartsLeft of them; 1: the product is stored
+  if (parts_left) *parts_left = 1;
   if (dtype != APS_F16 && dtype != APS_BF16) return APS_ERR_UNSUPPORTED;
   if (n % BN != 0 || k % BK != 0) return APS_ERR_UNSUPPORTED;
   if (x_stride < k || w_stride < k) return APS_ERR_INVALID_ARG;
@@ -1216,10 +1228,12 @@ static int launch_gemm(const void* x, const void* weight, const void* bias, cons
     if (parts == 1 || (workspace && workspace_bytes >= (int64_t)parts * m * n * 4 && !(addr(workspace) & 15))) {
       g.rows_per_wg = wp.rows;
       g.partial = parts > 1 ? (float*)workspace : nullptr;
-      g.tile_counters = parts > 1 ? (int*)tile_counters : nullptr;   // (at most kNumCus tiles are split)
+      const bool left = parts_left && parts > 1 && parts <= kMaxPartsLeft;
+      g.tile_counters = parts > 1 && !left ? (int*)tile_counters : nullptr;   // (at most kNumCus tiles are split)
       int st = dtype == APS_BF16 ? launch_weight_stream<true>(g, parts, k_per_part, s)
                                  : launch_weight_stream<false>(g, parts, k_per_part, s);
-      if (st != APS_OK || parts == 1 || g.tile_counters) return st;
+      if (left) *parts_left = parts;
+      if (st != APS_OK || parts == 1 || g.tile_counters || left) return st;
       const int64_t quads = m * n / 4;
       const dim3 rgrid((unsigned)((quads + 255) / 256));
       if (dtype == APS_BF16)
@@ -1304,6 +1318,10 @@ static int launch_gemm(const void* x, const void* weight, const void* bias, cons
     return launch_status();
   }
   if (st != APS_OK || splits <= 1) return st;
+  if (parts_left && splits <= kMaxPartsLeft) {
+    *parts_left = splits;
+    return st;
+  }
   const int64_t quads = (m * n + 3) / 4;
   const dim3 rgrid((unsigned)((quads + 255) / 256));
   if (dtype == APS_BF16)
@@ -1393,6 +1411,30 @@ int aps_linear_nt(const void* x, const void* weight, const void* bias, void* out
   if (addr(tile_counters) & 3) return APS_ERR_INVALID_ARG;
   return launch_gemm(x, weight, bias, om, m, n, k, x_stride, w_stride, dtype, workspace, workspace_bytes, stream,
                      nullptr, tile_counters);
+}
+
+int aps_linear_add_layer_norm(void* normed, void* sum, void* product, const void* x, const void* weight, const void* bias,
+                              const void* residual, const void* gamma, const void* beta, int64_t m, int64_t n, int64_t k,
+                              int64_t x_stride, int64_t w_stride, int64_t residual_stride, float eps, int dtype,
+                              void* workspace, int64_t workspace_bytes, int32_t* tile_counters, aps_stream_t stream) {
+  if (m < 0 || n <= 0 || k <= 0 || !(eps >= 0.f)) return APS_ERR_INVALID_ARG;
+  if (m == 0) return APS_OK;
+  if (!normed || !sum || !product || !x || !weight || !residual || !gamma || residual_stride < n) return APS_ERR_INVALID_ARG;
+  if (n > kLnMaxWidth || m > 0x7fffffff ||
+      common_vec_bytes({addr(normed), addr(sum), addr(product), addr(residual), addr(gamma), addr(beta),
+                        (uint64_t)residual_stride * 2}) != 16)
+    return APS_ERR_UNSUPPORTED;
+  if (addr(tile_counters) & 3) return APS_ERR_INVALID_ARG;
+  OutMap om{};
+  om.base[0] = (char*)product; om.ld = n; om.limit0 = m; om.aligned16 = 1;
+  int parts = 1;
+  const int st = launch_gemm(x, weight, bias, om, m, n, k, x_stride, w_stride, dtype, workspace, workspace_bytes, stream,
+                             nullptr, tile_counters, (addr(bias) & 15) ? nullptr : &parts);   // (the norm reads it by vectors)
+  if (st != APS_OK) return st;
+  if (parts > 1)
+    return aps_internal_parts_add_layer_norm(normed, sum, (const float*)workspace, parts, bias, residual, gamma, beta, m, n,
+                                             residual_stride, eps, dtype, stream);
+  return aps_add_layer_norm(normed, sum, product, residual, gamma, beta, m, n, n, residual_stride, n, n, eps, dtype, stream);
 }
 
 int aps_kv_reproject_to_cache(const void* x, const void* w_kv, const void* b_kv, void* ws_k_cache, void* ws_v_cache,

@@ -562,6 +562,22 @@ int aps_linear_nt(const void* x, const void* weight, const void* bias,
                   int flags, void* workspace, int64_t workspace_bytes,
                   int32_t* tile_counters, aps_stream_t stream);
 
+/* product = x weight^T + bias, then sum = product + residual and normed =
+ * LayerNorm(sum) * gamma + beta: aps_linear_nt and aps_add_layer_norm with the
+ * same results, bit for bit, but without a launch of its own for the sum over K
+ * where the product is split.  ref: the out projection and fc2 with what follows
+ * them, model_executor/models/aptserve_opt.py:186-211.  normed, sum and product
+ * are [m, n], contiguous; product is scratch (written where K is not split).
+ * n <= 16384; bias and beta may be NULL; workspace and tile_counters as for
+ * aps_linear_nt. */
+int aps_linear_add_layer_norm(
+    void* normed, void* sum, void* product, const void* x, const void* weight,
+    const void* bias, const void* residual, const void* gamma,
+    const void* beta, int64_t m, int64_t n, int64_t k, int64_t x_stride,
+    int64_t w_stride, int64_t residual_stride, float eps, int dtype,
+    void* workspace, int64_t workspace_bytes, int32_t* tile_counters,
+    aps_stream_t stream);
+
 /* K/V re-projection with the cache write fused into the epilogue: one pass that
  * replaces the kv_only projection (model_executor/models/aptserve_opt.py:123-124),
  * the chunk into key/value, and ranges (A) and (C) of mixed_kv_to_cache

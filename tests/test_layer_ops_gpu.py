@@ -46,6 +46,31 @@ def test_add_layer_norm_strided_rows_and_errors(dev):
     assert ops.add_layer_norm(x[:0], r[:0], w, b)[0].shape == (0, 768)
 
 
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("m,n,k", [(1, 768, 768), (5, 5120, 20480), (12, 768, 3072), (48, 2560, 2048), (49, 768, 20480),
+                                   (65, 5120, 5120), (361, 5120, 5120), (130, 7168, 4096), (700, 1024, 4096)])
+def test_product_with_the_norm_behind_it_equals_the_two_calls(dev, m, n, k, dtype):
+    """Products of one part, of few (the norm adds them) and of more than the norm adds; the same bits as linear_nt, then
+    add_layer_norm.  With and without biases, and with a bias that no vector load takes."""
+    x, w = randn((m, k), 1, dtype).to(dev), (randn((n, k), 2, dtype) * 0.02).to(dev)
+    r, g = randn((m, 2 * n), 3, dtype).to(dev)[:, n:], (1 + 0.1 * randn((n,), 4)).to(dtype).to(dev)
+    odd = randn((n + 1,), 5, dtype).to(dev)
+    for bias, beta in ((odd[:n].clone(), odd[1:].clone()), (None, None), (odd[1:], None)):
+        normed, total = ops.linear_add_layer_norm(x, w, bias, r, g, beta)
+        ref_n, ref_t = ops.add_layer_norm(ops.linear_nt(x, w, bias), r, g, beta)
+        assert torch.equal(total.view(torch.int16), ref_t.view(torch.int16))
+        assert torch.equal(normed.view(torch.int16), ref_n.view(torch.int16))
+
+
+def test_product_with_the_norm_behind_it_errors(dev):
+    x, w = randn((3, 768), 1).to(dev), randn((768, 768), 2).to(dev)
+    r, g = randn((3, 768), 3).to(dev), randn((768,), 4).to(dev)
+    for bad in (dict(residual=r[:2]), dict(residual=r.float()), dict(ln_weight=None), dict(ln_weight=g[:5]), dict(x=x[:, :64])):
+        with pytest.raises(ValueError):
+            ops.linear_add_layer_norm(**{**dict(x=x, weight=w, bias=None, residual=r, ln_weight=g, ln_bias=None), **bad})
+    assert ops.linear_add_layer_norm(x[:0], w, None, r[:0], g, None)[0].shape == (0, 768)
+
+
 def test_decoder_with_fused_norms_equals_plain_ops(dev):
     """Two decoder layers with the (add, LayerNorm) pairs fused against the same model on plain element-wise ops:
     same kernels everywhere else, so the hidden states agree to the norms' last-bit differences."""
