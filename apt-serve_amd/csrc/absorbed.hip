@@ -13,7 +13,8 @@
 //                                                            seq_plan_kernel
 //   2. S[s][h][t]   = <qt[s][h], h_t>  (fp32)               hidden_scores_kernel: tiles of 128 cached rows through
 //                                                            the row-streaming MFMA core, K in parts for small
-//                                                            batches (score_parts_sum_kernel adds them)
+//                                                            batches (score_parts_sum_kernel adds them, or the chunk
+//                                                            kernel of step 3 as it reads them)
 //   3. ctx[s][h][:] = sum_t softmax_t(S[s][h])[t] h_t        hidden_wsum_kernel: one pass over the rows with the
 //                                                            online softmax inside (long sequences in partitions);
 //                                                            few cached rows in all: hidden_wsum_chunk_kernel, one
@@ -575,6 +576,7 @@ __device__ __forceinline__ float half_wave_max(float x) {
 
 struct WsumArgs {
   const float* s; int64_t s_batch_stride, s_row_stride;  // S[z][h][t], complete scores
+  int score_parts; int64_t s_part_stride;                 // the chunk kernel: parts of S over K, added there in order
   const char* cache; int64_t slot_stride_b, num_slots;
   const int64_t* row_ids; const int64_t* row_start;
   const char* zero_row;                                   // n zeros (what a token without a cached row reads)
@@ -898,6 +900,30 @@ __device__ __forceinline__ void hidden_wsum_chunk_body(const WsumArgs& g) {
       slot[st][i] = g.row_ids[rs + kbeg + (t < n_tok ? t : 0)];
       if (t >= n_tok) slot[st][i] = -1;
     }
+  // the other parts of the scores, nine in flight together: they arrive with the slots, which the rows wait for anyway
+  // (ten parts, 3 sequences of 640 rows: 15.5 us, and 12.4 behind a launch of 4.8 that added them)
+  constexpr int kPartsInFlight = 9;
+  for (int p0 = 1; p0 < g.score_parts; p0 += kPartsInFlight) {
+    const char* s_base = (const char*)(g.s + (int64_t)z * g.s_batch_stride);
+    const int ts = quad_ok ? kbeg + 4 * tq : 0;
+    float4v t[kPartsInFlight][NJ];
+#pragma unroll
+    for (int p = 0; p < kPartsInFlight; ++p)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int head = m0 + hl + kWsHeadsPerPass * j;
+        t[p][j] = *(const float4v*)(s_base + ((int64_t)min(p0 + p, g.score_parts - 1) * g.s_part_stride +
+                                              (int64_t)(head < g.heads ? head : 0) * g.s_row_stride + ts) * 4);
+      }
+#pragma unroll
+    for (int p = 0; p < kPartsInFlight; ++p)
+      if (p0 + p < g.score_parts) {
+#pragma unroll
+        for (int j = 0; j < NJ; ++j)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) sv[j][i] += t[p][j][i];
+      }
+  }
   u32x4 r[kWsRing][8];
 #pragma unroll
   for (int st = 0; st < kWsRing; ++st)
@@ -1027,17 +1053,37 @@ __global__ __launch_bounds__(256) void wsum_combine_kernel(const float* __restri
   const int64_t idx = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) * 4;
   if (idx >= per_part) return;
   const int64_t col = idx % n, zh = idx / n;
+  // eight partitions in flight together (one after the other, behind the test that skips one, 7.8 us of latencies for 7 chunks
+  // of 3 sequences; so 5.6); one past the end of its sequence holds anything and is left out by selection
+  constexpr int kAhead = 8;
+  typedef float float2w __attribute__((ext_vector_type(2)));
+  const float2w* const mls = (const float2w*)ml + zh;
+  const int64_t ml_stride = (int64_t)n_seqs * heads;
+  float2w w[kAhead];
+  float4v v[kAhead];
+  auto fetch = [&](int p0) {
+#pragma unroll
+    for (int p = 0; p < kAhead; ++p) w[p] = mls[min(p0 + p, parts - 1) * ml_stride];
+#pragma unroll
+    for (int p = 0; p < kAhead; ++p) v[p] = *(const float4v*)(partial + (int64_t)min(p0 + p, parts - 1) * per_part + idx);
+  };
+  fetch(0);
   float mx = -INFINITY;
-  for (int p = 0; p < parts; ++p) mx = fmaxf(mx, ml[((int64_t)p * n_seqs * heads + zh) * 2]);
+#pragma unroll
+  for (int p = 0; p < kAhead; ++p) mx = fmaxf(mx, w[p][0]);   // (past the last: the last again)
+  for (int p = kAhead; p < parts; ++p) mx = fmaxf(mx, mls[p * ml_stride][0]);
   float4v num = {0.f, 0.f, 0.f, 0.f};
   float den = 0.f;
-  for (int p = 0; p < parts; ++p) {
-    const float mp = ml[((int64_t)p * n_seqs * heads + zh) * 2], lp = ml[((int64_t)p * n_seqs * heads + zh) * 2 + 1];
-    if (mp == -INFINITY) continue;  // a partition past the end of its sequence
-    const float w = exp2f(mp - mx);
-    const float4v v = *(const float4v*)(partial + p * per_part + idx);
-    num[0] += v[0] * w; num[1] += v[1] * w; num[2] += v[2] * w; num[3] += v[3] * w;
-    den += lp * w;
+  for (int p0 = 0; p0 < parts; p0 += kAhead) {
+    if (p0 > 0) fetch(p0);
+#pragma unroll
+    for (int p = 0; p < kAhead; ++p) {
+      const bool on = p0 + p < parts && w[p][0] != -INFINITY;
+      const float e = exp2f(w[p][0] - mx);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) num[i] = on ? num[i] + v[p][i] * e : num[i];
+      den = on ? den + w[p][1] * e : den;
+    }
   }
   const float inv = den > 0.f ? 1.f / den : 0.f;
   const int64_t h = zh % heads, z = zh / heads;
@@ -1310,7 +1356,7 @@ static int hybrid_attention_impl(const StoreJob* store_job, const PagedJob* kv_j
     const int st = launch_status();
     if (st != APS_OK) return st;
   }
-  if (p.score_parts > 1) {
+  if (p.score_parts > 1 && !p.chunked) {   // (the chunk kernel adds them)
     const int64_t n = n_seqs * num_heads * p.lp;   // a multiple of 32
     APS_LAUNCH(score_parts_sum_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s, sc, n, p.score_parts,
                s_part_stride);
@@ -1321,6 +1367,7 @@ static int hybrid_attention_impl(const StoreJob* store_job, const PagedJob* kv_j
   {
     WsumArgs g{};
     g.s = sc; g.s_batch_stride = (int64_t)num_heads * p.lp; g.s_row_stride = p.lp;
+    g.score_parts = p.score_parts; g.s_part_stride = s_part_stride;
     g.cache = (const char*)paged_cache; g.slot_stride_b = slot_stride * 2; g.num_slots = num_slots;
     g.row_ids = hidden_slots; g.row_start = seq_start;
     g.zero_row = ws + p.off_zero;
