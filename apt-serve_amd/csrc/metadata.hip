@@ -82,7 +82,7 @@ __device__ __forceinline__ int64_t slot_of(const int32_t* table, int width, int 
 // Decode step: a hidden-cached sequence contributes seq_len rows, a K/V-cached one a single row.  The rows of a sequence are
 // dealt over the grid's y, 256 at a time; everything of which a sequence has one is written by its workgroup y = 0.  What
 // bounds it is latency: lengths, table entry and stores one after the other (256 sequences, 173500 tokens: 15.2 us with one
-// workgroup a sequence, 7.2 with four).
+// workgroup a sequence, 9.4 with four).
 __global__ __launch_bounds__(kThreads) void decode_metadata_kernel(const MetaArgs a) {
   const int b = blockIdx.x;
   if (blockIdx.y != 0 && (a.use_hidden[b] == 0 || a.seq_lens[b] <= (int)blockIdx.y * kThreads)) return;
