@@ -216,6 +216,33 @@ def test_prefix_attention_parts_only_where_workgroups_are_few():
     assert need(0, 0, 0, 0, 40, 128) == 0 and need(1, 64, 64, 0, 40, 128) == 0 and need(1, 64, 64, 8064, 40, 96) == 0
 
 
+def test_prefix_attention_takes_no_length_off_the_device(dev):
+    """``max_seqlen_k`` on the GPU is not read, so such a call neither synchronises nor breaks a capture; without a length of
+    the host's, parts are not sized by the width of the tables: the bits of one part."""
+    from test_oracle_attention import build_paged
+    from aptserve_hip.ops import _stated_keys
+    assert _stated_keys(None, 2048) == _stated_keys(torch.tensor(1538), 2048) == 0
+    assert _stated_keys(1538, 2048) == _stated_keys(np.int32(1538), 2048) == 1538 and _stated_keys(5000, 2048) == 2048
+    H, D, klens, qlens = 2, 128, [1538, 64], [70, 3]
+    kc, vc, bt, _, _ = (x.to(dev) if isinstance(x, torch.Tensor) else x for x in build_paged(2, H, D, 16, klens, 3))
+    q = randn((sum(qlens), H, D), 4).to(dev)
+    cu_q, cu_k = (torch.tensor([0] + list(np.cumsum(n)), dtype=torch.int32, device=dev) for n in (qlens, klens))
+    on_device = torch.tensor(1538, device=dev)
+
+    def call(max_k):
+        return ops.flash_attn_varlen_func(q, kc, vc, cu_seqlens_q=cu_q, cu_seqlens_k=cu_k, max_seqlen_q=70, max_seqlen_k=max_k,
+                                          block_table=bt)
+    one, parts = call(0), call(1538)
+    assert not torch.equal(one, parts)
+    torch.cuda.set_sync_debug_mode("error")
+    try:
+        outs = [call(on_device), call(None)]
+    finally:
+        torch.cuda.set_sync_debug_mode("default")
+    for out in outs:
+        assert torch.equal(out, one)
+
+
 def test_prefix_attention_block_size_32_and_argument_errors(dev):
     run_prefix(dev, [100, 45], [33, 45], 4, 64, BS=32, seed=3)
     from test_oracle_attention import build_paged
