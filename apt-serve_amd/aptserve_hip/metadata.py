@@ -260,10 +260,11 @@ def _pack_tables(tables, lens: np.ndarray, out: np.ndarray, rows: Optional[np.nd
 
 
 def _packed_rows(tables, batch: int) -> bool:
-    """Whether ``tables`` is a packed int32 array whose rows native code can walk (contiguous entries, rows in order)."""
+    """Whether ``tables`` is a packed int32 array whose rows native code can walk (contiguous entries, rows in order).  One
+    without columns, the shared table of a batch without hidden-cached sequences, has no rows to walk."""
     return (type(tables) is np.ndarray and tables.ndim == 2 and tables.shape[0] == batch and tables.dtype == np.int32
-            and tables.shape[1] > 0 and tables.strides[1] == 4 and tables.strides[0] % 4 == 0
-            and tables.strides[0] >= 4 * tables.shape[1])
+            and (tables.shape[1] == 0 or tables.strides[1] == 4 and tables.strides[0] % 4 == 0
+                 and tables.strides[0] >= 4 * tables.shape[1]))
 
 
 def _build_decode_packed(lens: np.ndarray, hid: np.ndarray, tables: np.ndarray, shared: np.ndarray, block_size: int,

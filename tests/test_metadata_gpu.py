@@ -67,15 +67,16 @@ def test_packed_tables_give_the_same_metadata_as_lists(dev, frac, prompt):
 
 @pytest.mark.parametrize("frac", [0.0, 0.4, 1.0])
 @pytest.mark.parametrize("n,bs", [(1, 16), (11, 16), (257, 32)])
-def test_native_packing_equals_the_general_path(dev, frac, n, bs):
+def test_native_packing_equals_the_general_path(dev, monkeypatch, frac, n, bs):
     """Packed int32 tables are packed, uploaded and expanded by one native call: every field, tensors and numbers alike,
     equals what the general path makes of the same batch (lists; int64, transposed and reversed arrays take it too), for
-    close rows, row slices, wider rows and lengths and flags that are strided."""
+    close rows, row slices, wider rows and lengths and flags that are strided; without hidden-cached sequences with the
+    shared table that packed_tables() makes, which has no columns, and with one that has some."""
     import dataclasses
     batch = workloads.small_decode_batch(7, n, 300, frac, 400 * (n // 11 + 1), bs)
     bt, bts = batch.packed_tables()
-    if bts.shape[1] == 0:
-        bts = np.zeros((n, 1), dtype=np.int32)
+    none_hidden = not any(batch.use_hidden)
+    assert (bts.shape[1] == 0) == none_hidden
     lens, hid = np.asarray(batch.seq_lens), np.asarray(batch.use_hidden, dtype=bool)
     general = metadata.build_from_batch(batch, dev)
     wide = lambda a: np.concatenate([a, np.full((n, 5), 99, dtype=a.dtype)], axis=1)
@@ -84,9 +85,17 @@ def test_native_packing_equals_the_general_path(dev, frac, n, bs):
              (np.repeat(bt, 2, 0)[::2], bts, np.repeat(lens, 2)[::2], np.repeat(hid, 2)[::2]),
              (bt.astype(np.int64), bts, lens, hid), (np.asfortranarray(bt), np.asfortranarray(bts), lens, hid),
              (reverse(bt), reverse(bts), reverse(lens), reverse(hid))]
-    native = [metadata._packed_rows(f[0], n) and metadata._packed_rows(f[1], n) for f in forms]
-    assert native[:4] == [True, True, True, False] and (n == 1 or native[5] is False)
+    if none_hidden:
+        forms.append((bt, np.zeros((n, 1), dtype=np.int32), lens, hid))
+    native, build = [], metadata._build_decode_packed
+
+    def recorded(*args):
+        md = build(*args)
+        native[-1] = md is not None
+        return md
+    monkeypatch.setattr(metadata, "_build_decode_packed", recorded)
     for f in forms:
+        native.append(False)
         md = metadata.build_metadata(False, f[2], f[3], f[0], f[1], bs, dev, check_totals=True)
         for field in dataclasses.fields(md):
             a, b = getattr(md, field.name), getattr(general, field.name)
@@ -94,6 +103,7 @@ def test_native_packing_equals_the_general_path(dev, frac, n, bs):
                 assert a.dtype == b.dtype and a.shape == b.shape and torch.equal(a, b), field.name
             else:
                 assert a == b and type(a) is type(b), field.name
+    assert native[:4] == [True, True, True, False] and (n == 1 or native[5] is False) and native[6:] == [True] * none_hidden
 
 
 def test_native_packing_checks_its_sizes():
