@@ -111,7 +111,9 @@ def test_absorbed_attention_equals_reprojection_flow(dev):
 @pytest.mark.parametrize("H,D,lens,N", [(40, 128, [2048, 130], 320),        # 16 softmax chunks, OPT-13B rows
                                         (12, 64, [700, 1, 129, 384, 33], 256),
                                         (4, 64, [5000, 300], 720),           # token partitions (beyond 4096 tokens)
-                                        (8, 128, [1500] * 3 + [64] * 30, 512)])
+                                        (8, 128, [1500] * 3 + [64] * 30, 512),
+                                        # 11 partitions of 192 tokens: of a sequence 1, 2, 8, 9 and 11 of them, to their edges
+                                        (12, 64, [2000, 192, 193, 1, 1536, 1537, 384, 385], 512)])
 def test_absorbed_attention_long_sequences(dev, H, D, lens, N):
     """Sequences of many 128-token softmax chunks: the weighted sum keeps a running maximum per head and rescales
     its sums when it moves; with `ramp` the later rows carry the larger scores, so it moves in every chunk."""
