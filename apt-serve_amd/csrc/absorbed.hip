@@ -13,8 +13,8 @@
 //                                                            seq_plan_kernel
 //   2. S[s][h][t]   = <qt[s][h], h_t>  (fp32)               hidden_scores_kernel: tiles of 128 cached rows through
 //                                                            the row-streaming MFMA core, K in parts for small
-//                                                            batches (score_parts_sum_kernel adds them, or the chunk
-//                                                            kernel of step 3 as it reads them)
+//                                                            batches (score_parts_sum_kernel adds them, or, up to ten,
+//                                                            the chunk kernel of step 3 as it reads them)
 //   3. ctx[s][h][:] = sum_t softmax_t(S[s][h])[t] h_t        hidden_wsum_kernel: one pass over the rows with the
 //                                                            online softmax inside (long sequences in partitions);
 //                                                            few cached rows in all: hidden_wsum_chunk_kernel, one
@@ -574,9 +574,14 @@ __device__ __forceinline__ float half_wave_max(float x) {
   return fmaxf(y, __shfl_xor(y, 16));
 }
 
+// Score parts that the chunk kernel adds itself: as many as its registers hold in flight together beside the slots.  A second
+// round of loads costs more than the launch that adds them all (hidden size 7168, 2 sequences, 300 rows, 14 parts: the layer 118.3
+// us with two rounds, 115.8 with the launch; 5120, 3 sequences, 1160 rows, 10 parts 86.8 and 90.9 us).
+constexpr int kWsScoreParts = 10;
+
 struct WsumArgs {
-  const float* s; int64_t s_batch_stride, s_row_stride;  // S[z][h][t], complete scores
-  int score_parts; int64_t s_part_stride;                 // the chunk kernel: parts of S over K, added there in order
+  const float* s; int64_t s_batch_stride, s_row_stride;  // S[z][h][t], complete scores or (chunk kernel) the first of their parts
+  int score_parts; int64_t s_part_stride;                 // the chunk kernel: parts of S over K, added there in order (<= kWsScoreParts)
   const char* cache; int64_t slot_stride_b, num_slots;
   const int64_t* row_ids; const int64_t* row_start;
   const char* zero_row;                                   // n zeros (what a token without a cached row reads)
@@ -900,28 +905,29 @@ __device__ __forceinline__ void hidden_wsum_chunk_body(const WsumArgs& g) {
       slot[st][i] = g.row_ids[rs + kbeg + (t < n_tok ? t : 0)];
       if (t >= n_tok) slot[st][i] = -1;
     }
-  // the other parts of the scores, nine in flight together: they arrive with the slots, which the rows wait for anyway
+  // the other parts of the scores, all in flight together: they arrive with the slots, which the rows wait for anyway
   // (ten parts, 3 sequences of 640 rows: 15.5 us, and 12.4 behind a launch of 4.8 that added them)
-  constexpr int kPartsInFlight = 9;
-  for (int p0 = 1; p0 < g.score_parts; p0 += kPartsInFlight) {
+  if (g.score_parts > 1) {
     const char* s_base = (const char*)(g.s + (int64_t)z * g.s_batch_stride);
     const int ts = quad_ok ? kbeg + 4 * tq : 0;
-    float4v t[kPartsInFlight][NJ];
+    float4v t[kWsScoreParts - 1][NJ];
 #pragma unroll
-    for (int p = 0; p < kPartsInFlight; ++p)
+    for (int p = 1; p < kWsScoreParts; ++p)
+      if (p < g.score_parts) {
 #pragma unroll
-      for (int j = 0; j < NJ; ++j) {
-        const int head = m0 + hl + kWsHeadsPerPass * j;
-        t[p][j] = *(const float4v*)(s_base + ((int64_t)min(p0 + p, g.score_parts - 1) * g.s_part_stride +
-                                              (int64_t)(head < g.heads ? head : 0) * g.s_row_stride + ts) * 4);
+        for (int j = 0; j < NJ; ++j) {
+          const int head = m0 + hl + kWsHeadsPerPass * j;
+          t[p - 1][j] = *(const float4v*)(s_base + ((int64_t)p * g.s_part_stride +
+                                                    (int64_t)(head < g.heads ? head : 0) * g.s_row_stride + ts) * 4);
+        }
       }
 #pragma unroll
-    for (int p = 0; p < kPartsInFlight; ++p)
-      if (p0 + p < g.score_parts) {
+    for (int p = 1; p < kWsScoreParts; ++p)
+      if (p < g.score_parts) {
 #pragma unroll
         for (int j = 0; j < NJ; ++j)
 #pragma unroll
-          for (int i = 0; i < 4; ++i) sv[j][i] += t[p][j][i];
+          for (int i = 0; i < 4; ++i) sv[j][i] += t[p - 1][j][i];
       }
   }
   u32x4 r[kWsRing][8];
@@ -1120,7 +1126,7 @@ inline int64_t align_up(int64_t v, int64_t a) { return (v + a - 1) / a * a; }
 struct Plan {
   int64_t lp;        // padded row length of S
   int kparts;        // token partitions of the weighted sum
-  int score_parts;   // parts of K in the scores kernel (partial scores, made whole by score_parts_sum_kernel)
+  int score_parts;   // parts of K in the scores kernel (partial scores, made whole by score_parts_sum_kernel or the chunk kernel)
   int64_t score_k_per_part;
   int k_per_part;
   bool chunked;      // few cached rows: one chunk of tokens per workgroup of the weighted sum
@@ -1366,7 +1372,8 @@ static int hybrid_attention_impl(const StoreJob* store_job, const PagedJob* kv_j
     const int st = launch_status();
     if (st != APS_OK) return st;
   }
-  if (p.score_parts > 1 && !p.chunked) {   // (the chunk kernel adds them)
+  const bool summed = p.score_parts > 1 && (!p.chunked || p.score_parts > kWsScoreParts);   // (else the chunk kernel adds them)
+  if (summed) {
     const int64_t n = n_seqs * num_heads * p.lp;   // a multiple of 32
     APS_LAUNCH(score_parts_sum_kernel, dim3((unsigned)((n / 4 + 255) / 256)), dim3(256), 0, s, sc, n, p.score_parts,
                s_part_stride);
@@ -1377,7 +1384,7 @@ static int hybrid_attention_impl(const StoreJob* store_job, const PagedJob* kv_j
   {
     WsumArgs g{};
     g.s = sc; g.s_batch_stride = (int64_t)num_heads * p.lp; g.s_row_stride = p.lp;
-    g.score_parts = p.score_parts; g.s_part_stride = s_part_stride;
+    g.score_parts = summed ? 1 : p.score_parts; g.s_part_stride = s_part_stride;
     g.cache = (const char*)paged_cache; g.slot_stride_b = slot_stride * 2; g.num_slots = num_slots;
     g.row_ids = hidden_slots; g.row_start = seq_start;
     g.zero_row = ws + p.off_zero;

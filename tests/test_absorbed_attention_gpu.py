@@ -132,6 +132,8 @@ def test_absorbed_attention_partitions_agree_with_one_pass(dev):
                                         (40, 128, [310, 200, 130], 64),           # a serving step's handful
                                         (12, 64, [192, 193, 3, 289, 96, 40, 7, 100], 128),
                                         (4, 64, [700, 20], 64),                   # 8 chunks of one sequence, 1 of the other
+                                        # 14 and 18 parts of the scores over K, more than the kernel adds itself; two head groups
+                                        (56, 128, [200, 96], 32), (72, 128, [97], 16),
                                         (12, 64, [90], 16), (12, 64, [97, 97, 97, 97, 97, 97, 97, 97, 97, 97, 97], 128)])
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 def test_absorbed_attention_of_few_cached_rows_one_chunk_per_workgroup(dev, H, D, lens, N, dtype):
