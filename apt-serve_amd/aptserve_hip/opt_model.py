@@ -137,6 +137,12 @@ class HybridOPTDecoderLayer:
         final one)."""
         w, p = self.w, self.p
         a = self.self_attn
+        if type(a).__call__ is not HybridOPTAttention.forward or getattr(self._mlp, "__func__", None) is not _OWN_MLP:
+            # something else in place of the attention or of the MLP is called as a whole: its last product is its own
+            normed, residual = ops.add_layer_norm(a(normed, kv_cache, shared_cache, md), residual, w[p + "final_ln_w"],
+                                                  w[p + "final_ln_b"])
+            normed, residual = ops.add_layer_norm(self._mlp(normed), residual, next_ln_w, next_ln_b)
+            return residual, normed
         attn = a.attend(normed, kv_cache, shared_cache, md)
         with phase("projections"):
             normed, residual = ops.linear_add_layer_norm(attn, a.out_weight, a.out_bias, residual, w[p + "final_ln_w"],
@@ -146,6 +152,9 @@ class HybridOPTDecoderLayer:
         return residual, normed
 
     __call__ = forward
+
+
+_OWN_MLP = HybridOPTDecoderLayer._mlp
 
 
 class HybridOPTModel:

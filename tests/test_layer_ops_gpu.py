@@ -90,3 +90,52 @@ def test_decoder_with_fused_norms_equals_plain_ops(dev):
         model = opt_model.HybridOPTModel(cfg, w, fused_norm=fused)
         outs.append(model(ids, md.input_positions, kv, shared, md).float())
     assert (outs[0] - outs[1]).abs().max().item() < 2e-2
+
+
+@pytest.mark.parametrize("place", ["attention", "attention of a subclass", "mlp of a layer", "mlp of a subclass"])
+def test_decoder_with_fused_norms_calls_what_stands_in_for_its_parts(dev, monkeypatch, place):
+    """An object that can only be called in place of a layer's attention, or another MLP, is called in every layer; one that
+    calls what it replaces gives the same bits."""
+    from aptserve_hip import backend, metadata, opt_model, workloads
+    cfg = opt_model.OPTConfig(hidden_size=768, num_attention_heads=12, num_hidden_layers=2, ffn_dim=1024,
+                              vocab_size=500, max_position_embeddings=2048)
+    w = opt_model.random_weights(cfg, 0, dev)
+    N, BS = 96, 16
+    batch = workloads.small_decode_batch(5, 9, 100, 0.5, N)
+    md = metadata.build_from_batch(batch, dev)
+    ids = torch.arange(len(batch.seq_lens), device=dev) % 500
+    calls, outs = [], []
+
+    def counted(f):
+        return lambda *args: calls.append(1) or f(*args)
+
+    class Callable:
+        def __init__(self, f):
+            self.f = counted(f)
+
+        def __call__(self, *args):
+            return self.f(*args)
+
+    class Attention(backend.HybridOPTAttention):
+        def __call__(self, *args):
+            return counted(self.forward)(*args)
+
+    class Layer(opt_model.HybridOPTDecoderLayer):
+        def _mlp(self, x):
+            return counted(super()._mlp)(x)
+    for replaced in (False, True):
+        kv, shared = backend.allocate_caches(2, N, BS, 12, 64, torch.float16, dev)
+        for c in kv:
+            c.copy_(randn(tuple(c.shape), 9).to(dev))
+        model = opt_model.HybridOPTModel(cfg, w)
+        for layer in model.layers if replaced else ():
+            if place == "attention":
+                layer.self_attn = Callable(layer.self_attn)
+            elif place == "attention of a subclass":
+                layer.self_attn.__class__ = Attention
+            elif place == "mlp of a layer":
+                monkeypatch.setattr(layer, "_mlp", counted(layer._mlp))
+            else:
+                layer.__class__ = Layer
+        outs.append(model(ids, md.input_positions, kv, shared, md))
+    assert len(calls) == 2 and torch.equal(outs[0], outs[1])
