@@ -495,7 +495,8 @@ def step_replay_figures(torch, dev, seed, seq_lens=(310, 120, 200, 260, 130), us
             "replays": reps, "ms_per_step": ms,
             "eager_phase_us_per_layer": {k_: v_ * 1e3 / L for k_, v_ in per.items()},
             "note": "attention_on_hidden_rows = the one call for both kinds of sequence (stores, K/V attention, "
-                    "attention on hidden rows with its value projection); projections = qkv, out, fc1, fc2"}
+                    "attention on hidden rows with its value projection); projections = qkv, out, fc1, fc2, with the "
+                    "residual adds and layer norms behind out and fc2"}
 
 
 def step_loop_figures(torch, dev, seed, warm_steps=240, timed_steps=320, profile_steps=12, absorbed=False,
@@ -567,8 +568,9 @@ def step_loop_figures(torch, dev, seed, warm_steps=240, timed_steps=320, profile
         model_ms = host["model_ms"] / n_prof
         split = {"steps_profiled": n_prof, "metadata_ms": host["metadata_ms"] / n_prof, "model_ms": model_ms,
                  "gpu_ms": per, "rest_ms": model_ms - sum(per.values()),
-                 "note": "projections = q / out / MLP products (weight streaming); rest = layer norms, residual "
-                         "adds, embedding, logits, launch gaps"}
+                 "note": "projections = q / out / MLP products (weight streaming) and the residual adds and layer norms "
+                         "behind out and fc2, which the same calls take (projections_hbm: the weights' bytes over this "
+                         "whole time); rest = the first layer norm, embedding, logits, launch gaps"}
         frac = {}
         if per.get("gather"):
             frac["gather_hbm"] = work["gather_bytes"] / n_prof / per["gather"] / 1e6 / HBM_PEAK_GBS
