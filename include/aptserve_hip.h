@@ -564,12 +564,14 @@ int aps_linear_nt(const void* x, const void* weight, const void* bias,
 
 /* product = x weight^T + bias, then sum = product + residual and normed =
  * LayerNorm(sum) * gamma + beta: aps_linear_nt and aps_add_layer_norm with the
- * same results, bit for bit, but without a launch of its own for the sum over K
- * where the product is split.  ref: the out projection and fc2 with what follows
- * them, model_executor/models/aptserve_opt.py:186-211.  normed, sum and product
- * are [m, n], contiguous; product is scratch (written where K is not split).
- * n <= 16384; bias and beta may be NULL; workspace and tile_counters as for
- * aps_linear_nt. */
+ * same results, bit for bit.  A product split along K into at most 8 parts leaves
+ * them to the norm's launch (if bias is 16-byte aligned or NULL), instead of a sum
+ * of its own; every other product is stored first, as aps_linear_nt stores it, and
+ * read by the norm.  ref: the out projection and fc2 with what follows them,
+ * model_executor/models/aptserve_opt.py:186-211.  normed, sum and product are
+ * [m, n], contiguous; product is scratch that any call may write: it must not
+ * overlap the other operands.  n <= 16384; bias and beta may be NULL; workspace
+ * and tile_counters as for aps_linear_nt. */
 int aps_linear_add_layer_norm(
     void* normed, void* sum, void* product, const void* x, const void* weight,
     const void* bias, const void* residual, const void* gamma,

@@ -62,6 +62,30 @@ def test_product_with_the_norm_behind_it_equals_the_two_calls(dev, m, n, k, dtyp
         assert torch.equal(normed.view(torch.int16), ref_n.view(torch.int16))
 
 
+@pytest.mark.parametrize("m,n,k,parts_left", [(1, 768, 768, False), (5, 5120, 20480, True), (12, 768, 3072, True),
+                                              (48, 2560, 2560, True), (361, 5120, 5120, True), (130, 7168, 4096, True),
+                                              (49, 768, 20480, False), (48, 2560, 10240, False), (4096, 768, 768, False)])
+def test_which_products_leave_their_parts_to_the_norm(dev, m, n, k, parts_left):
+    """A product whose parts the norm adds is never stored: its scratch keeps what was in it.  One of one part, of more than
+    eight, or with a bias that no vector load takes is stored."""
+    from aptserve_hip import _lib
+    lib = _lib.load()
+    x, w, r, g = randn((m, k), 1).to(dev), (randn((n, k), 2) * 0.02).to(dev), randn((m, n), 3).to(dev), randn((n,), 4).to(dev)
+    odd = randn((n + 1,), 5).to(dev)
+    need = lib.aps_linear_nt_workspace_bytes(m, n, k)
+    ws = torch.empty(max(need, 16), dtype=torch.uint8, device=dev)
+    for bias in (None, odd[:n], odd[1:]):
+        normed, total, product = (torch.full((m, n), float("nan"), dtype=torch.float16, device=dev) for _ in range(3))
+        st = lib.aps_linear_add_layer_norm(
+            normed.data_ptr(), total.data_ptr(), product.data_ptr(), x.data_ptr(), w.data_ptr(),
+            None if bias is None else bias.data_ptr(), r.data_ptr(), g.data_ptr(), None, m, n, k, k, k, n, 1e-5, 0,
+            ws.data_ptr(), need, ops._tile_counters(dev).data_ptr(), torch.cuda.current_stream(dev).cuda_stream)
+        assert st == 0 and not normed.isnan().any() and not total.isnan().any()
+        stored = not product.isnan().any().item()
+        assert stored or product.isnan().all()
+        assert stored == (not parts_left or bias is not None and bias.data_ptr() % 16 != 0)
+
+
 def test_product_with_the_norm_behind_it_errors(dev):
     x, w = randn((3, 768), 1).to(dev), randn((768, 768), 2).to(dev)
     r, g = randn((3, 768), 3).to(dev), randn((768,), 4).to(dev)
