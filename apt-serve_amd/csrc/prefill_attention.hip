@@ -58,11 +58,12 @@ __device__ __forceinline__ int tiles_per_part(int n, int parts, int part_tiles) 
   const int p = min(parts, (n + part_tiles - 1) / part_tiles);
   return (n + p - 1) / p;
 }
+constexpr int kPartQueries = 64;   // queries per workgroup of a step in parts
 template <int D>
-__host__ __device__ constexpr int64_t unit_floats(int qt) { return 64 * qt * (D + 2); }
+__host__ __device__ constexpr int64_t unit_floats() { return kPartQueries * (D + 2); }
 // Units of a query tile: tiles before it are counted as if each sequence began a new one behind the tokens in front of it
-__device__ __forceinline__ int64_t first_unit(int s0, int seq, int q_tile, int bq, int heads, int head, int parts) {
-  return ((int64_t)(s0 / bq + seq + q_tile) * heads + head) * parts;
+__device__ __forceinline__ int64_t first_unit(int s0, int seq, int q_tile, int heads, int head, int parts) {
+  return ((int64_t)(s0 / kPartQueries + seq + q_tile) * heads + head) * parts;
 }
 
 // Two stages of a K and a V tile
@@ -355,7 +356,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 
   // ---- one of several key parts: sums as they are
   if (PARTS && several) {
-    float* const unit = a.partial + (first_unit(s0, seq, q_tile, BQ, a.num_heads, head, a.parts) + part) * unit_floats<D>(QT);
+    static_assert(!PARTS || BQ == kPartQueries, "units are laid out for one query tile a wavefront");
+    float* const unit = a.partial + (first_unit(s0, seq, q_tile, a.num_heads, head, a.parts) + part) * unit_floats<D>();
     float* const ml = unit + BQ * D + wave * (16 * QT) + qcol;
 #pragma unroll
     for (int u = 0; u < QT; ++u) {
@@ -390,9 +392,9 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))
 // out = sum of the key parts of a query tile, each weighted with exp2 of its maximum against the largest, over the sum of
 // their weights: the same sums in fp32, rounded once.  Same grid (without the parts) and same lanes as the kernel above, so
 // that units are written and read 1 KiB a wavefront.
-template <bool BF16, int D, int QT>
+template <bool BF16, int D>
 __global__ __launch_bounds__(kThreads) void prefill_combine_kernel(const PrefillArgs a) {
-  constexpr int BQ = 64 * QT, DT = D / 16;
+  constexpr int BQ = kPartQueries, DT = D / 16;
   const int seq = blockIdx.y, head = blockIdx.x, q_tile = blockIdx.z, q0 = q_tile * BQ;
   const int s0 = a.cu_seqlens[seq], s1 = a.cu_seqlens[seq + 1];
   if (s0 < 0 || s1 < s0 || s1 > a.num_tokens) return;
@@ -403,38 +405,35 @@ __global__ __launch_bounds__(kThreads) void prefill_combine_kernel(const Prefill
   const int per_part = tiles_per_part(n_tiles, a.parts, a.part_tiles), parts = (n_tiles + per_part - 1) / per_part;
   if (parts == 1) return;   // stored by its workgroup
   const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, qcol = lane & 15, quad = lane >> 4;
-  const float* const units = a.partial + first_unit(s0, seq, q_tile, BQ, a.num_heads, head, a.parts) * unit_floats<D>(QT);
+  const float* const units = a.partial + first_unit(s0, seq, q_tile, a.num_heads, head, a.parts) * unit_floats<D>();
+  const int row = wave * 16 + qcol;
+  float m = -INFINITY;
+  for (int p = 0; p < parts; ++p) m = fmaxf(m, units[p * unit_floats<D>() + BQ * D + row]);
+  const float m_use = m == -INFINITY ? 0.f : m;
+  float4v o[DT];
 #pragma unroll
-  for (int u = 0; u < QT; ++u) {
-    const int row = wave * (16 * QT) + 16 * u + qcol;
-    float m = -INFINITY;
-    for (int p = 0; p < parts; ++p) m = fmaxf(m, units[p * unit_floats<D>(QT) + BQ * D + row]);
-    const float m_use = m == -INFINITY ? 0.f : m;
-    float4v o[DT];
-#pragma unroll
-    for (int t = 0; t < DT; ++t) o[t] = float4v{0.f, 0.f, 0.f, 0.f};
-    float l = 0.f;
-    for (int p = 0; p < parts; ++p) {
-      const float* const unit = units + p * unit_floats<D>(QT);
-      const float w = __builtin_amdgcn_exp2f((unit[BQ * D + row] - m_use) * a.scale_log2);
-      l += w * unit[BQ * D + BQ + row];
-#pragma unroll
-      for (int t = 0; t < DT; ++t) {
-        const float4v v = ((const float4v*)unit)[(u * DT + t) * kThreads + tid];
-#pragma unroll
-        for (int e = 0; e < 4; ++e) o[t][e] = fmaf(w, v[e], o[t][e]);
-      }
-    }
-    if (q0 + row >= qlen) continue;
-    const float inv = l > 0.f ? 1.f / l : 0.f;
-    char* op = a.out + (int64_t)(s0 + q0 + row) * a.out_stride_b + (int64_t)head * D * 2 + quad * 8;
+  for (int t = 0; t < DT; ++t) o[t] = float4v{0.f, 0.f, 0.f, 0.f};
+  float l = 0.f;
+  for (int p = 0; p < parts; ++p) {
+    const float* const unit = units + p * unit_floats<D>();
+    const float w = __builtin_amdgcn_exp2f((unit[BQ * D + row] - m_use) * a.scale_log2);
+    l += w * unit[BQ * D + BQ + row];
 #pragma unroll
     for (int t = 0; t < DT; ++t) {
-      uint2 w;
-      w.x = pack2<BF16>(o[t][0] * inv, o[t][1] * inv);
-      w.y = pack2<BF16>(o[t][2] * inv, o[t][3] * inv);
-      *(uint2*)(op + t * 32) = w;
+      const float4v v = ((const float4v*)unit)[t * kThreads + tid];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[t][e] = fmaf(w, v[e], o[t][e]);
     }
+  }
+  if (q0 + row >= qlen) return;
+  const float inv = l > 0.f ? 1.f / l : 0.f;
+  char* op = a.out + (int64_t)(s0 + q0 + row) * a.out_stride_b + (int64_t)head * D * 2 + quad * 8;
+#pragma unroll
+  for (int t = 0; t < DT; ++t) {
+    uint2 w;
+    w.x = pack2<BF16>(o[t][0] * inv, o[t][1] * inv);
+    w.y = pack2<BF16>(o[t][2] * inv, o[t][3] * inv);
+    *(uint2*)(op + t * 32) = w;
   }
 }
 
@@ -454,25 +453,38 @@ int query_tiles(int64_t num_seqs, int64_t num_tokens, int64_t max_seqlen_q, int 
   return num_heads * (num_tokens / 128 + num_seqs) <= 384 && max_seqlen_q <= 65535 * 64 ? 1 : 2;
 }
 // Key parts of a step on cached prefixes.  Few new tokens on a long prefix leave CUs idle while each workgroup walks its key
-// tiles: the tiles are dealt over as many workgroups as 512 places (two a CU) take, about (tokens / tile + half a tile per
-// sequence) x heads of them being wanted without parts, and at least 8 tiles each, below which writing and adding the
-// parts costs what it saves; and from about 25 us on, since the second launch takes the host 4 (12 x 64 heads, 26 tokens on
-// 1000 cached 20, in two parts 23.5).  Measured (us; 1 part, then as planned): 40 x 128 heads, 1 sequence, 64 tokens on 8000 cached
-// 163, 55; 128 on 1900 48, 33; 4 sequences, 64 on 4000 45, 34; 200 on 4000 48, 39; 8, 64 on 8000 58, 43; 12 x 64 heads, 64 on
-// 8000 103, 25; 4 sequences, 1000 on 4000 35, 25.  Full places lose: 1 sequence, 512 on 1500 52, in two parts 56; 6 sequences,
+// tiles: the tiles are dealt over as many workgroups as 512 places (two a CU) take, and at least 8 tiles each, below which writing and
+// adding the parts costs what it saves; and from about 25 us on, since the second launch takes the host 4 (12 x 64 heads, 26
+// tokens on 1000 cached 20, in two parts 23.5).
+// Measured (us; 1 part, then as planned): 40 x 128 heads, 1 sequence, 64 tokens on 8000 cached 167, 49; 128 on 1900 49, 29.5; 4
+// sequences, 64 on 4000 46, 30; 12 x 64 heads, 64 on 8000 100, 24; 8 sequences, 400 on 8000 36, 24; 4, 1000 on 4000 35, 27.
+// Parts lose where workgroups are many already: beyond 512 places they stand in a second round, beyond 256 two share a CU.  How
+// many there are without parts is known only from above (`groups`: each sequence may end with a partly filled tile, and none
+// has more tiles than the longest), and that other sequences are shorter than the longest, which leaves places to its parts,
+// is not known at all.  So the line lies where no batch measured loses, even lengths being the worst (1127 steps of 1 to 16
+// sequences, 1 to 600 new tokens on up to 6000 cached, 12 to 64 heads: 433 in parts, 3 % to 4 times faster than in one; where
+// only likely groups were counted, and no line drawn, 35 were 4 to 25 % slower).  Even lengths, us, at 128 wide, groups / key
+// tiles: 96 / 16 26.8, 25.6; 144 / 16 27.4, 29.4; 120 / 20 32.3, 28.8; 160 / 20 34.3, 34.6; 160 / 24 37.6, 36.0; 216 / 24 37.4, 36.1;
+// 240 / 24 39.1, 43.2; 240 / 64 110.9, 110.1; 280 / 18 36.7, 47.8.  64 wide: 256 / 24 25.8, 26.2; 256 / 32 31.9, 31.5; 320 / 24 29.4,
+// 34.9.  Uneven ones would gain beyond it (40 x 128, 8 sequences, 64 on 8000 60, 45).  Full places lose in any case: 6 sequences,
 // 2048 on 4200 99, in parts of 8 tiles 119; prompts without a prefix (1 x 1500 44, in two parts 52).
+// (`likely` counts half a tile per sequence; more parts than it allows were not measured.)
 struct KeyParts { int parts, part_tiles; int64_t bytes; };
 KeyParts key_parts(int64_t num_seqs, int64_t num_tokens, int64_t max_seqlen_q, int64_t max_seqlen_k, int num_heads,
                    int head_size) {
-  const int qt = query_tiles(num_seqs, num_tokens, max_seqlen_q, num_heads);
-  const int64_t bq = 64 * qt, q_tiles = (max_seqlen_q + bq - 1) / bq, tiles = (max_seqlen_k + BKV - 1) / BKV;
-  const int64_t wanted = (2 * num_tokens / bq + num_seqs) * num_heads / 2;
-  const int64_t most = std::min<int64_t>(512 / std::max<int64_t>(wanted, 1), tiles / 8);
-  if (most < 2 || tiles < (head_size == 64 ? 24 : 16) || q_tiles * most > 65535) return KeyParts{1, INT32_MAX / 2, 0};
-  const int part_tiles = (int)std::min<int64_t>((tiles + most - 1) / most, INT32_MAX / 2);
-  return KeyParts{(int)most, part_tiles,
-                  (num_tokens / bq + num_seqs) * num_heads * most *
-                      (head_size == 64 ? unit_floats<64>(qt) : unit_floats<128>(qt)) * 4};
+  constexpr KeyParts kOne{1, INT32_MAX / 2, 0};
+  if (64 * query_tiles(num_seqs, num_tokens, max_seqlen_q, num_heads) != kPartQueries) return kOne;
+  const int64_t q_tiles = (max_seqlen_q + kPartQueries - 1) / kPartQueries, tiles = (max_seqlen_k + BKV - 1) / BKV;
+  const int64_t most_tiles = num_tokens / kPartQueries + num_seqs;   // in all sequences
+  const int64_t groups = std::min(most_tiles, num_seqs * q_tiles) * num_heads;
+  const int64_t likely = (2 * num_tokens / kPartQueries + num_seqs) * num_heads / 2;
+  const int64_t from = head_size == 64 ? (groups <= 192 ? 24 : 32)   // (beyond 256 groups there are no two parts)
+                                       : groups <= 96 ? 16 : groups <= 128 ? 20 : groups <= 216 ? 24 : 64;
+  const int64_t parts = std::min<int64_t>(512 / std::max<int64_t>({groups, likely, 1}), tiles / 8);
+  if (parts < 2 || tiles < from || q_tiles * parts > 65535) return kOne;
+  const int part_tiles = (int)std::min<int64_t>((tiles + parts - 1) / parts, INT32_MAX / 2);
+  return KeyParts{(int)parts, part_tiles,
+                  most_tiles * num_heads * parts * (head_size == 64 ? unit_floats<64>() : unit_floats<128>()) * 4};
 }
 
 int launch_prefill(PrefillArgs& a, bool paged, int64_t num_seqs, int64_t max_seqlen_q, int64_t max_seqlen_k, int num_heads,
@@ -497,7 +509,7 @@ int launch_prefill(PrefillArgs& a, bool paged, int64_t num_seqs, int64_t max_seq
   }
 #define APS_LAUNCH_PF_Q(B, D_, P, Q_)                                                                                 \
   do {                                                                                                                \
-    constexpr bool kMayPart = P == kPaged16 || P == kPagedAny;                                                        \
+    constexpr bool kMayPart = (P == kPaged16 || P == kPagedAny) && 64 * Q_ == kPartQueries;                           \
     if (kMayPart && a.parts > 1)                                                                                      \
       APS_LAUNCH((prefill_attention_kernel<B, D_, P, Q_, kMayPart>), grid, dim3(kThreads), prefill_lds_bytes<D_>(), s, a); \
     else                                                                                                              \
@@ -517,11 +529,7 @@ int launch_prefill(PrefillArgs& a, bool paged, int64_t num_seqs, int64_t max_seq
   const int st = launch_status();
   if (st != APS_OK || a.parts == 1) return st;
   const dim3 cgrid((unsigned)num_heads, (unsigned)num_seqs, (unsigned)q_tiles);
-#define APS_LAUNCH_PC(B, D_)                                                                              \
-  do {                                                                                                    \
-    if (qt == 2) APS_LAUNCH((prefill_combine_kernel<B, D_, 2>), cgrid, dim3(kThreads), 0, s, a);          \
-    else APS_LAUNCH((prefill_combine_kernel<B, D_, 1>), cgrid, dim3(kThreads), 0, s, a);                  \
-  } while (0)
+#define APS_LAUNCH_PC(B, D_) APS_LAUNCH((prefill_combine_kernel<B, D_>), cgrid, dim3(kThreads), 0, s, a)
 #define APS_LAUNCH_PC_D(B) do { if (head_size == 64) APS_LAUNCH_PC(B, 64); else APS_LAUNCH_PC(B, 128); } while (0)
   if (dtype == APS_F16) APS_LAUNCH_PC_D(false); else APS_LAUNCH_PC_D(true);
 #undef APS_LAUNCH_PC_D

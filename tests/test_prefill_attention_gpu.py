@@ -169,10 +169,10 @@ def test_longest_sequence_stated_beyond_the_tokens(dev, max_seqlen):
         ops.flash_attn_varlen_func(q, k, v, cu_seqlens_q=cu, max_seqlen_q=65535 * 128 + 1, softmax_scale=0.125)
 
 
-@pytest.mark.parametrize("H,D,BS,dtype", [(2, 64, 16, torch.float16), (2, 128, 48, torch.bfloat16), (80, 128, 16, torch.float16),
-                                          (80, 64, 32, torch.bfloat16)])
+@pytest.mark.parametrize("H,D,BS,dtype", [(2, 64, 16, torch.float16), (2, 128, 48, torch.bfloat16), (36, 128, 16, torch.float16),
+                                          (32, 64, 32, torch.bfloat16)])
 def test_prefix_attention_in_key_parts(dev, H, D, BS, dtype):
-    """Few new tokens on long prefixes: the keys of a sequence in parts (64 queries a workgroup with 2 heads, 128 with 80).
+    """Few new tokens on long prefixes: the keys of a sequence in parts, three of them with 2 heads, two with the others.
     Lengths on and about the edges of the parts, one that fits a single part, queries that see nothing of the last part;
     NaN behind every sequence.  A null workspace means one part, whose 16-bit probabilities are rounded against another
     maximum: each may differ by 2 u of itself (u = 2^-11, bf16 2^-8) and, below fp16's normal numbers, by 2^-24, so the
@@ -214,6 +214,15 @@ def test_prefix_attention_parts_only_where_workgroups_are_few():
     assert need(1, 64, 64, 960, 40, 128) == 0 < need(1, 64, 64, 961, 40, 128)       # parts of fewer than 8 key tiles
     assert need(1, 64, 64, 1472, 12, 64) == 0 < need(1, 64, 64, 1473, 12, 64)       # too short for a second launch
     assert need(0, 0, 0, 0, 40, 128) == 0 and need(1, 64, 64, 0, 40, 128) == 0 and need(1, 64, 64, 8064, 40, 96) == 0
+    # the more workgroups there are without parts, the more key tiles it takes; sequences of 20 new tokens, one workgroup a head
+    def tiles(n, heads, dim, k):
+        return need(n, 20 * n, 20, 64 * k, heads, dim) > 0
+    for n, heads, dim, first in ((8, 12, 128, 16), (9, 12, 128, 20), (10, 12, 128, 20), (11, 12, 128, 24), (18, 12, 128, 24),
+                                 (19, 12, 128, 64), (21, 12, 128, 64), (16, 12, 64, 24), (17, 12, 64, 32), (21, 12, 64, 32)):
+        assert tiles(n, heads, dim, first) and not tiles(n, heads, dim, first - 1), (n, heads, dim)
+    assert not any(tiles(n, heads, dim, 1000) for n, heads, dim in ((7, 40, 128), (22, 12, 128), (5, 64, 64), (22, 12, 64)))
+    # 140 new tokens: in one sequence three workgroups a head, dealt over ten it may be as many as eleven
+    assert need(1, 140, 140, 1024, 32, 128) > 0 == need(10, 140, 131, 1024, 12, 128)
 
 
 def test_prefix_attention_takes_no_length_off_the_device(dev):
