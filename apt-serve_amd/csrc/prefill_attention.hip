@@ -453,9 +453,10 @@ int query_tiles(int64_t num_seqs, int64_t num_tokens, int64_t max_seqlen_q, int 
   return num_heads * (num_tokens / 128 + num_seqs) <= 384 && max_seqlen_q <= 65535 * 64 ? 1 : 2;
 }
 // Key parts of a step on cached prefixes.  Few new tokens on a long prefix leave CUs idle while each workgroup walks its key
-// tiles: the tiles are dealt over as many workgroups as 512 places (two a CU) take, and at least 8 tiles each, below which writing and
-// adding the parts costs what it saves; and from about 25 us on, since the second launch takes the host 4 (12 x 64 heads, 26
-// tokens on 1000 cached 20, in two parts 23.5).
+// tiles: the tiles are dealt over as many workgroups as 512 places (two a CU) take, the longest sequence's at least 8 tiles each;
+// those of a shorter one, which tiles_per_part evens out, may hold 5 (9 tiles in parts of 8).  Writing and adding the parts
+// takes about as long as five tiles (40 x 128 heads, 51 tokens, 16 tiles 25.5, in parts of 8 20.5), and the second launch 4 us of
+// the host (12 x 64 heads, 26 tokens on 1000 cached 20, in two parts 23.5).
 // Measured (us; 1 part, then as planned): 40 x 128 heads, 1 sequence, 64 tokens on 8000 cached 167, 49; 128 on 1900 49, 29.5; 4
 // sequences, 64 on 4000 46, 30; 12 x 64 heads, 64 on 8000 100, 24; 8 sequences, 400 on 8000 36, 24; 4, 1000 on 4000 35, 27.
 // Parts lose where workgroups are many already: beyond 512 places they stand in a second round, beyond 256 two share a CU.  How
