@@ -109,13 +109,16 @@ __global__ __launch_bounds__(kLnThreads) void add_layer_norm_kernel(const AddLnA
     gw[j] = *(const u32x4*)(g.gamma + (int64_t)i * 16);
     gb[j] = g.beta ? *(const u32x4*)(g.beta + (int64_t)i * 16) : u32x4{0u, 0u, 0u, 0u};
   }
-  // (past the row's end: its last vector, loaded and not used, so that no load stands behind a branch)
+  // (past the row's end: its last vector, loaded and not used, so that no load stands behind a branch; a lone vector waits for
+  // none, and there a branch spares the loads)
   u32x4 pa[VECS], pb[VECS];
 #pragma unroll
   for (int j = 0; j < VECS; ++j) {
     const int i = min((int)threadIdx.x + j * kLnThreads, nvec - 1);
-    if constexpr (!PARTS) pa[j] = *(const u32x4*)(x + (int64_t)i * 16);
-    pb[j] = r ? *(const u32x4*)(r + (int64_t)i * 16) : u32x4{0u, 0u, 0u, 0u};
+    if (VECS > 1 || (int)threadIdx.x < nvec) {
+      if constexpr (!PARTS) pa[j] = *(const u32x4*)(x + (int64_t)i * 16);
+      pb[j] = r ? *(const u32x4*)(r + (int64_t)i * 16) : u32x4{0u, 0u, 0u, 0u};
+    }
   }
   if constexpr (PARTS) product_vecs<BF16, VECS>(g, row, nvec, pa);
 #pragma unroll
@@ -178,16 +181,23 @@ namespace {
 template <bool PARTS>
 int launch_add_layer_norm(const AddLnArgs& g, int64_t rows, int dtype, aps_stream_t stream) {
   const dim3 grid((unsigned)rows);
-  // rows of up to 3 * 256 * 8 = 6144 elements (every OPT up to 13B) keep 3 vectors per thread, wider ones 8
-  const bool narrow = g.width <= 3 * kLnThreads * 8;
+  // As many vectors per thread as the row takes, since all of them are loaded, those past the row's end too (us with the residual
+  // add, f16; a load behind a branch each, always three or eight vectors, and so: 8192 rows of 768 15.6, 18.0, 12.7; 361 of
+  // 2560 4.57, 4.71, 4.57; 361 of 7168 7.1, 7.3, 6.5; 8192 of 7168 112, 87.8, 87.2; 1 of 16384 6.4, 5.5, 5.5).
+  const int vecs = (g.width + kLnThreads * 8 - 1) / (kLnThreads * 8);
   hipStream_t s = (hipStream_t)stream;
-  if (dtype == APS_BF16) {
-    if (narrow) APS_LAUNCH((add_layer_norm_kernel<true, 3, PARTS>), grid, dim3(kLnThreads), 0, s, g);
-    else APS_LAUNCH((add_layer_norm_kernel<true, kLnVecs, PARTS>), grid, dim3(kLnThreads), 0, s, g);
-  } else {
-    if (narrow) APS_LAUNCH((add_layer_norm_kernel<false, 3, PARTS>), grid, dim3(kLnThreads), 0, s, g);
-    else APS_LAUNCH((add_layer_norm_kernel<false, kLnVecs, PARTS>), grid, dim3(kLnThreads), 0, s, g);
+#define APS_LAUNCH_LN(B, V) APS_LAUNCH((add_layer_norm_kernel<B, V, PARTS>), grid, dim3(kLnThreads), 0, s, g)
+#define APS_LAUNCH_LN_V(B)                \
+  switch (vecs) {                         \
+    case 1: APS_LAUNCH_LN(B, 1); break;   \
+    case 2: APS_LAUNCH_LN(B, 2); break;   \
+    case 3: APS_LAUNCH_LN(B, 3); break;   \
+    case 4: APS_LAUNCH_LN(B, 4); break;   \
+    default: APS_LAUNCH_LN(B, kLnVecs);   \
   }
+  if (dtype == APS_BF16) { APS_LAUNCH_LN_V(true) } else { APS_LAUNCH_LN_V(false) }
+#undef APS_LAUNCH_LN_V
+#undef APS_LAUNCH_LN
   return launch_status();
 }
 }  // namespace

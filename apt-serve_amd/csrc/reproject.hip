@@ -1178,8 +1178,8 @@ int64_t aps_linear_nt_workspace_bytes(int64_t m, int64_t n, int64_t k) {
 
 // A row's workgroup adds the parts of a product that its norm reads; many of them want a launch of their own, whose workgroups
 // are not bound to rows (us, product and norm, parts added by the norm against by themselves; f16).  Up to 8 parts the norm wins
-// or is even at all sizes measured, 11 weight shapes and 2 to 1000 rows (768 x 3072, 130 rows, 8 parts 14.6 and 15.5; 4096 x 16384,
-// 48 rows, 8 parts 40.5 and 44.5; 7168 x 28672, 200 rows, 8 parts 151.6 and 154.5), and 27 to 32 lose (256 x 20480, 49 rows, 32
+// or is even at all sizes measured, 11 weight shapes and 2 to 1000 rows (768 x 3072, 130 rows, 8 parts 13.7 and 15.2; 4096 x 16384,
+// 48 rows, 8 parts 40.5 and 44.5; 7168 x 28672, 200 rows, 8 parts 150.6 and 154.5), and 27 to 32 lose (256 x 20480, 49 rows, 32
 // parts 26.9 and 23.5; 768 x 20480, 200 rows, 27 parts 36.0 and 33.8).  The line may lie higher: 10 parts still win (2560 x 10240,
 // 48 rows 22.9 and 31.5; 5120 x 20480, 65 rows 66.7 and 68.0), 13 and 16 win or lose by size (2048 x 8192, 24 rows 18.8 and 22.0,
 // 49 rows 19.5 and 19.3).

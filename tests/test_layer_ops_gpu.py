@@ -13,7 +13,9 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
-@pytest.mark.parametrize("rows,width", [(1, 8), (5, 768), (7, 5120), (256, 5120), (3, 16384), (2, 1000)])
+@pytest.mark.parametrize("rows,width", [(1, 8), (5, 768), (7, 5120), (256, 5120), (3, 16384), (2, 1000),
+                                        # on both sides of where a thread takes one vector more
+                                        (3, 2048), (3, 2056), (3, 4096), (3, 4104), (3, 6144), (3, 6152), (3, 8192), (3, 8200)])
 def test_add_layer_norm_matches_the_two_operator_definition(dev, dtype, rows, width):
     x, r = randn((rows, width), 1, dtype), (randn((rows, width), 2) * 3).to(dtype)
     w, b = (1 + 0.1 * randn((width,), 3)).to(dtype), (0.1 * randn((width,), 4)).to(dtype)
@@ -48,7 +50,8 @@ def test_add_layer_norm_strided_rows_and_errors(dev):
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("m,n,k", [(1, 768, 768), (5, 5120, 20480), (12, 768, 3072), (48, 2560, 2048), (49, 768, 20480),
-                                   (65, 5120, 5120), (361, 5120, 5120), (130, 7168, 4096), (700, 1024, 4096)])
+                                   (65, 5120, 5120), (361, 5120, 5120), (130, 7168, 4096), (700, 1024, 4096), (5, 2048, 2048),
+                                   (5, 2304, 2304), (12, 4096, 4096), (12, 6144, 6144), (12, 8192, 8192), (12, 8448, 8448)])
 def test_product_with_the_norm_behind_it_equals_the_two_calls(dev, m, n, k, dtype):
     """Products of one part, of few (the norm adds them) and of more than the norm adds; the same bits as linear_nt, then
     add_layer_norm.  With and without biases, and with a bias that no vector load takes."""
