@@ -802,12 +802,17 @@ def kv_reproject_gathered(hidden_states, paged_cache, holder_src, w_kv, b_kv, ws
 
 # ------------------------------------------------------------------ prompt attention
 
-def _stated_keys(max_seqlen_k, capacity: int) -> int:
+def _stated_keys(max_seqlen_k) -> int:
     """Longest sequence by which the key parts of a step are sized; 0 (one part, one launch) where the caller states none: tables
     are usually wider than their sequences are long, and parts sized by the width leave workgroups and a second launch that
     do nothing (4 sequences, 64 tokens on 200 cached, tables of 2048: 10.8 -> 12.7 us).  Only a number of the host is looked at: a
     tensor is not worth a synchronisation, which a capture would refuse."""
-    return min(int(max_seqlen_k), capacity) if isinstance(max_seqlen_k, numbers.Integral) else 0
+    return int(max_seqlen_k) if isinstance(max_seqlen_k, numbers.Integral) else 0
+
+
+#: Keys that no step splits, by head size (23 and 15 tiles of 64): short steps, 16 us of the host, are spared the 0.5 us of asking
+#: the library.
+_KEYS_IN_ONE_PART = {64: 1472, 128: 960}
 
 
 def flash_attn_varlen_func(q, k, v, cu_seqlens_q=None, cu_seqlens_k=None, max_seqlen_q=None, max_seqlen_k=None,
@@ -857,15 +862,18 @@ def flash_attn_varlen_func(q, k, v, cu_seqlens_q=None, cu_seqlens_k=None, max_se
               block_table.device == dev and (block_table.size(1) <= 1 or block_table.stride(1) == 1),
               "block_table must be int32 [seqs, width] with contiguous rows on the same GPU")
         lib = _lib.load()
-        max_k = _stated_keys(max_seqlen_k, block_table.size(1) * k.size(1))
-        need = lib.aps_paged_prefill_attention_workspace_bytes(n_seq, T, max_len, max_k, H, D)
-        ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None     # (few tokens on long prefixes)
+        max_k, ws, need = max_seqlen_k if type(max_seqlen_k) is int else _stated_keys(max_seqlen_k), None, 0
+        if max_k > _KEYS_IN_ONE_PART.get(D, 0):                             # few tokens on long prefixes, it may be
+            max_k = min(max_k, block_table.size(1) * k.size(1))
+            need = lib.aps_paged_prefill_attention_workspace_bytes(n_seq, T, max_len, max_k, H, D)
+            ws = torch.empty(need, dtype=torch.uint8, device=dev) if need else None
         with _on(dev):
             st = lib.aps_paged_prefill_attention_split(
                 out.data_ptr() if T else None, q.data_ptr() if T else None, k.data_ptr(), v.data_ptr(),
                 _ptr(block_table), _ptr(cu_seqlens_q), _ptr(cu_seqlens_k), n_seq if T else 0, T, max_len, H, D,
                 k.size(1), block_table.stride(0), block_table.size(1), q.stride(0), out.stride(0), k.stride(0),
-                k.size(0), float(softmax_scale), _DTYPE_CODE[q.dtype], max_k, _ptr(ws), need, _stream(q))
+                k.size(0), float(softmax_scale), _DTYPE_CODE[q.dtype], max_k if need else 0, _ptr(ws) if need else None, need,
+                _stream(q))
         _lib.check(st, "flash_attn_varlen_func (prefix branch)")
         return out
     _need(cu_seqlens_k is None or cu_seqlens_k is cu_seqlens_q or torch.equal(cu_seqlens_k, cu_seqlens_q),

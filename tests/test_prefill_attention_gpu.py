@@ -214,6 +214,8 @@ def test_prefix_attention_parts_only_where_workgroups_are_few():
     assert need(1, 64, 64, 960, 40, 128) == 0 < need(1, 64, 64, 961, 40, 128)       # parts of fewer than 8 key tiles
     assert need(1, 64, 64, 1472, 12, 64) == 0 < need(1, 64, 64, 1473, 12, 64)       # too short for a second launch
     assert need(0, 0, 0, 0, 40, 128) == 0 and need(1, 64, 64, 0, 40, 128) == 0 and need(1, 64, 64, 8064, 40, 96) == 0
+    for dim, keys in ops._KEYS_IN_ONE_PART.items():     # about these the library is not asked
+        assert need(1, 1, 1, keys, 1, dim) == 0 < need(1, 1, 1, keys + 1, 1, dim)
     # the more workgroups there are without parts, the more key tiles it takes; sequences of 20 new tokens, one workgroup a head
     def tiles(n, heads, dim, k):
         return need(n, 20 * n, 20, 64 * k, heads, dim) > 0
@@ -230,8 +232,7 @@ def test_prefix_attention_takes_no_length_off_the_device(dev):
     the host's, parts are not sized by the width of the tables: the bits of one part."""
     from test_oracle_attention import build_paged
     from aptserve_hip.ops import _stated_keys
-    assert _stated_keys(None, 2048) == _stated_keys(torch.tensor(1538), 2048) == 0
-    assert _stated_keys(1538, 2048) == _stated_keys(np.int32(1538), 2048) == 1538 and _stated_keys(5000, 2048) == 2048
+    assert _stated_keys(None) == _stated_keys(torch.tensor(1538)) == 0 and _stated_keys(1538) == _stated_keys(np.int32(1538)) == 1538
     H, D, klens, qlens = 2, 128, [1538, 64], [70, 3]
     kc, vc, bt, _, _ = (x.to(dev) if isinstance(x, torch.Tensor) else x for x in build_paged(2, H, D, 16, klens, 3))
     q = randn((sum(qlens), H, D), 4).to(dev)
@@ -242,7 +243,8 @@ def test_prefix_attention_takes_no_length_off_the_device(dev):
         return ops.flash_attn_varlen_func(q, kc, vc, cu_seqlens_q=cu_q, cu_seqlens_k=cu_k, max_seqlen_q=70, max_seqlen_k=max_k,
                                           block_table=bt)
     one, parts = call(0), call(1538)
-    assert not torch.equal(one, parts)
+    assert not torch.equal(one, parts) and torch.equal(parts, call(np.int64(1538)))
+    assert torch.equal(parts, call(1 << 40))     # no more than the tables hold
     torch.cuda.set_sync_debug_mode("error")
     try:
         outs = [call(on_device), call(None)]
