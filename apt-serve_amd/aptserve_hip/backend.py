@@ -343,9 +343,9 @@ class HybridOPTAttention:
             return ops.linear_nt(attn_output, self.out_weight, self.out_bias)
 
     def attend(self, hidden_states, kv_cache, shared_cache, attn_metadata: HybridAttentionMetadata, hidden_cache=None):
-        """Everything up to the out projection.  ``hidden_cache``: where hidden rows are cached when it is not ``kv_cache`` itself — a separate
-        ``(2, N, BS, H, D)`` tensor in the activation dtype, needed with an fp8 K/V cache (whose bytes cannot hold
-        16-bit hidden rows)."""
+        """Everything up to the out projection.  ``hidden_cache``: where hidden rows are cached when it is not
+        ``kv_cache`` itself — a separate ``(2, N, BS, H, D)`` tensor in the activation dtype, needed with an fp8 K/V
+        cache (whose bytes cannot hold 16-bit hidden rows)."""
         md = attn_metadata
         hc = kv_cache if hidden_cache is None else hidden_cache
         same = kv_cache is not None and kv_cache.dtype == hidden_states.dtype      # K/V cached in the activation dtype

@@ -2,10 +2,11 @@
 //
 // Input is one small per-sequence description (length, cache type, block
 // tables); everything whose size grows with the number of cached tokens — slot
-// mappings and the row-index vectors — is expanded on the device.  One launch,
-// one workgroup per sequence: the workgroup first reduces the per-sequence row
-// counts of all earlier sequences (its exclusive prefix, O(batch) reads that
-// stay in L2), then its threads write the rows of its own sequence.
+// mappings and the row-index vectors — is expanded on the device.  One launch;
+// the workgroups of a sequence (one in a prompt step, up to eight in a decode
+// step) first reduce the per-sequence row counts of all earlier sequences (their
+// exclusive prefix, O(batch) reads that stay in L2), then their threads write the
+// rows of the sequence.
 #include <string.h>
 
 #include <algorithm>
